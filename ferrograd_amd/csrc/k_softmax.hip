@@ -9,37 +9,26 @@
 // buffer, and its gradient is then pushed through the softmax Jacobian a
 // second time (defect).
 //
-// Here one workgroup owns one row.  The fast path keeps the whole row in
-// registers (NV float4 per thread; 256 threads, or 1024 for rows of more
-// than 16384 columns: up to 32768 columns), so the logits are read from HBM
-// exactly once and dlogits written exactly once: 8*C bytes per row, the
-// minimum.  Reductions are wavefront shuffles (64 lanes) followed by one LDS
-// exchange across the waves.  Rows too long for registers, or not 16-byte
-// aligned, use a two-pass streaming kernel with an online max/sum.
+// Here a row is owned by one wave or one workgroup, which reads the logits
+// from HBM once and writes dlogits once, whatever the row's length (up to
+// 8192 16-byte chunks) and alignment (fg_softmax_any.h); longer rows are
+// read twice.  Rows whose outputs lie differently against 16-byte boundaries
+// than the logits take a two-pass kernel one element a lane.
 //
-// Long rows (up to 32768 columns): 1024 threads with 8 float4 each, held
-// to 64 VGPRs so that two workgroups share a CU, read and written with
-// buffer instructions: the 8192 x 32000 CE at 5.76-5.84 TB/s (median of 30)
-// against 5.70-5.75 for 512 threads with 16 float4 (two or three
-// workgroups per CU) and 4.5-4.8 for 1024 threads at 4 waves per SIMD (one
-// workgroup per CU: its reductions and exponentials leave the CU's memory
-// idle).  Earlier, on the 512-thread kernel: 363.5 us (5.77 TB/s) against
-// 372.5 us for 256 threads with 32 float4 and plain global accesses; measured
-// and dropped: rotating each row's chunk order by the row index (366.9 us),
-// holding the 512-thread kernel to 80 VGPRs for a sixth wave per SIMD (it
-// then spills: 381 us), 256 threads with buffer instructions (377 us).  For
-// scale: a flat copy of the same bytes reaches 6.5-6.6 TB/s, and copy kernels
-// with this kernel's row structure (one workgroup reads a 128 KB row into
-// registers, reduces it, writes it) 5.8 TB/s with 512 threads and 6.0 with
-// 1024; capping each wave's loads in flight at 4, 8 or 12 of 16, walking the
-// rows in another order, or a persistent workgroup that loads the next row
-// while it finishes one leave them within 1-3 %.
+// The 8192 x 32000 fp32 CE: 5.86 TB/s (358 us).  For scale: a flat copy of
+// the same bytes reaches 6.5-6.6 TB/s, and copy kernels with this kernel's
+// row structure (one workgroup reads a 128 KB row into registers, reduces it,
+// writes it) 5.8 TB/s with 512 threads and 6.0 with 1024; capping each wave's
+// loads in flight at 4, 8 or 12 of 16, walking the rows in another order, or
+// a persistent workgroup that loads the next row while it finishes one leave
+// them within 1-3 %.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 
 #include "fg_half.h"
 #include "fg_internal.h"
+#include "fg_softmax_any.h"
 #include "fg_softmax_row.h"
 
 namespace {
@@ -131,7 +120,11 @@ __device__ __forceinline__ void row_outputs(const void *xr, int dt, int C, const
     }
 }
 
-// Register-resident fast path with NT threads.  out (may be NULL) receives
+// fp32 rows of 16385 to 32768 columns, 16-byte aligned and in whole chunks:
+// the same held row with the accesses' bounds in buffer descriptors.  8192 x
+// 32000 360.3 us, 361.6 for softmax_any<fp32, 8, 16> (which checks each
+// chunk's bounds in the vector unit and has two registers too many for the
+// two rows a CU); shorter rows were faster there.  out (may be NULL) receives
 //   labels ? scale*(p - onehot) : scale*p.
 // Thread t holds the float4 chunks t + NT*i of the row (i < NV); argmax ties
 // go to the lowest column (a row of -inf gives 0, as the CPU restatement's
@@ -151,15 +144,15 @@ constexpr int kBufNT = 2;              // cache-policy bits: non-temporal
 // A 1024-thread workgroup is held to 64 VGPRs (8 waves per SIMD), so that
 // two rows share a CU and one's reductions and exponentials overlap the
 // other's memory traffic.
-template <int NV, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ? 8 : 1)))
+constexpr int kWideNV = 8, kWideNT = 1024;
+__global__ __launch_bounds__(kWideNT) __attribute__((amdgpu_waves_per_eu(8)))
 void softmax_rows_v4(const float *__restrict__ x, int ldx,
                                                       const uint32_t *__restrict__ labels, int C,
                                                       float scale, float *__restrict__ row_loss,
                                                       float *__restrict__ out, int ldo,
                                                       uint32_t *__restrict__ argmax,
                                                       float *__restrict__ probs, int ldp) {
-    constexpr int NW = NT / 64;
+    constexpr int NV = kWideNV, NT = kWideNT, NW = NT / 64;
     __shared__ float sm[NW];
     __shared__ int si[NW];
     const int r = blockIdx.x;
@@ -230,8 +223,8 @@ void softmax_rows_v4(const float *__restrict__ x, int ldx,
     }
 }
 
-// Streaming path for any C, alignment and element type dt (x and out share
-// it): pass 1 online (max, sum, argmax), pass 2 recomputes exp and writes,
+// Any C, alignment and element type dt (x and out share it), for outputs out
+// of phase with the logits: pass 1 online (max, sum, argmax), pass 2 recomputes exp and writes,
 // rounding to dt.
 __global__ __launch_bounds__(kNT) void softmax_rows_stream(const void *__restrict__ x, int ldx,
                                                            const uint32_t *__restrict__ labels,
@@ -267,96 +260,6 @@ __global__ __launch_bounds__(kNT) void softmax_rows_stream(const void *__restric
             const float p = expf(fg::load_as_f(x, dt, xb + c) - m) * inv;
             if (out) fg::store_from_f(out, dt, ob + c, scale * (c == t ? p - 1.0f : p));
             if (probs) fg::store_from_f(probs, dt, pb + c, p);
-        }
-    }
-}
-
-// Register-resident path for 16-bit rows (fp16 / bf16, 8-byte aligned,
-// C % 4 == 0): NV groups of 4 elements per thread, read once, written once.
-template <int NV>
-__global__ __launch_bounds__(kNT) void softmax_rows_h4(const uint16_t *__restrict__ x, int ldx,
-                                                       const uint32_t *__restrict__ labels, int C,
-                                                       float scale, float *__restrict__ row_loss,
-                                                       uint16_t *__restrict__ out, int ldo,
-                                                       uint32_t *__restrict__ argmax, int dt,
-                                                       uint16_t *__restrict__ probs, int ldp) {
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    __shared__ float sm[kWaves];
-    __shared__ int si[kWaves];
-    const int r = blockIdx.x;
-    const uint16_t *xr = x + (size_t)r * ldx;
-    const int C4 = C >> 2;
-    f32x4 v[NV];
-    float m = -INFINITY;
-    int am = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int j = threadIdx.x + i * kNT;
-        if (j < C4) {
-            const u32x2 w = __builtin_nontemporal_load(reinterpret_cast<const u32x2 *>(xr) + j);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                v[i][e] = fg::h16_to_f(dt, (uint16_t)(w[e >> 1] >> (16 * (e & 1))));
-        } else {
-            v[i] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int c0 = 4 * (threadIdx.x + i * kNT);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (v[i][e] > m) {
-                m = v[i][e];
-                am = c0 + e;
-            }
-    }
-    block_argmax(m, am, sm, si);
-    float s = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[i][e] = expf(v[i][e] - m);
-            s += v[i][e];
-        }
-    }
-    s = block_sum(s, sm);
-    row_outputs(xr, dt, C, labels, r, m, s, am, row_loss, argmax);
-    if (out) {
-        const float inv = 1.0f / s;
-        const int t = labels ? (int)labels[r] : -1;
-        uint16_t *orow = out + (size_t)r * ldo;
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int j = threadIdx.x + i * kNT;
-            if (j < C4) {
-                uint16_t d[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float p = v[i][e] * inv;
-                    d[e] = fg::f_to_h16(dt, scale * (4 * j + e == t ? p - 1.0f : p));
-                }
-                const u32x2 w = {(uint32_t)d[0] | ((uint32_t)d[1] << 16),
-                                 (uint32_t)d[2] | ((uint32_t)d[3] << 16)};
-                __builtin_nontemporal_store(w, reinterpret_cast<u32x2 *>(orow) + j);
-            }
-        }
-    }
-    if (probs) {
-        const float inv = 1.0f / s;
-        uint16_t *prow = probs + (size_t)r * ldp;
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int j = threadIdx.x + i * kNT;
-            if (j < C4) {
-                uint16_t d[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) d[e] = fg::f_to_h16(dt, v[i][e] * inv);
-                const u32x2 w = {(uint32_t)d[0] | ((uint32_t)d[1] << 16),
-                                 (uint32_t)d[2] | ((uint32_t)d[3] << 16)};
-                __builtin_nontemporal_store(w, reinterpret_cast<u32x2 *>(prow) + j);
-            }
         }
     }
 }
@@ -541,6 +444,70 @@ __global__ __launch_bounds__(kNT) void softmax_bwd_rows(const void *__restrict__
     }
 }
 
+// Every row of q lies against 16-byte boundaries as the same row of x does
+// (q NULL: nothing to place).
+bool same_phase(int dt, const void *x, int ldx, const void *q, int ldq, int R) {
+    const uint32_t esz = dt == fg::kF32 ? 4 : 2;
+    return !q || (((uintptr_t)x ^ (uintptr_t)q) & 15u) == 0 &&
+                     (R <= 1 || (((uint32_t)ldx - (uint32_t)ldq) * esz & 15u) == 0);
+}
+
+// Runs f<NV, NW>() for a row of at most `chunks` whole 16-byte chunks: the
+// kinds of row kernel (NV chunks a thread on NW waves), as measured
+// (fg_softmax_any.h).  False: longer than any holds.
+template <class F>
+bool with_kind(int chunks, F f) {
+    using std::integral_constant;
+#define FG_SM_KIND(NV, NW)                                                \
+    if (chunks <= NV * NW * 64) {                                         \
+        f(integral_constant<int, NV>{}, integral_constant<int, NW>{});    \
+        return true;                                                      \
+    }
+    FG_SM_KIND(1, 1)
+    FG_SM_KIND(2, 1)
+    FG_SM_KIND(4, 1)
+    FG_SM_KIND(2, 4)
+    FG_SM_KIND(4, 4)
+    FG_SM_KIND(8, 4)
+    FG_SM_KIND(8, 8)
+    FG_SM_KIND(8, 16)
+#undef FG_SM_KIND
+    return false;
+}
+
+template <int DT>
+void launch_any(hipStream_t st, const void *x, int ldx, const uint32_t *labels, int R, int C,
+                float scale, float *row_loss, void *out, int ldo, uint32_t *argmax, void *probs,
+                int ldp) {
+    using T = typename fg::smany::Io<DT>::T;
+    const T *xt = static_cast<const T *>(x);
+    T *ot = static_cast<T *>(out), *pt = static_cast<T *>(probs);
+    const bool held = with_kind(C / fg::smany::Io<DT>::E, [&](auto nv, auto nw) {
+        fg::smany::softmax_any<DT, nv(), nw()>
+            <<<nw() == 1 ? (R + 3) / 4 : R, fg::smany::threads_of(nw()), 0, st>>>(
+                xt, ldx, labels, R, C, scale, row_loss, ot, ldo, argmax, pt, ldp);
+    });
+    if (!held)
+        fg::smany::softmax_long<DT><<<R, fg::smany::kLongNW * 64, 0, st>>>(
+            xt, ldx, labels, C, scale, row_loss, ot, ldo, argmax, pt, ldp);
+}
+
+template <int DT>
+void launch_bwd_any(hipStream_t st, const void *y, const void *dy, int R, int C, void *dx,
+                    int accumulate) {
+    using T = typename fg::smany::Io<DT>::T;
+    const T *yt = static_cast<const T *>(y), *dt = static_cast<const T *>(dy);
+    T *xt = static_cast<T *>(dx);
+    const bool held = with_kind(C / fg::smany::Io<DT>::E, [&](auto nv, auto nw) {
+        fg::smany::softmax_bwd_any<DT, nv(), nw()>
+            <<<nw() == 1 ? (R + 3) / 4 : R, fg::smany::threads_of(nw()), 0, st>>>(yt, dt, R, C, xt,
+                                                                               accumulate);
+    });
+    if (!held)
+        fg::smany::softmax_bwd_long<DT><<<R, fg::smany::kLongNW * 64, 0, st>>>(yt, dt, C, xt,
+                                                                            accumulate);
+}
+
 // The row kernels for R rows of C; `probs` (may be NULL) receives the
 // softmax.  With `mean` given and a small problem, the one-workgroup kernel
 // also writes the mean loss and *mean_done is set; otherwise the caller
@@ -579,53 +546,24 @@ int launch_rows(fg_ctx *ctx, int dt, const void *x, int ldx, const uint32_t *lab
         if (mean_done) *mean_done = mean != nullptr;
         return FG_OK;
     }
-    const unsigned align = dt == fg::kF32 ? 16u : 8u;
-    const bool aligned = ((((uintptr_t)x) | ((uintptr_t)out) | ((uintptr_t)probs)) &
-                          (align - 1)) == 0 &&
-                         (C % 4 == 0) && (ldx % 4 == 0) && (!out || ldo % 4 == 0) &&
-                         (!probs || ldp % 4 == 0);
-    const int C4 = C / 4;
-    dim3 grid(R), block(kNT);
-    if (dt == fg::kF32) {
-        const float *xf = static_cast<const float *>(x);
-        float *of = static_cast<float *>(out);
-#define FG_SM_LAUNCH(NV, NT)                                                               \
-    softmax_rows_v4<NV, NT><<<grid, NT, 0, st>>>(xf, ldx, labels, C, scale, row_loss, of, ldo, \
-                                                 argmax, static_cast<float *>(probs), ldp)
-        if (aligned && C4 <= kNT * 1)
-            FG_SM_LAUNCH(1, kNT);
-        else if (aligned && C4 <= kNT * 2)
-            FG_SM_LAUNCH(2, kNT);
-        else if (aligned && C4 <= kNT * 4)
-            FG_SM_LAUNCH(4, kNT);
-        else if (aligned && C4 <= kNT * 8)
-            FG_SM_LAUNCH(8, kNT);
-        else if (aligned && C4 <= kNT * 16)
-            FG_SM_LAUNCH(16, kNT);
-        else if (aligned && C4 <= 4 * kNT * 8)
-            FG_SM_LAUNCH(8, 4 * kNT);
+    if (same_phase(dt, x, ldx, out, ldo, R) && same_phase(dt, x, ldx, probs, ldp, R)) {
+        const bool whole = dt == fg::kF32 && C % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15u) == 0;
+        if (whole && C > 4 * 4096 && C <= 4 * kWideNV * kWideNT)
+            softmax_rows_v4<<<R, kWideNT, 0, st>>>(
+                static_cast<const float *>(x), ldx, labels, C, scale, row_loss,
+                static_cast<float *>(out), ldo, argmax, static_cast<float *>(probs), ldp);
+        else if (dt == fg::kF32)
+            launch_any<fg::kF32>(st, x, ldx, labels, R, C, scale, row_loss, out, ldo, argmax, probs,
+                                 ldp);
+        else if (dt == fg::kBF16)
+            launch_any<fg::kBF16>(st, x, ldx, labels, R, C, scale, row_loss, out, ldo, argmax,
+                                  probs, ldp);
         else
-            softmax_rows_stream<<<grid, block, 0, st>>>(x, ldx, labels, C, scale, row_loss, out,
-                                                        ldo, argmax, dt, probs, ldp);
-#undef FG_SM_LAUNCH
+            launch_any<fg::kF16>(st, x, ldx, labels, R, C, scale, row_loss, out, ldo, argmax,
+                                 probs, ldp);
     } else {
-        const uint16_t *xh = static_cast<const uint16_t *>(x);
-        uint16_t *oh = static_cast<uint16_t *>(out);
-#define FG_SM_LAUNCH(NV)                                                                        \
-    softmax_rows_h4<NV><<<grid, block, 0, st>>>(xh, ldx, labels, C, scale, row_loss, oh, ldo, \
-                                                argmax, dt, static_cast<uint16_t *>(probs), ldp)
-        if (aligned && C4 <= kNT * 1)
-            FG_SM_LAUNCH(1);
-        else if (aligned && C4 <= kNT * 4)
-            FG_SM_LAUNCH(4);
-        else if (aligned && C4 <= kNT * 16)
-            FG_SM_LAUNCH(16);
-        else if (aligned && C4 <= kNT * 32)
-            FG_SM_LAUNCH(32);
-        else
-            softmax_rows_stream<<<grid, block, 0, st>>>(x, ldx, labels, C, scale, row_loss, out,
-                                                        ldo, argmax, dt, probs, ldp);
-#undef FG_SM_LAUNCH
+        softmax_rows_stream<<<R, kNT, 0, st>>>(x, ldx, labels, C, scale, row_loss, out, ldo,
+                                               argmax, dt, probs, ldp);
     }
     FG_LAUNCH_CHECK("softmax_rows");
     return FG_OK;
@@ -719,7 +657,16 @@ FG_API int fg_softmax_bwd(fg_ctx *ctx, int dtype, const void *d_y, const void *d
     FG_REQUIRE(R >= 0 && C > 0, FG_ERR_SHAPE, "fg_softmax_bwd: bad shape R=%d C=%d", R, C);
     if (R == 0) return FG_OK;
     FG_HIP(hipSetDevice(ctx->device));
-    softmax_bwd_rows<<<R, kNT, 0, ctx->stream>>>(d_y, d_dy, C, d_dx, accumulate, dtype);
+    if (same_phase(dtype, d_y, C, d_dy, C, R) && same_phase(dtype, d_y, C, d_dx, C, R)) {
+        if (dtype == FG_DTYPE_F32)
+            launch_bwd_any<fg::kF32>(ctx->stream, d_y, d_dy, R, C, d_dx, accumulate);
+        else if (dtype == FG_DTYPE_BF16)
+            launch_bwd_any<fg::kBF16>(ctx->stream, d_y, d_dy, R, C, d_dx, accumulate);
+        else
+            launch_bwd_any<fg::kF16>(ctx->stream, d_y, d_dy, R, C, d_dx, accumulate);
+    } else {
+        softmax_bwd_rows<<<R, kNT, 0, ctx->stream>>>(d_y, d_dy, C, d_dx, accumulate, dtype);
+    }
     FG_LAUNCH_CHECK("softmax_bwd_rows");
     return FG_OK;
 }

@@ -756,6 +756,89 @@ def test_softmax_and_backward(gpu_ctx):
         assert normwise_rel(host(dx), O.softmax_bwd(host(y), dy)) < 1e-5
 
 
+# Columns at the edges of the row kernels' capacities: 64 / 128 / 256 / 512 /
+# 1024 / 2048 / 4096 / 8192 chunks of 4 (fp32) or 8 (16-bit) elements, and past.
+@pytest.mark.parametrize("place", ["aligned", "offset", "out-of-phase", "in-place"])
+@pytest.mark.parametrize("dtype", [0, 1, 2], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("chunks", [1, 64, 128, 256, 512, 1024, 2048, 4096, 8192, 12000])
+def test_softmax_rows_any(gpu_ctx, chunks, dtype, place):
+    """softmax + CE and the plain softmax's backward on rows of any length,
+    against float64: rows that start anywhere against 16-byte boundaries,
+    outputs that start elsewhere than the logits, outputs over the logits; a
+    row half -inf, a row of the type's lowest value, ties."""
+    torch = _torch()
+    E, dt = (4, torch.float32) if dtype == 0 else (8, [None, torch.float16, torch.bfloat16][dtype])
+    # Unit of the stored type (round to nearest: half of it), and its least spacing.
+    unit = {0: 2.0 ** -24, 1: 2.0 ** -11, 2: 2.0 ** -8}[dtype]
+    tiny = {0: 0.0, 1: 2.0 ** -25, 2: 0.0}[dtype]
+    off = 0 if place == "aligned" else 1
+    for C in (chunks * E - 1, chunks * E, chunks * E + E + 3):
+        R = 6 if C > 70 else 1030  # (few short rows take the one-workgroup kernels)
+        note(f"softmax_rows_any dtype={dtype} C={C} {place}")
+        g = torch.Generator().manual_seed(C)
+        x = (2 * torch.randn(R, C, generator=g)).to(dt)
+        x[1, : C // 2] = float("-inf")
+        x[2, :] = torch.finfo(dt).min
+        x[3, C // 3] = x[3, C // 2] = 60.0
+        lab = torch.randint(0, C, (R,), generator=g, dtype=torch.int32)
+        lab[1] = C - 1
+        xd = x.double()
+        m = xd.max(1, keepdim=True).values
+        e = torch.exp(xd - m)
+        s = e.sum(1, keepdim=True)
+        p = e / s
+        rows = (m + torch.log(s)).squeeze(1) - xd.gather(1, lab.long()[:, None]).squeeze(1)
+        ref = p.clone()
+        ref[torch.arange(R), lab.long()] -= 1.0
+        first = (xd == m).int().argmax(1)
+
+        def put(t, at):  # t in device memory, `at` elements past an aligned start
+            b = torch.zeros(t.numel() + 64, dtype=t.dtype, device="cuda")
+            b[at:at + t.numel()] = t.reshape(-1).cuda()
+            return b, b[at:at + t.numel()]
+
+        _, dx = put(x, off)
+        if place == "in-place":
+            out = dx
+        else:
+            _, out = put(torch.zeros_like(x), off + (1 if place == "out-of-phase" else 0))
+        dl = lab.cuda()
+        loss, am = empty((R,)), empty((R,), torch.int32)
+        gpu_ctx.softmax_ce(dx, C, dl, R, C, 1.0, row_loss=loss, dlogits=out, ldd=C, argmax=am,
+                           dtype=dtype)
+        torch.cuda.synchronize()
+        assert torch.equal(am.cpu().long(), first)
+        fin = torch.isfinite(rows)
+        # The loss is (max + log s) - x_label in fp32: the first sum rounds at
+        # the maximum's magnitude.
+        bound = 1e-6 * rows.abs().clamp(min=1) + 2.0 ** -23 * m.squeeze(1).abs()
+        assert ((loss.cpu().double() - rows).abs() <= bound)[fin].all()
+        err = (out.view(R, C).cpu().double() - ref).abs()
+        # p in fp32 is off by its exponential's argument rounding: 2.5e-7.
+        assert (err <= unit * ref.abs() + tiny + 2.5e-7).all(), float(err.max())
+        if place == "in-place":
+            continue
+        # Plain softmax of the same logits, then its backward.
+        _, y = put(torch.zeros_like(x), off + (1 if place == "out-of-phase" else 0))
+        gpu_ctx.softmax(dx, R, C, y, dtype=dtype)
+        torch.cuda.synchronize()
+        yh = y.view(R, C).cpu()
+        assert ((yh.double() - p).abs() <= unit * p + tiny + 2.5e-7).all()
+        dy = torch.randn(R, C, generator=g).to(dt)
+        old = torch.randn(R, C, generator=g).to(dt)
+        _, ddy = put(dy, off)
+        for acc in (False, True):
+            _, gx = put(old, off)
+            gpu_ctx.softmax_bwd(y, ddy, R, C, gx, accumulate=acc, dtype=dtype)
+            torch.cuda.synchronize()
+            yd, dyd = yh.double(), dy.double()
+            rb = yd * (dyd - (yd * dyd).sum(1, keepdim=True)) + (old.double() if acc else 0.0)
+            # fp32 dot product of terms y * dy (sum of |y| is 1), then one rounding.
+            big = dyd.abs().amax(1, keepdim=True)
+            e2 = (gx.view(R, C).cpu().double() - rb).abs()
+            assert (e2 <= unit * rb.abs() + tiny + 1e-6 * (yd * big + acc)).all(), float(e2.max())
+
+
 # ------------------------------------------------------------ optimisers
 SIZES = [1, 3, 4096, 4097, 100003, 262144]
 
