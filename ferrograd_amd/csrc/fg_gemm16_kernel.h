@@ -1203,6 +1203,12 @@ __global__ __launch_bounds__(256) void sum_slices16(Args p, int splits) {
     }
 }
 
+template <bool BF>
+void launch_sum16(const Args &a, int splits, hipStream_t st) {
+    const int64_t threads = (int64_t)a.M * ((a.N + 3) / 4);
+    sum_slices16<BF><<<(unsigned)((threads + 255) / 256), 256, 0, st>>>(a, splits);
+}
+
 template <int BM, int BN, int WGM, int WGN, int BK, bool AK, bool BNC, bool BF, bool KT = false>
 void launch_pipe16(const Args &a0, hipStream_t st) {
     Args a = a0;
@@ -1211,10 +1217,7 @@ void launch_pipe16(const Args &a0, hipStream_t st) {
     const int splits = a.ksplit > 0 ? (a.K + a.ksplit - 1) / a.ksplit : 1;
     gemm16_pipe<BM, BN, BK, WGM, WGN, AK, BNC, BF, KT>
         <<<dim3(a.tiles_m * a.tiles_n, splits), 64 * WGM * WGN, 0, st>>>(a);
-    if (splits > 1) {
-        const int64_t threads = (int64_t)a.M * ((a.N + 3) / 4);
-        sum_slices16<BF><<<(unsigned)((threads + 255) / 256), 256, 0, st>>>(a, splits);
-    }
+    if (splits > 1) launch_sum16<BF>(a, splits, st);
 }
 
 template <int BM, int BN, int WGM, int WGN, int BK, bool AK, bool BNC, bool VEC, bool BF>
@@ -1276,6 +1279,9 @@ void launch_layout(const Args &a, bool vec, bool pipe, int cfg, hipStream_t st) 
 // Defined in k_gemm16_{bf16,f16}.hip.  layout: FG_NN / FG_NT / FG_TN.
 void launch_bf16(int layout, const Args &a, bool vec, bool pipe, int cfg, hipStream_t st);
 void launch_f16(int layout, const Args &a, bool vec, bool pipe, int cfg, hipStream_t st);
+// sum_slices16 of a's slots.
+void launch_sum_bf16(const Args &a, int splits, hipStream_t st);
+void launch_sum_f16(const Args &a, int splits, hipStream_t st);
 // gemm16_pair_big: dW (TN, a1) and dX (NT, a2), both planned pipelined on
 // kPair16CfgW / kPair16CfgX without a K split.
 void launch_pair_bf16(const Args &a1, const Args &a2, hipStream_t st);

@@ -9,6 +9,7 @@
 
 #include "fg_bias_grad.h"
 #include "fg_gemm_kernel.h"
+#include "fg_gemm_rows.h"
 #include "fg_gemm_skinny.h"
 #include "fg_half.h"
 #include "fg_internal.h"
@@ -142,16 +143,30 @@ bool use_skinny(fg_ctx *ctx, const GemmArgs &a, int pro) {
            a.K <= fg::gemm::kSkinnyK && (int64_t)a.M <= 16LL * cus;
 }
 
+// Few output rows (a small batch): the kernel of fg_gemm_rows.h up to 32
+// rows, where it beat the tiles at every size (us: 16 x 4096 x 4096 65.6 ->
+// 18.7, 32 x 1000 x 4096 19.0 -> 11.4, 32 x 256 x 784 9.9 -> 8.3), and up to 64
+// where reading B outweighs the fp32 matrix units' time (64 x 4096 x 4096 67.5
+// -> 40.4, 48 x 4096 x 1024 16.4 -> 14.6; but 64 x 1001 x 1001 16.5 -> 18.9, 64 x
+// 256 x 784 10.5 -> 14.4).  A data gradient of a small layer (under 2^20
+// weights) stays with the tiles, in one launch with its weight gradient.
+bool use_rows(int layout, const GemmArgs &a, int pro) {
+    const int64_t nk = (int64_t)a.N * a.K;
+    return pro == fg::gemm::kProNone && !a.colsum &&
+           fg::rows::applies(layout, a.M, a.N, a.K) && (a.M <= 32 || nk >= 1 << 22) &&
+           (a.mode == 0 || nk >= 1 << 20);
+}
+
 // The kernel choices of one GEMM call (sets a.vec_out, and a.partial /
 // a.ksplit when K is split): the skinny kernel (skinny; then nothing else
 // applies), 16-byte operand loads (vec), the pipelined kernel (pipe) and
 // whether its last K tile is partial (ktail), the tile configuration and the
 // number of K slices.  pro: the prologue code (fg::gemm::kPro*), whose
 // tensor Pz must meet the same 16-byte conditions as the operand it scales.
-void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &vec, bool &pipe,
-               bool &ktail, int &cfg, int &splits, int pro = fg::gemm::kProNone) {
+void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &rows, bool &vec,
+               bool &pipe, bool &ktail, int &cfg, int &splits, int pro = fg::gemm::kProNone) {
     skinny = use_skinny(ctx, a, pro);
-    vec = pipe = ktail = false;
+    vec = pipe = ktail = rows = false;
     cfg = 0;
     splits = 1;
     if (skinny) return;
@@ -179,6 +194,17 @@ void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &vec, bo
     // masked).  A partial last K tile (K % BK != 0) is zero-filled by the
     // staged-tile instances (ktail); the prologue instances need whole tiles
     // and leave such shapes to gemm_f32_mfma.
+    rows = use_rows(layout, a, pro);
+    if (rows) {
+        int ks;
+        splits = fg::rows::split_of(ctx->cu_count > 0 ? ctx->cu_count : 256, 4, a.M, a.N, a.K,
+                                    ctx->ws_bytes, ks);
+        if (splits > 1) {
+            a.partial = static_cast<float *>(ctx->ws);
+            a.ksplit = ks;
+        }
+        return;
+    }
     pipe = fg::gemm::kPipe && vec && a.K > 0 && a.M >= 4 && a.N >= 4;
     ktail = false;
     if (pipe && a.K % fg::gemm::cfg_bk(cfg) != 0) {
@@ -197,7 +223,7 @@ void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &vec, bo
 struct Planned {
     GemmArgs a{};
     int layout = FG_NN, pro = fg::gemm::kProNone, cfg = 0, splits = 1;
-    bool skinny = false, vec = false, pipe = false, ktail = false;
+    bool skinny = false, rows = false, vec = false, pipe = false, ktail = false;
     bool empty = false;  // M == 0 or N == 0: nothing to launch
 };
 
@@ -226,7 +252,7 @@ int gemm_prepare(fg_ctx *ctx, int layout, const GemmArgs &a0, const char *who, i
                a.ldb, a.ldc);
     FG_HIP(hipSetDevice(ctx->device));
     if (a.K == 0) a.A = a.B;  // loads are all masked; K=0 yields the epilogue of zero
-    plan_gemm(ctx, layout, a, P.skinny, P.vec, P.pipe, P.ktail, P.cfg, P.splits, pro);
+    plan_gemm(ctx, layout, a, P.skinny, P.rows, P.vec, P.pipe, P.ktail, P.cfg, P.splits, pro);
     return FG_OK;
 }
 
@@ -250,7 +276,9 @@ int gemm_launch(fg_ctx *ctx, const Planned &P, const char *who, bool reduce = tr
         FG_LAUNCH_CHECK(who);
         return FG_OK;
     }
-    switch (P.layout) {
+    if (P.rows)
+        fg::rows::launch_f32(P.layout, P.a, ctx->stream);
+    else switch (P.layout) {
         case FG_NN: fg::gemm::launch_nn(P.a, P.vec, P.pipe, P.ktail, P.cfg, ctx->stream); break;
         case FG_NT:
             fg::gemm::launch_nt(P.a, P.vec, P.pipe, P.ktail, P.cfg, P.pro, ctx->stream);
@@ -275,7 +303,7 @@ int gemm_common(fg_ctx *ctx, int layout, GemmArgs &a, const char *who,
 
 // The pair kernel that a planned GEMM would take (-1: it does not pair).
 int pair_kind(const Planned &P) {
-    if (P.empty || P.pro != fg::gemm::kProNone) return -1;
+    if (P.empty || P.rows || P.pro != fg::gemm::kProNone) return -1;
     if (P.skinny) return fg::gemm::kPairSkinny;
     if (!P.vec) return fg::gemm::kPairElem;
     if (P.pipe && !P.ktail && P.cfg == 4) return fg::gemm::kPairPipe;
@@ -380,9 +408,9 @@ int gemm_f32_dispatches(fg_ctx *ctx, int layout, int M, int N, int K, const void
     a.ldb = ldb;
     a.colsum = colsum ? reinterpret_cast<float *>(1) : nullptr;  // only tested for null
     if (K == 0) a.A = a.B;
-    bool skinny, vec, pipe, ktail;
+    bool skinny, rows, vec, pipe, ktail;
     int cfg, splits;
-    plan_gemm(ctx, layout, a, skinny, vec, pipe, ktail, cfg, splits);
+    plan_gemm(ctx, layout, a, skinny, rows, vec, pipe, ktail, cfg, splits);
     return splits > 1 ? 2 : 1;
 }
 }  // namespace fg
@@ -587,7 +615,7 @@ void plan_quiet(fg_ctx *ctx, int layout, const GemmArgs &a0, Planned &P) {
     const float *aligned = reinterpret_cast<const float *>(256);
     if (!P.a.A) P.a.A = aligned;
     if (!P.a.B) P.a.B = aligned;
-    plan_gemm(ctx, layout, P.a, P.skinny, P.vec, P.pipe, P.ktail, P.cfg, P.splits);
+    plan_gemm(ctx, layout, P.a, P.skinny, P.rows, P.vec, P.pipe, P.ktail, P.cfg, P.splits);
 }
 }  // namespace
 

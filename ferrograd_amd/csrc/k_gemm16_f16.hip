@@ -19,5 +19,9 @@ void launch_pair_f16(const Args &a1, const Args &a2, hipStream_t st) {
     launch_pair16<false>(a1, a2, st);
 }
 
+void launch_sum_f16(const Args &a, int splits, hipStream_t st) {
+    launch_sum16<false>(a, splits, st);
+}
+
 }  // namespace gemm16
 }  // namespace fg

@@ -648,6 +648,69 @@ def test_act_bwd_parity(gpu_ctx, n):
     assert np.max(np.abs(host(out) - ref) / np.maximum(np.abs(ref), 1.0)) < 1e-5
 
 
+# Few-row GEMMs: a whole step, its remainders, the columns' and rows' edges,
+# odd rows; 4100 and more of K split it.
+@pytest.mark.parametrize("place", ["plain", "padded", "offset"])
+@pytest.mark.parametrize("layout", [O.NN, O.NT], ids=["NN", "NT"])
+@pytest.mark.parametrize("dtype", [0, 1, 2], ids=["f32", "f16", "bf16"])
+def test_gemm_few_rows(gpu_ctx, dtype, layout, place):
+    """Small-integer operands (every sum exact in fp32, whatever its order),
+    with NaN around every row (padded) and before and after the tensors:
+    outputs bit for bit, forward with bias + ReLU + Z, backward through a ReLU
+    mask, C +=."""
+    torch = _torch()
+    dt = [torch.float32, torch.float16, torch.bfloat16][dtype]
+    gpu_ctx.reserve_workspace(8 << 20)
+    g = torch.Generator().manual_seed(7)
+
+    def ints(r, c, lim):  # a [r][c] tensor inside NaN, its leading dimension
+        ld = c + (3 if place == "padded" else 0)
+        off = 1 if place == "offset" else 64
+        v = torch.randint(-lim, lim + 1, (r, c), generator=g).to(dt)
+        buf = torch.full((off + r * ld + 64,), float("nan"), dtype=dt)
+        buf[off:off + r * ld].view(r, ld)[:, :c] = v
+        buf = buf.cuda()
+        return v.double(), buf, buf[off:], ld
+
+    for M, N, K in [(1, 2, 1), (1, 33, 129), (16, 31, 64), (17, 100, 63), (33, 64, 517),
+                    (64, 95, 1024), (7, 1000, 4100), (32, 129, 8191), (64, 2100, 2050)]:
+        if dtype == 0 and M > 32 and N * K < 1 << 22:
+            M = 30  # (the fp32 kernel's range)
+        note(f"gemm_few_rows {dtype} {layout} {place} {M}x{N}x{K}")
+        a, _ka, A, lda = ints(M, K, 2)
+        b, _kb, B, ldb = ints(*((K, N) if layout == O.NN else (N, K)), 2)
+        bias, _kc, dbias, _ = ints(1, N, 4)
+        zs, _kd, dZs, ldzs = ints(M, N, 1)
+        old, _ke, C, ldc = ints(M, N, 8)
+        v = (a @ (b if layout == O.NN else b.T)).to(dt)
+        z = (v.double() + bias).to(dt)
+        Z = torch.empty(M, N, dtype=dt, device="cuda")
+
+        def got(t, ld):
+            torch.cuda.synchronize()
+            return t[:M * ld].view(M, ld)[:, :N].cpu()
+
+        def call(mode, acc, act):
+            kw = dict(act=act, accumulate=acc)
+            if mode == 0:
+                kw.update(bias=dbias, Z=Z, ldz=N)
+            else:
+                kw.update(Zs=dZs, ldzs=ldzs)
+            args = (layout, M, N, K, A, lda, B, ldb, C, ldc)
+            if dtype == 0:
+                (gpu_ctx.gemm if mode == 0 else gpu_ctx.gemm_bwd)(*args, **kw)
+            else:
+                (gpu_ctx.gemm_x16 if mode == 0 else gpu_ctx.gemm_bwd_x16)(dtype, *args, **kw)
+
+        call(0, True, O.ACT_NONE)
+        assert torch.equal(got(C, ldc), (z.double() + old).to(dt))
+        call(0, False, O.ACT_RELU)
+        assert torch.equal(got(C, ldc), z.clamp(min=0))
+        assert torch.equal(Z.cpu(), z)
+        call(1, False, O.ACT_RELU)
+        assert torch.equal(got(C, ldc), torch.where(zs > 0, v, torch.zeros_like(v)))
+
+
 # --------------------------------------------------------- softmax + CE
 def check_softmax_ce(ctx, x, labels, scale=1.0):
     torch = _torch()
