@@ -41,6 +41,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "fg_act.h"
 #include "fg_sched.h"
 
@@ -49,6 +52,9 @@ namespace gemm {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+// Four floats anywhere: 16-byte accesses need 4-byte alignment only, and cost
+// no more for rows that start between 16-byte boundaries.
+typedef f32x4 f32x4_u __attribute__((aligned(4)));
 
 constexpr int kThreads = 256;
 
@@ -89,7 +95,7 @@ struct GemmArgs {
     int mode;  // 0 forward epilogue, 1 backward (act-derivative) epilogue
     int accumulate;
     int tiles_m, tiles_n;
-    int vec_out;  // C (and Z / Zs) rows 16-byte aligned: float4 epilogue I/O
+    int vec_out;  // C and Z rows and the bias 16-byte aligned (the chained skinny kernel)
     // TN only: colsum[n] (=|+=) sum_k B[k][n] -- the bias gradient of the
     // layer whose weight gradient this GEMM computes -- taken from the B
     // tiles already in LDS by the workgroups of the first tile row.
@@ -98,8 +104,10 @@ struct GemmArgs {
     // Split K (0: off): workgroup row blockIdx.y multiplies the K slice
     // [ksplit * y, ksplit * (y + 1)) into its own M x N slot of `partial`
     // (row stride N); splitk_reduce then sums the slots in order and applies
-    // the epilogue.
+    // the epilogue.  With colsum, slice y leaves its N column sums in slot y
+    // of colsum_partial, which splitk_reduce sums alike.
     float *partial;
+    float *colsum_partial;
     int ksplit;
     // Prologue (kernels instantiated with PRO != 0): the operand that holds
     // dC -- A of NT (dA = dZ.B^T) or B of TN (dB = A^T.dZ) -- is multiplied
@@ -144,8 +152,10 @@ __device__ __forceinline__ void split_k_view(GemmArgs &p, int s) {
     p.bias = nullptr;
     p.Z = nullptr;
     p.accumulate = 0;
-    p.colsum = nullptr;
-    p.vec_out = p.N % 4 == 0;
+    if (p.colsum) {  // this slice's column sums, after the output slots
+        p.colsum = p.colsum_partial + (size_t)s * p.N;
+        p.colsum_accumulate = 0;
+    }
 }
 
 // Column sums of the B tiles (TN layout, B row-contiguous [k][n]) for the
@@ -312,31 +322,6 @@ __device__ __forceinline__ float epi_value(const GemmArgs &p, float v, float bv,
     return v;
 }
 
-// Split K: output (row, col) of the whole product -- the slots' raw
-// products summed in slot order, then the epilogue (splitk_reduce and the
-// summing blocks of the fused SGD launch, k_optim.hip).
-__device__ __forceinline__ void split_sum_store(const GemmArgs &p, int splits, int row, int col) {
-    const size_t mn = (size_t)p.M * p.N, i = (size_t)row * p.N + col;
-    float v = p.partial[i];
-    for (int s = 1; s < splits; ++s) v += p.partial[s * mn + i];
-    const float b = (p.mode == 0 && p.bias) ? p.bias[col] : 0.0f;
-    float z;
-    float o = epi_value(p, v, b, row, col, &z);
-    if (p.mode == 0 && p.Z) p.Z[(size_t)row * p.ldz + col] = z;
-    float *c = p.C + (size_t)row * p.ldc + col;
-    if (p.accumulate) o += *c;  // (in its own statement: no contraction with o)
-    *c = o;
-}
-
-// Blocks [0, nblocks) of a summing pass over M x N outputs, block b of them
-// (kThreads threads, grid-stride).
-__device__ __forceinline__ void split_sum_blocks(const GemmArgs &p, int splits, int b,
-                                                 int nblocks) {
-    const size_t mn = (size_t)p.M * p.N;
-    for (size_t i = (size_t)b * kThreads + threadIdx.x; i < mn; i += (size_t)nblocks * kThreads)
-        split_sum_store(p, splits, (int)(i / p.N), (int)(i % p.N));
-}
-
 // Four consecutive outputs of one row (the vector path of the epilogue):
 // the same operations as epi_value per element, with the uniform choices
 // (mode, activation, Z, accumulate) taken once per four.  Returns the four
@@ -345,20 +330,75 @@ __device__ __forceinline__ f32x4 epi_x4(const GemmArgs &p, f32x4 v, f32x4 bv, in
 #pragma clang fp contract(off)
     if (p.mode == 0) {
         v += bv;
-        if (p.Z) *reinterpret_cast<f32x4 *>(p.Z + (size_t)row * p.ldz + col) = v;
+        if (p.Z) *reinterpret_cast<f32x4_u *>(p.Z + (size_t)row * p.ldz + col) = v;
         if (p.act != kActNone) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) v[t] = act_fwd(p.act, v[t]);
         }
     } else if (p.act != kActNone) {
-        const f32x4 z = *reinterpret_cast<const f32x4 *>(p.Zs + (size_t)row * p.ldzs + col);
+        const f32x4 z = *reinterpret_cast<const f32x4_u *>(p.Zs + (size_t)row * p.ldzs + col);
 #pragma unroll
         for (int t = 0; t < 4; ++t) v[t] *= act_grad(p.act, z[t]);
     }
     float *c = p.C + (size_t)row * p.ldc + col;
-    if (p.accumulate) v += *reinterpret_cast<const f32x4 *>(c);
-    *reinterpret_cast<f32x4 *>(c) = v;
+    if (p.accumulate) v += *reinterpret_cast<const f32x4_u *>(c);
+    *reinterpret_cast<f32x4_u *>(c) = v;
     return v;
+}
+
+// Split K: the slots' values at offset i, summed in slot order (loads of
+// four slots in flight).
+template <class V>
+__device__ __forceinline__ V slot_sum(const float *src, size_t stride, int splits) {
+    typedef V VU __attribute__((aligned(4)));
+    V v = *reinterpret_cast<const VU *>(src);
+    int s = 1;
+    for (; s + 4 <= splits; s += 4) {
+        V x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = *reinterpret_cast<const VU *>(src + (s + q) * stride);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v += x[q];
+    }
+    for (; s < splits; ++s) v += *reinterpret_cast<const VU *>(src + s * stride);
+    return v;
+}
+
+// Blocks [0, nblocks) of a summing pass over M x N outputs, block b of them
+// (kThreads threads, grid-stride): the slots' raw products summed in slot
+// order, then the epilogue (splitk_reduce and the summing blocks of the fused
+// SGD launch, k_optim.hip); and the column sums' slots.
+__device__ __forceinline__ void split_sum_blocks(const GemmArgs &p, int splits, int b,
+                                                 int nblocks) {
+    const size_t mn = (size_t)p.M * p.N, step = (size_t)nblocks * kThreads;
+    const size_t first = (size_t)b * kThreads + threadIdx.x;
+    if (p.N % 4 == 0) {
+        const size_t g4 = p.N / 4;
+        for (size_t q = first; q < mn / 4; q += step) {
+            const int row = (int)(q / g4), col = (int)(q % g4) * 4;
+            const f32x4 v = slot_sum<f32x4>(p.partial + 4 * q, mn, splits);
+            f32x4 bv = {0.f, 0.f, 0.f, 0.f};
+            if (p.mode == 0 && p.bias) bv = *reinterpret_cast<const f32x4_u *>(p.bias + col);
+            (void)epi_x4(p, v, bv, row, col);
+        }
+    } else {
+        for (size_t i = first; i < mn; i += step) {
+            const int row = (int)(i / p.N), col = (int)(i % p.N);
+            const float v = slot_sum<float>(p.partial + i, mn, splits);
+            const float bias = (p.mode == 0 && p.bias) ? p.bias[col] : 0.0f;
+            float z;
+            float o = epi_value(p, v, bias, row, col, &z);
+            if (p.mode == 0 && p.Z) p.Z[(size_t)row * p.ldz + col] = z;
+            float *c = p.C + (size_t)row * p.ldc + col;
+            if (p.accumulate) o += *c;  // (in its own statement: no contraction with o)
+            *c = o;
+        }
+    }
+    if (p.colsum)
+        for (size_t i = first; i < (size_t)p.N; i += step) {
+            const float v = slot_sum<float>(p.colsum_partial + i, p.N, splits);
+            p.colsum[i] = p.colsum_accumulate ? p.colsum[i] + v : v;
+        }
 }
 
 // Epilogue shared by the GEMM kernels.  Accumulator register r of lane
@@ -388,9 +428,9 @@ __device__ __forceinline__ void store_tile(const GemmArgs &p, const f32x16 (&acc
     static_assert(64 % F4 == 0 && 32 % RPP == 0, "epilogue lane mapping");
     const int c4 = (lane % F4) * 4, rr0 = lane / F4;
     const int col = c0 + c4;
-    const bool vec = p.vec_out && col + 4 <= p.N;
+    const bool vec = col + 4 <= p.N;
     f32x4 bv = {0.f, 0.f, 0.f, 0.f};
-    if (p.mode == 0 && p.bias && vec) bv = *reinterpret_cast<const f32x4 *>(p.bias + col);
+    if (p.mode == 0 && p.bias && vec) bv = *reinterpret_cast<const f32x4_u *>(p.bias + col);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -429,7 +469,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs &p, const f32x16 (&acc
 
 // ------------------------------------------------ register epilogue
 // The pipelined kernels' epilogue when the workgroup's whole tile is in
-// bounds and rows are 16-byte aligned: no LDS, no workgroup barrier.
+// bounds: no LDS, no workgroup barrier.
 // Accumulator registers 4k .. 4k+3 of lane (h, l32) hold rows x = 8k + 4h +
 // 0..3 of a block's column; the block's rows and columns in C follow
 // store_tile's mapping (interleaved or not).  Without column interleave, a
@@ -454,7 +494,7 @@ __device__ __forceinline__ void epi_x4_k(const GemmArgs &p, f32x4 v, f32x4 bv, f
 #pragma clang fp contract(off)
     if constexpr (MODE == 0) {
         v += bv;
-        if (p.Z) *reinterpret_cast<f32x4 *>(p.Z + (size_t)row * p.ldz + col) = v;
+        if (p.Z) *reinterpret_cast<f32x4_u *>(p.Z + (size_t)row * p.ldz + col) = v;
         if constexpr (ACT != kActNone) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) v[t] = act_fwd(ACT, v[t]);
@@ -464,8 +504,8 @@ __device__ __forceinline__ void epi_x4_k(const GemmArgs &p, f32x4 v, f32x4 bv, f
         for (int t = 0; t < 4; ++t) v[t] *= act_grad(ACT, z[t]);
     }
     float *c = p.C + (size_t)row * p.ldc + col;
-    if (p.accumulate) v += *reinterpret_cast<const f32x4 *>(c);
-    *reinterpret_cast<f32x4 *>(c) = v;
+    if (p.accumulate) v += *reinterpret_cast<const f32x4_u *>(c);
+    *reinterpret_cast<f32x4_u *>(c) = v;
 }
 
 template <int TM, int TN, int IA, int IB, int MODE, int ACT>
@@ -481,7 +521,7 @@ __device__ __forceinline__ void store_direct_k(const GemmArgs &p, const f32x16 (
         for (int j = 0; j < TN; ++j) {
             const int col = c0 + 32 * j + a4;
             f32x4 bv = {0.f, 0.f, 0.f, 0.f};
-            if (MODE == 0 && p.bias) bv = *reinterpret_cast<const f32x4 *>(p.bias + col);
+            if (MODE == 0 && p.bias) bv = *reinterpret_cast<const f32x4_u *>(p.bias + col);
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
                 const f32x16 &a = acc[i][j];
@@ -490,7 +530,7 @@ __device__ __forceinline__ void store_direct_k(const GemmArgs &p, const f32x16 (
                 if constexpr (kZs) {
 #pragma unroll
                     for (int k = 0; k < 4; ++k)
-                        zr[k] = *reinterpret_cast<const f32x4 *>(
+                        zr[k] = *reinterpret_cast<const f32x4_u *>(
                             p.Zs + (size_t)crow(i, 8 * k + 4 * h + e) * p.ldzs + col);
                 }
 #pragma unroll 1
@@ -508,6 +548,7 @@ __device__ __forceinline__ void store_direct_k(const GemmArgs &p, const f32x16 (
         }
     } else {
         typedef float vec_t __attribute__((ext_vector_type(IB)));
+        typedef vec_t vec_u __attribute__((aligned(4)));
         const int col = c0 + TN * l32;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -523,8 +564,8 @@ __device__ __forceinline__ void store_direct_k(const GemmArgs &p, const f32x16 (
                                0.0f;
                     }
                     float *c = p.C + (size_t)crow(i, 8 * k + 4 * h + q) * p.ldc + col;
-                    if (p.accumulate) v += *reinterpret_cast<const vec_t *>(c);
-                    *reinterpret_cast<vec_t *>(c) = v;
+                    if (p.accumulate) v += *reinterpret_cast<const vec_u *>(c);
+                    *reinterpret_cast<vec_u *>(c) = v;
                 }
     }
 }
@@ -709,10 +750,15 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_f32_mfma(GemmArgs p) {
     gemm_f32_mfma_body<BM, BN, BK, WGM, WGN, AK, BNC, VEC, PRO>(p, blockIdx.x, blockIdx.y);
 }
 
-// KT: K need not be a multiple of BK (staged tiles, no prologue): the tile
-// loop runs over the whole tiles only, and the K % BK values of k past them
-// are multiplied into the accumulators straight from global memory at the
-// end (see the K tail below), so the loop keeps the whole-tile addressing.
+// KT: any K and any rows (staged tiles, no prologue; M, N >= 4): the tile
+// loop runs over the whole tiles only, and the values of k past them are
+// multiplied into the accumulators straight from global memory at the end
+// (see the K tail below), so the loop keeps the whole-tile addressing.  Rows
+// that are not 16-byte aligned take it too: what bounds it there is what bounds
+// aligned rows, as 16-byte loads at 4-byte alignment cost no more.  Against
+// one element a lane on 64x64 tiles (us): 2047 x 4095 x 4093 NN 813.7 -> 501.3,
+// 1000 x 2003 x 1501 NN 104.8 -> 70.3, its layer's TN and NT 98.4 / 121.5 -> 77.9 /
+// 78.6 (with the same tiles as then: see choose in k_gemm.hip).
 // LDS of the pipelined kernel, in floats: its stages (staged tiles: two;
 // direct: three when they fit in the 160 KiB of LDS, else two) or the
 // epilogue's staging, whichever is larger.
@@ -724,6 +770,25 @@ struct PipeLds {
     static constexpr int kEpi = WGM * WGN * 32 * (BN / WGN + 4);
     static constexpr int floats = (kStages * kStageSz > kEpi) ? kStages * kStageSz : kEpi;
 };
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>), in order.
+template <class F, int... I>
+__device__ __forceinline__ void each_of_seq(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void each_of(F f) {
+    each_of_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// Register sets of a staged tile, i.e. tiles in flight.  A 64x64 tile is a
+// quarter of a microsecond of MFMAs, less than a load takes, and often the only
+// workgroup of its CU: with four sets instead of two 1024^3 took 20.5 us for
+// 25.5, 1024 x 1024 x 2048 NT 35.8 for 42.8 (six: no better; the 128x64 tiles,
+// twice the time: 2, 3 and 4 sets alike).
+constexpr int staged_sets(int BM, int BN, int pro) {
+    return pro == kProNone && BM * BN <= 64 * 64 ? 4 : 2;
+}
 
 // The kernel's LDS buffer of N floats: one static array per N, so bodies
 // that ask for the same N in one launch share it.
@@ -738,6 +803,8 @@ __device__ __forceinline__ float (&lds_buffer())[N] {
 template <int BM, int BN, int BK, int WGM, int WGN, bool AK, bool BNC, int PRO, bool KT,
           int LDSN = 0>
 __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
+    // This workgroup's K ends where the operands do.
+    const bool last = p.ksplit <= 0 || (by + 1) * p.ksplit >= p.K;
     split_k_view<AK, BNC, PRO>(p, by);
     constexpr int NW = WGM * WGN;
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
@@ -755,6 +822,7 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
     static_assert(PRO == kProNone || kStaged, "prologue needs the staged path");
     static_assert(!KT || (kStaged && PRO == kProNone), "K tail: staged tiles, no prologue");
     constexpr int kStages = PL::kStages;
+    constexpr int kSets = staged_sets(BM, BN, PRO);
     static_assert(LDSN == 0 || LDSN >= PL::floats, "LDS buffer too small");
     float(&lds)[LDSN ? LDSN : PL::floats] = lds_buffer<LDSN ? LDSN : PL::floats>();
 
@@ -789,7 +857,8 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
     auto src_rc = [&](const float *base, int ld, int r0, int rmax, int k0, int pos, int R) {
         const int k = pos / (R / 4), pc = pos % (R / 4);
         const int c = pc ^ swz_r(k);
-        return base + (size_t)(k0 + k) * ld + min(r0 + 4 * c, rmax - 4);
+        // (KT: a row's last chunk may end past it, in the next row.)
+        return base + (size_t)(k0 + k) * ld + min(r0 + 4 * c, KT ? (rmax - 1) & ~3 : rmax - 4);
     };
     // Wave load q (0 .. kLoads-1) of a tile: this wave's share of A first,
     // then of B.  Source of this lane's chunk, and its place in a stage.
@@ -826,7 +895,10 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
             __builtin_amdgcn_global_load_lds(src, sa + kASz + li * 256, 16, 0, 0);
         }
     };
-    auto load_reg = [&](int kt, int q) { return *reinterpret_cast<const f32x4 *>(src_of(kt, q)); };
+    auto load_reg = [&](int kt, int q) -> f32x4 {
+        if constexpr (KT) return *reinterpret_cast<const f32x4_u *>(src_of(kt, q));
+        else return *reinterpret_cast<const f32x4 *>(src_of(kt, q));
+    };
     auto store_reg = [&](int stage, int q, const f32x4 &v) {
         *reinterpret_cast<f32x4 *>(run_of(stage, q) + 4 * lane) = v;
     };
@@ -858,7 +930,11 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
         return R[q];
     };
 
-    const int nk = p.K / BK;  // whole tiles (KT: the rest is the K tail)
+    // Whole tiles (KT: the rest is the K tail).  A row-contiguous operand whose
+    // rows are not whole chunks leaves its last row to the tail: a chunk past
+    // the end of that row would be past the operand's end.
+    const bool ragged = KT && last && ((!AK && (p.M & 3)) || (BNC && (p.N & 3)));
+    const int nk = (p.K - (ragged ? 1 : 0)) / BK;
     constexpr bool kTN = !AK && BNC;
     ColSum<BN, BK, 64 * NW> cs;
     const bool do_cs = kTN && p.colsum && tile_m == 0;
@@ -1032,9 +1108,10 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
     // the barrier.  Past that barrier every wave holds all of tile kt's
     // operands and its stage may be refilled.
     f32x4 ca[TM], cb[TN];
+    // st: kt, or a number equal to it modulo kStages.
     auto tile = [&](int kt, int kl, int slot, const f32x4 *Rw, f32x4 *Rl, const f32x4 *Zw,
-                    f32x4 *Zl) {
-        const float *As = lds + (kt % kStages) * kStageSz;
+                    f32x4 *Zl, int st) {
+        const float *As = lds + (st % kStages) * kStageSz;
         const float *Bs = As + kASz;
         const int kst = min(kt + 1, nk - 1);  // staged: the tile Rw holds
 #pragma unroll
@@ -1063,7 +1140,7 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
         // Group 0 of tile kt+1 (past the last tile: a stage nothing uses,
         // read and discarded).
         f32x4 na[TM], nb[TN];
-        const float *An = lds + ((kt + 1) % kStages) * kStageSz;
+        const float *An = lds + ((st + 1) % kStages) * kStageSz;
         run_group(ca, cb, An, An + kASz, 0, na, nb, false, 0, 0, Rw, Rl, Zw, Zl, 0);
 #pragma unroll
         for (int i = 0; i < TM; ++i) ca[i] = na[i];
@@ -1071,47 +1148,46 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
         for (int j = 0; j < TN; ++j) cb[j] = nb[j];
     };
     if constexpr (kStaged) {
-        // Tile t is loaded into register set t % 2 during tile t-2 (one load
-        // after each of the first kLoads MFMAs of the tile's first group),
+        // Tile t is loaded into register set t % kSets during tile t-kSets (one
+        // load after each of the first kLoads MFMAs of the tile's first group),
         // and written from there to stage t % 2 during tile t-1 (the stage of
-        // tile t-2, free since the barrier that ended tile t-2); each write
-        // goes out right before the load that refills its registers.  Past
-        // the last tile, tile nk-1 is reloaded and written to the free stage,
-        // which nothing reads.  The kt loop is unrolled by two so that the
+        // tile t-2, free since the barrier that ended tile t-2); the set of
+        // tile t is free from then on and refilled during tile t.  Past the
+        // last tile, tile nk-1 is reloaded and written to the free stage,
+        // which nothing reads.  The kt loop is unrolled by kSets so that the
         // register sets swap roles without copies.
+        static_assert(kSets % 2 == 0, "stage parity");
         if (nk > 0) {
-            f32x4 R0[kLoads], R1[kLoads];
-            f32x4 Z0[kProN], Z1[kProN];  // prologue chunks (unused without PRO)
+            f32x4 R[kSets][kLoads];
+            f32x4 Z[kSets][kProN];  // prologue chunks (unused without PRO)
 #pragma unroll
-            for (int q = 0; q < kLoads; ++q) {
-                R0[q] = load_reg(0, q);
-                if constexpr (PRO != kProNone)
-                    if (is_pro(q)) Z0[q - kProFirst] = load_pz(0, q);
-            }
+            for (int d = 0; d < kSets; ++d)
 #pragma unroll
-            for (int q = 0; q < kLoads; ++q) {
-                R1[q] = load_reg(min(1, nk - 1), q);
-                if constexpr (PRO != kProNone)
-                    if (is_pro(q)) Z1[q - kProFirst] = load_pz(min(1, nk - 1), q);
-            }
+                for (int q = 0; q < kLoads; ++q) {
+                    R[d][q] = load_reg(min(d, nk - 1), q);
+                    if constexpr (PRO != kProNone)
+                        if (is_pro(q)) Z[d][q - kProFirst] = load_pz(min(d, nk - 1), q);
+                }
 #pragma unroll
-            for (int q = 0; q < kLoads; ++q) store_reg(0, q, staged_value(R0, Z0, q, 0));
+            for (int q = 0; q < kLoads; ++q) store_reg(0, q, staged_value(R[0], Z[0], q, 0));
             wait_lgkm0();
             asm volatile("s_barrier" ::: "memory");
             frag(lds, lds + kASz, 0, ca, cb);
-            // Tile kt writes the set holding tile kt+1 and refills the other
-            // with tile kt+2; that set was loaded a whole tile ago.
+            // Tile kt (set d) writes the set holding tile kt+1, which was
+            // loaded kSets-1 tiles ago: all but the newest kSets-2 sets have
+            // landed.
+            auto turn = [&](int kt, auto dc) {
+                constexpr int d = decltype(dc)::value, w = (d + 1) % kSets;
+                wait_vmcnt<(kSets - 2) * (kLoads + kPro)>();
+                tile(kt, min(kt + kSets, nk - 1), (d + 1) % kStages, R[w], R[d], Z[w], Z[d], d);
+            };
+            // (An even kSets, so that the stage of a turn is a constant too.)
             int kt = 0;
-            for (; kt + 1 < nk; kt += 2) {
-                wait_vmcnt<0>();
-                tile(kt, min(kt + 2, nk - 1), (kt + 1) % kStages, R1, R0, Z1, Z0);
-                wait_vmcnt<0>();
-                tile(kt + 1, min(kt + 3, nk - 1), kt % kStages, R0, R1, Z0, Z1);
-            }
-            if (kt < nk) {
-                wait_vmcnt<0>();
-                tile(kt, nk - 1, (kt + 1) % kStages, R1, R0, Z1, Z0);
-            }
+            for (; kt + kSets <= nk; kt += kSets)
+                each_of<kSets>([&](auto d) { turn(kt + d(), d); });
+            each_of<kSets - 1>([&](auto d) {
+                if (kt + d() < nk) turn(kt + d(), d);
+            });
         }
     } else {
         // Tile t goes to stage t % kStages.  The prologue issues tiles
@@ -1130,7 +1206,7 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
             frag(lds, lds + kASz, 0, ca, cb);
             for (int kt = 0; kt < nk; ++kt)
                 tile(kt, min(kt + kAhead, nk - 1), (kt + kAhead) % kStages, nullptr, nullptr,
-                     nullptr, nullptr);
+                     nullptr, nullptr, kt);
             wait_vmcnt<0>();  // the reloads past the last tile, before the LDS reuse
         }
     }
@@ -1140,9 +1216,9 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
     // s), as from a last tile zero-filled past K: a group whose k are all
     // past K is skipped, and a lane supplies zeros for its k past K.  A lane
     // takes the four k of a group from a k-contiguous operand with one
-    // 16-byte load (K % 4 == 0 there), from a row-contiguous one with four
-    // loads that are coalesced across the lanes; every address is clamped
-    // into the operand, and all loads go out before the first MFMA.  The
+    // 16-byte load (one element at a time where K % 4 != 0), from a
+    // row-contiguous one with four loads that are coalesced across the lanes;
+    // every address is clamped into the operand, and all loads go out before the first MFMA.  The
     // column sums (TN) take the same k, after the tiles'.
     if constexpr (KT) {
         const int kb = nk * BK;
@@ -1158,13 +1234,14 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
             // column r of a row-contiguous one; zeros past K.
             auto four = [&](const float *base, int ld, bool kc, int r, int k4) {
                 f32x4 v;
-                if (kc) {
-                    v = *reinterpret_cast<const f32x4 *>(base + (size_t)r * ld + min(k4, p.K - 4));
+                if (kc && (p.K & 3) == 0) {
+                    v = *reinterpret_cast<const f32x4_u *>(base + (size_t)r * ld + min(k4, p.K - 4));
                     if (k4 >= p.K) v = f32x4{0.f, 0.f, 0.f, 0.f};
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const float x = base[(size_t)min(k4 + e, p.K - 1) * ld + r];
+                        const int k = min(k4 + e, p.K - 1);
+                        const float x = kc ? base[(size_t)r * ld + k] : base[(size_t)k * ld + r];
                         v[e] = k4 + e < p.K ? x : 0.0f;
                     }
                 }
@@ -1205,7 +1282,7 @@ __device__ __forceinline__ void gemm_f32_pipe_body(GemmArgs p, int bx, int by) {
         if (do_cs) cs.finish(p, lds, n0);
     // The whole tile in bounds: the register epilogue (the choice is uniform
     // across the workgroup, as store_tile has workgroup barriers).
-    if (!(p.vec_out && m0 + BM <= p.M && n0 + BN <= p.N &&
+    if (!(m0 + BM <= p.M && n0 + BN <= p.N &&
           store_direct<TM, TN, IA, IB>(p, acc, m0 + wm0, n0 + wn0, lane)))
         store_tile<TM, TN, WTN, NW, IA, IB>(p, acc, lds, m0 + wm0, n0 + wn0, wave, lane);
 }
@@ -1353,13 +1430,19 @@ void launch_skinny_pre(const GemmArgs &a, const GemmArgs &pre, hipStream_t st,
 // (k_gemm_pair.hip): kinds of the kernels they would take alone.  x1 / x2:
 // output tiles (skinny: its workgroups), n1 / n2: workgroups (tiles x K
 // slices).  tiles_m / tiles_n of each GemmArgs are set by the caller.
-// The first three kinds (256 threads, small LDS) pair with each other; the
-// last two only with their own kind, both bodies then sharing one LDS buffer:
+// The first three kinds (256 threads, small LDS; kPairTail: the 64x64 tiles
+// with a K tail or unaligned rows) pair with each other; the others only with
+// their own kind (the two kPairMid kinds with each other), both bodies then
+// sharing one LDS buffer:
 // kPairBig: the 8-wave pipelined tiles of large layers, dW on 256x256 (cfg
 // 6, TN) with dX on 256x128 (cfg 7, NT), 512 threads;
-// kPairMid: both on the 4-wave 128x64 pipelined tiles (cfg 5), 256 threads.
-enum : int { kPairSkinny = 0, kPairElem = 1, kPairPipe = 2, kPairBig = 3, kPairMid = 4 };
-inline bool pair_exclusive(int kind) { return kind == kPairBig || kind == kPairMid; }
+// kPairMid: both on the 4-wave 128x64 pipelined tiles (cfg 5), 256 threads;
+// kPairMidTail: the same with a K tail or unaligned rows.
+enum : int {
+    kPairSkinny = 0, kPairTail = 1, kPairPipe = 2, kPairBig = 3, kPairMid = 4, kPairMidTail = 5
+};
+inline bool pair_exclusive(int kind) { return kind >= kPairBig; }
+inline bool pair_mid(int kind) { return kind == kPairMid || kind == kPairMidTail; }
 void launch_pair(int k1, int k2, const GemmArgs &a1, const GemmArgs &a2, int x1, int n1, int x2,
                  int n2, hipStream_t st);
 // A skinny TN weight gradient (n1 workgroups) with a pair (kinds k2, k3 as

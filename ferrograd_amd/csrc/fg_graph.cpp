@@ -1650,7 +1650,7 @@ int run_optim(fg_plan &P, fg_mt *mt) {
     if (P.wctx.pending_splits > 0) {
         bool fuse = sgd;
         if (fuse) {
-            fg::ByteRange red[3];
+            fg::ByteRange red[4];
             fg::pending_reduce_ranges(&P.wctx, red);
             for (const fg::ByteRange &o : optim_ranges(P))
                 for (const fg::ByteRange &q : red) fuse = fuse && !q.overlaps(o);

@@ -89,10 +89,10 @@ struct ByteRange {
 
 // The held split-K summing launch (fg_ctx::pending, k_gemm.hip): its block
 // count for M x N outputs, a launch of it alone (clears it), and the memory
-// it writes (C) and reads besides its slices (act' operand, bias).
+// it writes (C, the column sums) and reads besides its slices (act' operand, bias).
 int reduce_blocks(const fg_ctx *ctx, int M, int N);
 int launch_pending_reduce(fg_ctx *ctx);
-void pending_reduce_ranges(const fg_ctx *ctx, ByteRange out[3]);
+void pending_reduce_ranges(const fg_ctx *ctx, ByteRange out[4]);
 // The held mean loss (fg_ctx::mean_*) in a launch of its own; clears it.
 int launch_pending_mean(fg_ctx *ctx);
 // SGD over `mt` with the summing launch and / or the mean loss held in

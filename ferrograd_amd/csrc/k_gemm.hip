@@ -23,47 +23,70 @@ using fg::gemm::kThreads;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------ dispatch
-// Tile configuration per call (indices as in fg_gemm_kernel.h), from a
-// measured sweep of every configuration of the pipelined kernel on MI355X
-// (256 CUs, N(0,1) operands, HIP events) over the BASELINE shapes, TFLOP/s:
-//  * NN (forward): 256x256 with 8 waves for K >= 4096 squares that fill the
-//    chip (138-145 at 4096^3, against 139-142 for the 256x128 tiles); else
-//    256x128 with 8 waves when it yields >= one tile per CU (125 at
-//    2048x4096x4096, 135 at K = 1024); else 128x64 (131 for the 1000-wide
-//    head, against 70 for 128x128 on a quarter of the CUs); 64x64 for
-//    anything smaller.
-//  * NT (dA): 256x256 with 8 waves for large-K squares that fill the chip
-//    (145 at 4096^3); else 256x128 with 8 waves when it gives >= one tile per
-//    CU (137 at 2048x4096x4096); else 128x128 or 128x64 (137 for 128x64 at
-//    2048x1024x4096, against 73 for 128x128).
-//  * TN (dW): 256x256 with 8 waves whenever it fills the chip (143 at 4096^3;
-//    141 at 4096x4096x2048, the c5 hidden dW, against 136.5 for 256x128 with
-//    4 waves, with the interleaved fragments of the TN layout); 256x128 with
-//    4 waves at >= two tiles per CU; then 128x64 at >= two tiles per CU
-//    (131-133 for the 1024- and 1000-wide layers, against 125-127 for
-//    128x128); else 128x128; else 128x64.
-// K % BK != 0 (the 1000-deep head dA) takes the pipelined kernel's staged
-// instances with a zero-filled last K tile (the 256x256 tiles give way to
-// 256x128).
 int tiles(int M, int N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-int pick_cfg(int layout, int M, int N, int K, int cus) {
-    if (layout == FG_NN) {
-        if (K >= 4096 && tiles(M, N, 256, 256) >= cus) return 6;
-        if (tiles(M, N, 256, 128) >= cus) return 7;
-        if (tiles(M, N, 128, 64) >= cus) return 5;
-        return 4;
+// Tile configuration (indices as in fg_gemm_kernel.h) and K slices of a call,
+// by a model of its time.  Every configuration multiplies at nearly the same
+// rate per CU once a CU has a workgroup (measured on MI355X, 256 CUs, N(0,1)
+// operands, HIP events: kRate, us per k per 64x64 of output, from 1024^3 to
+// 4096^3 products in each layout), so what tells them apart is how their
+// tiles fill the CUs: a CU with n workgroups takes n tiles' time.  K slices cut
+// the tiles' depth, for a summing launch and the slots' traffic.  Modelled
+// against measured (us, NN): 1536^3 on 128x64 tiles 102 / 102, 64x64 77 / 77;
+// 777 x 1333 x 2049 on 64x64 tiles 70 / 71, in four slices 56 / 57.  Against the
+// choice by thresholds on the tile counts before: 1536^3 96 -> 76, 777 x
+// 1333 x 2049 74 -> 67, 512 x 1024 x 2048 46 -> 23, 2100 x 4096 x 1000 252 -> 166;
+// TN with column sums (not split before) 500 x 1000 x 3000 67 -> 34.
+// The candidates' order settles ties: the larger tiles first, which read
+// less from the L2s.
+struct Choice {
+    int cfg = 4, splits = 1, ks = 0;
+    float us = 0.0f;
+};
+struct Rate {
+    int cfg;
+    float us;
+};
+constexpr Rate kRates[3][5] = {
+    {{7, 0.0146f}, {6, 0.0145f}, {3, 0.0150f}, {5, 0.0153f}, {4, 0.0159f}},   // NN
+    {{7, 0.0146f}, {6, 0.0145f}, {3, 0.0150f}, {5, 0.0155f}, {4, 0.0159f}},   // NT
+    {{6, 0.0145f}, {1, 0.0152f}, {3, 0.0153f}, {5, 0.0150f}, {4, 0.0157f}}};  // TN
+// The summing launch: its own time, and the rate at which it and the GEMM
+// move the slots.
+constexpr float kSumUs = 2.0f, kSumBytesPerUs = 4.0e6f;
+
+// one_cfg: only that configuration (-1: any).  A K that is not whole tiles
+// (or rows unaligned: !aligned) takes the staged tiles, not 256x256.
+Choice choose(int layout, int M, int N, int K, int cus, bool aligned, bool colsum,
+              uint64_t ws_bytes, int one_cfg = -1) {
+    Choice best;
+    best.us = 1e30f;
+    for (const Rate &r : kRates[layout]) {
+        int bm, bn;
+        fg::gemm::cfg_tile(r.cfg, true, bm, bn);
+        const int bk = fg::gemm::cfg_bk(r.cfg);
+        if (one_cfg >= 0 && r.cfg != one_cfg) continue;
+        if (r.cfg == 6 && (!aligned || K % bk != 0 || (layout != FG_TN && K < 4096))) continue;
+        const int64_t t = tiles(M, N, bm, bn);
+        const float unit = r.us * (bm / 64) * (bn / 64);
+        for (int s = 1; s <= 16; ++s) {
+            int ks = K;
+            if (s > 1) {
+                // At least eight K tiles in all and four a slice, whole ones;
+                // slices only while the CUs have under four tiles each.
+                // (A weight gradient of a narrow head stays one launch.)
+                if ((colsum && N < 64) || K < 8 * bk || s > K / (4 * bk) || t * s > 4 * (int64_t)cus) break;
+                ks = ((K + s - 1) / s + bk - 1) / bk * bk;
+                if ((K + ks - 1) / ks != s) continue;
+                if ((uint64_t)s * ((uint64_t)M * N + (colsum ? N : 0)) * sizeof(float) > ws_bytes)
+                    break;
+            }
+            float us = (float)((t * s + cus - 1) / cus) * ks * unit;
+            if (s > 1) us += kSumUs + (2 * s + 1) * (float)M * N * 4.0f / kSumBytesPerUs;
+            if (us < 0.99f * best.us) best = Choice{r.cfg, s, s > 1 ? ks : 0, us};
+        }
     }
-    if ((K >= 4096 || layout == FG_TN) && tiles(M, N, 256, 256) >= cus) return 6;
-    if (layout == FG_NT) {
-        if (tiles(M, N, 256, 128) >= cus) return 7;
-    } else {
-        if (tiles(M, N, 256, 128) >= 2 * cus) return 1;
-        if (tiles(M, N, 128, 64) >= 2 * cus) return 5;
-    }
-    if (tiles(M, N, 128, 128) >= cus) return 3;
-    if (tiles(M, N, 128, 64) >= cus) return 5;
-    return 4;
+    return best;
 }
 
 // Split-K epilogue: out[m][n] = epilogue(sum over the slots, in order, of
@@ -102,38 +125,6 @@ __global__ __launch_bounds__(kThreads) void mean_rows_kernel(const float *__rest
     fg::smrow::mean_rows(src, R, dst, sh);
 }
 
-// Split K over workgroup rows when the output gives few tiles (under half
-// the CUs) and K is long (at least kSplitMinKTiles K tiles, and at least 4
-// per slice; c1's K = 256 GEMMs, 16 K tiles, run 62 us per step split and
-// 69 us unsplit, though unsplit saves two dispatches): each slice's raw
-// product goes to the context's workspace, which must already hold them
-// (every plan has its own of at least 1 MiB; direct callers reserve one with
-// fg_ctx_reserve_workspace; it is never grown here, so launches stay
-// capturable).  The fused column sum of fg_gemm_dw is not split.
-// Returns the number of slices (1: no split).
-#ifndef FG_SPLIT_MIN_KTILES  // tuning builds may set it
-#define FG_SPLIT_MIN_KTILES 8
-#endif
-constexpr int kSplitMinKTiles = FG_SPLIT_MIN_KTILES;
-
-int plan_split_k(fg_ctx *ctx, GemmArgs &a, int cfg, bool vec) {
-    if (a.colsum || a.K <= 0) return 1;
-    int bm, bn;
-    fg::gemm::cfg_tile(cfg, vec, bm, bn);
-    const int bk = vec ? fg::gemm::cfg_bk(cfg) : 16;
-    if (a.K < kSplitMinKTiles * bk) return 1;
-    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    int s = std::min(cus / (2 * tiles(a.M, a.N, bm, bn)), a.K / (4 * bk));
-    if (s < 2) return 1;
-    int ks = (a.K + s - 1) / s;
-    ks = (ks + bk - 1) / bk * bk;  // whole K tiles per slice
-    s = (a.K + ks - 1) / ks;
-    if (s < 2 || (uint64_t)s * a.M * a.N * sizeof(float) > ctx->ws_bytes) return 1;
-    a.partial = static_cast<float *>(ctx->ws);
-    a.ksplit = ks;
-    return s;
-}
-
 // Skinny shapes (few columns, short K, at most one 16-row workgroup per CU)
 // take the one-round-trip kernel of k_gemm_skinny.hip: c1's second layer
 // (64x10x256) and its weight gradient with the bias gradient (TN 256x10x64).
@@ -157,6 +148,14 @@ bool use_rows(int layout, const GemmArgs &a, int pro) {
            (a.mode == 0 || nk >= 1 << 20);
 }
 
+// A choice's K slices in the arguments.
+void set_choice(const fg_ctx *ctx, GemmArgs &a, const Choice &ch) {
+    a.partial = ch.splits > 1 ? static_cast<float *>(ctx->ws) : nullptr;
+    a.ksplit = ch.ks;
+    a.colsum_partial =
+        ch.splits > 1 && a.colsum ? a.partial + (size_t)ch.splits * a.M * a.N : nullptr;
+}
+
 // The kernel choices of one GEMM call (sets a.vec_out, and a.partial /
 // a.ksplit when K is split): the skinny kernel (skinny; then nothing else
 // applies), 16-byte operand loads (vec), the pipelined kernel (pipe) and
@@ -164,9 +163,10 @@ bool use_rows(int layout, const GemmArgs &a, int pro) {
 // number of K slices.  pro: the prologue code (fg::gemm::kPro*), whose
 // tensor Pz must meet the same 16-byte conditions as the operand it scales.
 void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &rows, bool &vec,
-               bool &pipe, bool &ktail, int &cfg, int &splits, int pro = fg::gemm::kProNone) {
+               bool &pipe, bool &ktail, bool &aligned, int &cfg, int &splits,
+               int pro = fg::gemm::kProNone) {
     skinny = use_skinny(ctx, a, pro);
-    vec = pipe = ktail = rows = false;
+    vec = pipe = ktail = rows = aligned = false;
     cfg = 0;
     splits = 1;
     if (skinny) return;
@@ -180,42 +180,53 @@ void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &rows, b
     if (layout == FG_NT) vec = vec && a.K % 4 == 0;
     if (layout == FG_TN) vec = vec && a.M % 4 == 0 && a.N % 4 == 0;
     if (pro != fg::gemm::kProNone) vec = vec && (((uintptr_t)a.Pz) & 15u) == 0 && a.ldp % 4 == 0;
-#ifdef FG_GEMM_FORCE_CFG  // tuning builds: one tile configuration for every shape
-    cfg = FG_GEMM_FORCE_CFG;
-#else
-    cfg = pick_cfg(layout, a.M, a.N, a.K, ctx->cu_count > 0 ? ctx->cu_count : 256);
-#endif
-    if (pro != fg::gemm::kProNone) cfg = fg::gemm::pro_cfg(cfg);
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     auto al16 = [](const void *q) { return (((uintptr_t)q) & 15u) == 0; };
     a.vec_out = al16(a.C) && a.ldc % 4 == 0 && (!a.Z || (al16(a.Z) && a.ldz % 4 == 0)) &&
                 (!a.bias || al16(a.bias));
-    // The pipelined kernel's 16-byte tile loads need at least one 16-byte
-    // chunk per row-contiguous operand row (edge chunks are clamped, not
-    // masked).  A partial last K tile (K % BK != 0) is zero-filled by the
-    // staged-tile instances (ktail); the prologue instances need whole tiles
-    // and leave such shapes to gemm_f32_mfma.
     rows = use_rows(layout, a, pro);
     if (rows) {
         int ks;
-        splits = fg::rows::split_of(ctx->cu_count > 0 ? ctx->cu_count : 256, 4, a.M, a.N, a.K,
-                                    ctx->ws_bytes, ks);
+        splits = fg::rows::split_of(cus, 4, a.M, a.N, a.K, ctx->ws_bytes, ks);
         if (splits > 1) {
             a.partial = static_cast<float *>(ctx->ws);
             a.ksplit = ks;
         }
         return;
     }
-    pipe = fg::gemm::kPipe && vec && a.K > 0 && a.M >= 4 && a.N >= 4;
+    // The pipelined kernel's 16-byte tile loads need at least one 16-byte
+    // chunk per row-contiguous operand row (edge chunks are clamped, not
+    // masked).  A K that is not whole tiles, and rows that are not 16-byte
+    // aligned, take the staged-tile instances with a K tail (ktail); the
+    // prologue instances need whole aligned tiles and leave other shapes to
+    // gemm_f32_mfma.
+    // K slices go to the context's workspace, which must already hold them
+    // (every plan has its own; direct callers reserve one with
+    // fg_ctx_reserve_workspace; it is never grown here, so launches stay
+    // capturable).
+    const bool chunks = fg::gemm::kPipe && a.K > 0 && a.M >= 4 && a.N >= 4;
+    aligned = vec;
+    if (chunks && pro == fg::gemm::kProNone) vec = true;
+    Choice ch;
+    if (vec) {
+        ch = choose(layout, a.M, a.N, a.K, cus, aligned, a.colsum != nullptr, ctx->ws_bytes);
+    } else {  // the element-load kernel's tile
+        ch = choose(layout, a.M, a.N, a.K, cus, true, a.colsum != nullptr, ctx->ws_bytes, 4);
+    }
+    if (pro != fg::gemm::kProNone) ch.cfg = fg::gemm::pro_cfg(ch.cfg);
+    set_choice(ctx, a, ch);
+    cfg = ch.cfg;
+    splits = ch.splits;
+    const bool whole = aligned && a.K % fg::gemm::cfg_bk(cfg) == 0;
+    pipe = chunks && vec;
     ktail = false;
-    if (pipe && a.K % fg::gemm::cfg_bk(cfg) != 0) {
+    if (pipe && !whole) {
         if (pro != fg::gemm::kProNone) {
             pipe = false;
         } else {
             ktail = true;
-            cfg = fg::gemm::pro_cfg(cfg);  // staged tiles
         }
     }
-    splits = plan_split_k(ctx, a, cfg, vec);
 }
 
 // One GEMM call, validated and planned (gemm_prepare), then launched
@@ -224,6 +235,7 @@ struct Planned {
     GemmArgs a{};
     int layout = FG_NN, pro = fg::gemm::kProNone, cfg = 0, splits = 1;
     bool skinny = false, rows = false, vec = false, pipe = false, ktail = false;
+    bool aligned = false;  // whole 16-byte chunks on 16-byte boundaries
     bool empty = false;  // M == 0 or N == 0: nothing to launch
 };
 
@@ -252,7 +264,7 @@ int gemm_prepare(fg_ctx *ctx, int layout, const GemmArgs &a0, const char *who, i
                a.ldb, a.ldc);
     FG_HIP(hipSetDevice(ctx->device));
     if (a.K == 0) a.A = a.B;  // loads are all masked; K=0 yields the epilogue of zero
-    plan_gemm(ctx, layout, a, P.skinny, P.rows, P.vec, P.pipe, P.ktail, P.cfg, P.splits, pro);
+    plan_gemm(ctx, layout, a, P.skinny, P.rows, P.vec, P.pipe, P.ktail, P.aligned, P.cfg, P.splits, pro);
     return FG_OK;
 }
 
@@ -305,12 +317,11 @@ int gemm_common(fg_ctx *ctx, int layout, GemmArgs &a, const char *who,
 int pair_kind(const Planned &P) {
     if (P.empty || P.rows || P.pro != fg::gemm::kProNone) return -1;
     if (P.skinny) return fg::gemm::kPairSkinny;
-    if (!P.vec) return fg::gemm::kPairElem;
-    if (P.pipe && !P.ktail && P.cfg == 4) return fg::gemm::kPairPipe;
+    if (P.pipe && P.cfg == 4) return P.ktail ? fg::gemm::kPairTail : fg::gemm::kPairPipe;
     if (P.pipe && !P.ktail && P.splits == 1 &&
         ((P.layout == FG_TN && P.cfg == 6) || (P.layout == FG_NT && P.cfg == 7)))
         return fg::gemm::kPairBig;
-    if (P.pipe && !P.ktail && P.cfg == 5) return fg::gemm::kPairMid;
+    if (P.pipe && P.cfg == 5) return P.ktail ? fg::gemm::kPairMidTail : fg::gemm::kPairMid;
     return -1;
 }
 
@@ -324,7 +335,7 @@ void pair_grid(Planned &P, int &x, int &n) {
     if (pair_kind(P) == fg::gemm::kPairBig) {
         bm = 256;
         bn = P.layout == FG_TN ? 256 : 128;
-    } else if (pair_kind(P) == fg::gemm::kPairMid) {
+    } else if (fg::gemm::pair_mid(pair_kind(P))) {
         bm = 128;
     }
     P.a.tiles_m = (P.a.M + bm - 1) / bm;
@@ -383,7 +394,7 @@ int launch_pending_mean(fg_ctx *ctx) {
     return FG_OK;
 }
 
-void pending_reduce_ranges(const fg_ctx *ctx, ByteRange out[3]) {
+void pending_reduce_ranges(const fg_ctx *ctx, ByteRange out[4]) {
     GemmArgs a;
     std::memcpy(&a, ctx->pending, sizeof a);
     const uintptr_t rows = a.M > 0 ? (uintptr_t)(a.M - 1) : 0;
@@ -393,6 +404,8 @@ void pending_reduce_ranges(const fg_ctx *ctx, ByteRange out[3]) {
                  : ByteRange{0, 0};
     out[2] = a.mode == 0 && a.bias ? ByteRange{(uintptr_t)a.bias, (uintptr_t)(a.bias + a.N)}
                                    : ByteRange{0, 0};
+    out[3] = a.colsum ? ByteRange{(uintptr_t)a.colsum, (uintptr_t)(a.colsum + a.N)}
+                      : ByteRange{0, 0};
 }
 
 int gemm_f32_dispatches(fg_ctx *ctx, int layout, int M, int N, int K, const void *A, int lda,
@@ -408,9 +421,9 @@ int gemm_f32_dispatches(fg_ctx *ctx, int layout, int M, int N, int K, const void
     a.ldb = ldb;
     a.colsum = colsum ? reinterpret_cast<float *>(1) : nullptr;  // only tested for null
     if (K == 0) a.A = a.B;
-    bool skinny, rows, vec, pipe, ktail;
+    bool skinny, rows, vec, pipe, ktail, aligned;
     int cfg, splits;
-    plan_gemm(ctx, layout, a, skinny, rows, vec, pipe, ktail, cfg, splits);
+    plan_gemm(ctx, layout, a, skinny, rows, vec, pipe, ktail, aligned, cfg, splits);
     return splits > 1 ? 2 : 1;
 }
 }  // namespace fg
@@ -560,7 +573,56 @@ GemmArgs dx_args(int M, int N, int K, const float *A, int lda, const float *B, i
 bool pairable(const Planned &P1, const Planned &P2) {
     const int k1 = pair_kind(P1), k2 = pair_kind(P2);
     if (k1 < 0 || k2 < 0 || (P1.splits > 1 && P2.splits > 1)) return false;
+    if (fg::gemm::pair_mid(k1) && fg::gemm::pair_mid(k2)) return true;
     return fg::gemm::pair_exclusive(k1) || fg::gemm::pair_exclusive(k2) ? k1 == k2 : true;
+}
+
+// Two unsplit pipelined GEMMs of different kinds (dW and dX of a layer) on the
+// 64x64 or the 128x64 tiles both, where one launch of all their tiles is
+// shorter than the two they would take alone: the tiles of the second fill the
+// CUs that the last of the first leave (and their bits are those of any tile:
+// each output sums its K in the same order).
+void join(const fg_ctx *ctx, Planned &P1, Planned &P2) {
+    auto plain = [](const Planned &P) {
+        return !P.empty && !P.skinny && !P.rows && P.pipe && P.splits == 1 &&
+               P.pro == fg::gemm::kProNone;
+    };
+    if (pairable(P1, P2) || !plain(P1) || !plain(P2)) return;
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    // (Each with work for every CU: a narrow head's two stay apart.)
+    if (tiles(P1.a.M, P1.a.N, 64, 64) < cus || tiles(P2.a.M, P2.a.N, 64, 64) < cus) return;
+    auto cost = [&](const Planned &P, int cfg, float &granule) {
+        int bm, bn;
+        fg::gemm::cfg_tile(cfg, true, bm, bn);
+        float r = 0.0f;
+        for (const Rate &q : kRates[P.layout])
+            if (q.cfg == cfg) r = q.us;
+        granule = r * (bm / 64) * (bn / 64) * P.a.K;
+        return granule * tiles(P.a.M, P.a.N, bm, bn) / cus;
+    };
+    auto alone = [&](const Planned &P) {
+        float g;
+        const float t = cost(P, P.cfg, g);
+        return std::ceil(t / g) * g;
+    };
+    const float apart = alone(P1) + alone(P2) + kSumUs;
+    int best = -1;
+    float us = apart;
+    for (int cfg : {5, 4}) {
+        float g1, g2;
+        // (On average half of the larger tile's time is left at the end.)
+        const float t = cost(P1, cfg, g1) + cost(P2, cfg, g2);
+        const float j = std::max(t + 0.5f * std::max(g1, g2), std::max(g1, g2));
+        if (j < us) {
+            us = j;
+            best = cfg;
+        }
+    }
+    if (best < 0) return;
+    for (Planned *P : {&P1, &P2}) {
+        P->cfg = best;
+        P->ktail = !P->aligned || P->a.K % fg::gemm::cfg_bk(best) != 0;
+    }
 }
 
 // Both validated and planned, and pairable.
@@ -568,6 +630,7 @@ bool plan_pair(fg_ctx *ctx, const GemmArgs &w, const GemmArgs &x, Planned &P1, P
     if (gemm_prepare(ctx, FG_TN, w, "fg_gemm_dw_f32", fg::gemm::kProNone, P1) ||
         gemm_prepare(ctx, FG_NT, x, "fg_gemm_bwd_f32", fg::gemm::kProNone, P2))
         return false;
+    join(ctx, P1, P2);
     return pairable(P1, P2);
 }
 
@@ -615,7 +678,7 @@ void plan_quiet(fg_ctx *ctx, int layout, const GemmArgs &a0, Planned &P) {
     const float *aligned = reinterpret_cast<const float *>(256);
     if (!P.a.A) P.a.A = aligned;
     if (!P.a.B) P.a.B = aligned;
-    plan_gemm(ctx, layout, P.a, P.skinny, P.rows, P.vec, P.pipe, P.ktail, P.cfg, P.splits);
+    plan_gemm(ctx, layout, P.a, P.skinny, P.rows, P.vec, P.pipe, P.ktail, P.aligned, P.cfg, P.splits);
 }
 }  // namespace
 
@@ -788,6 +851,7 @@ int gemm_dw_dw_dx_dispatches(fg_ctx *ctx, int M0, int N0, int K0, const void *A0
                                    c, N1, 0, c, 0), P1);
     plan_quiet(ctx, FG_NT, dx_args(M2, N2, K2, (const float *)A2, lda2, (const float *)B2, ldb2,
                                    FG_ACT_NONE, nullptr, 0, c, N2, 0), P2);
+    join(ctx, P1, P2);
     if (pair_kind(P0) != fg::gemm::kPairSkinny || !pairable(P1, P2) ||
         fg::gemm::pair_exclusive(pair_kind(P1)))
         return sep;
@@ -809,6 +873,7 @@ int gemm_dw_dx_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A1, i
                                    c, N1, 0, c, 0), P1);
     plan_quiet(ctx, FG_NT, dx_args(M2, N2, K2, (const float *)A2, lda2, (const float *)B2, ldb2,
                                    FG_ACT_NONE, nullptr, 0, c, N2, 0), P2);
+    join(ctx, P1, P2);
     if (!pairable(P1, P2)) return sep;
     return 1 + (P1.splits > 1) + (P2.splits > 1);
 }

@@ -6,7 +6,7 @@
 // first n1 workgroups run the dW body and the rest the dX body, each exactly
 // as its own kernel would (same tile walk, same K slices, same bits).  The
 // small 256-thread kernels pair with each other (the skinny kernel and the
-// 64x64 tiles, element loads or pipelined); the pipelined 128x64 tiles and
+// 64x64 tiles); the pipelined 128x64 tiles and
 // the large layers' 8-wave tiles each pair with their own kind.
 #include "fg_gemm_skinny.h"
 
@@ -21,9 +21,9 @@ struct PkSkinny {
     }
 };
 template <bool AK, bool BNC>
-struct PkElem {  // 64x64, element loads (gemm_f32_mfma, VEC false)
+struct PkTail {  // 64x64, pipelined, K tail and unaligned rows
     __device__ static void run(const GemmArgs &p, int bx, int by) {
-        gemm_f32_mfma_body<64, 64, 16, 2, 2, AK, BNC, false, kProNone>(p, bx, by);
+        gemm_f32_pipe_body<64, 64, 16, 2, 2, AK, BNC, kProNone, true>(p, bx, by);
     }
 };
 template <bool AK, bool BNC>
@@ -55,8 +55,8 @@ void launch_with(int k2, const GemmArgs &a1, const GemmArgs &a2, int x1, int n1,
         case kPairSkinny:
             gemm_pair<G1, PkSkinny<true, false>><<<grid, block, 0, st>>>(a1, a2, x1, n1, x2);
             break;
-        case kPairElem:
-            gemm_pair<G1, PkElem<true, false>><<<grid, block, 0, st>>>(a1, a2, x1, n1, x2);
+        case kPairTail:
+            gemm_pair<G1, PkTail<true, false>><<<grid, block, 0, st>>>(a1, a2, x1, n1, x2);
             break;
         default:
             gemm_pair<G1, PkPipe<true, false>><<<grid, block, 0, st>>>(a1, a2, x1, n1, x2);
@@ -89,8 +89,8 @@ void triple_with(int k3, const GemmArgs &a1, const GemmArgs &a2, const GemmArgs 
         case kPairSkinny:
             gemm_triple<G2, PkSkinny<true, false>><<<grid, block, 0, st>>>(a1, a2, a3, n1, x2, n2, x3);
             break;
-        case kPairElem:
-            gemm_triple<G2, PkElem<true, false>><<<grid, block, 0, st>>>(a1, a2, a3, n1, x2, n2, x3);
+        case kPairTail:
+            gemm_triple<G2, PkTail<true, false>><<<grid, block, 0, st>>>(a1, a2, a3, n1, x2, n2, x3);
             break;
         default:
             gemm_triple<G2, PkPipe<true, false>><<<grid, block, 0, st>>>(a1, a2, a3, n1, x2, n2, x3);
@@ -133,15 +133,16 @@ __global__ __launch_bounds__(512) void gemm_pair_big(GemmArgs a1, GemmArgs a2, i
 // LDS buffer, the same size for both).  Alone, a 128x64 data gradient of
 // 256 tiles runs one wave per SIMD; beside the weight gradient's tiles the
 // CUs hold three workgroups and the waves hide each other's waits.
+template <bool KT>
 __global__ __launch_bounds__(256) void gemm_pair_mid(GemmArgs a1, GemmArgs a2, int x1, int n1,
                                                      int x2) {
     if (FG_PAIR_PRIO > 0) __builtin_amdgcn_s_setprio(FG_PAIR_PRIO);
     const int w = blockIdx.x;
     if (w < n1) {
-        gemm_f32_pipe_body<128, 64, 32, 2, 2, false, true, kProNone, false>(a1, w % x1, w / x1);
+        gemm_f32_pipe_body<128, 64, 32, 2, 2, false, true, kProNone, KT>(a1, w % x1, w / x1);
     } else {
         const int v = w - n1;
-        gemm_f32_pipe_body<128, 64, 32, 2, 2, true, false, kProNone, false>(a2, v % x2, v / x2);
+        gemm_f32_pipe_body<128, 64, 32, 2, 2, true, false, kProNone, KT>(a2, v % x2, v / x2);
     }
 }
 
@@ -153,8 +154,8 @@ void launch_triple(const GemmArgs &a1, int n1, int k2, const GemmArgs &a2, int x
         case kPairSkinny:
             triple_with<PkSkinny<false, true>>(k3, a1, a2, a3, n1, x2, n2, x3, n3, st);
             break;
-        case kPairElem:
-            triple_with<PkElem<false, true>>(k3, a1, a2, a3, n1, x2, n2, x3, n3, st);
+        case kPairTail:
+            triple_with<PkTail<false, true>>(k3, a1, a2, a3, n1, x2, n2, x3, n3, st);
             break;
         default: triple_with<PkPipe<false, true>>(k3, a1, a2, a3, n1, x2, n2, x3, n3, st); break;
     }
@@ -166,13 +167,16 @@ void launch_pair(int k1, int k2, const GemmArgs &a1, const GemmArgs &a2, int x1,
         gemm_pair_big<<<dim3(n1 + n2), dim3(512), 0, st>>>(a1, a2, x1, n1, x2);
         return;
     }
-    if (k1 == kPairMid) {  // likewise
-        gemm_pair_mid<<<dim3(n1 + n2), dim3(256), 0, st>>>(a1, a2, x1, n1, x2);
+    if (pair_mid(k1)) {  // likewise; the tail's body runs whole tiles as the other does
+        if (k1 == kPairMid && k2 == kPairMid)
+            gemm_pair_mid<false><<<dim3(n1 + n2), dim3(256), 0, st>>>(a1, a2, x1, n1, x2);
+        else
+            gemm_pair_mid<true><<<dim3(n1 + n2), dim3(256), 0, st>>>(a1, a2, x1, n1, x2);
         return;
     }
     switch (k1) {  // GEMM 1 is the TN weight gradient
         case kPairSkinny: launch_with<PkSkinny<false, true>>(k2, a1, a2, x1, n1, x2, n2, st); break;
-        case kPairElem: launch_with<PkElem<false, true>>(k2, a1, a2, x1, n1, x2, n2, st); break;
+        case kPairTail: launch_with<PkTail<false, true>>(k2, a1, a2, x1, n1, x2, n2, st); break;
         default: launch_with<PkPipe<false, true>>(k2, a1, a2, x1, n1, x2, n2, st); break;
     }
 }

@@ -711,6 +711,59 @@ def test_gemm_few_rows(gpu_ctx, dtype, layout, place):
         assert torch.equal(got(C, ldc), torch.where(zs > 0, v, torch.zeros_like(v)))
 
 
+# fp32 tiles on rows of any alignment: every K remainder of the tile pipeline
+# (1 to 9 tiles of 16 and a tail), rows that end between 16-byte chunks (whose
+# last one the K tail takes), edges of 64- and 128-wide tiles, K slices with
+# column sums.
+@pytest.mark.parametrize("place", ["plain", "padded", "offset"])
+@pytest.mark.parametrize("layout", [O.NN, O.NT, O.TN], ids=["NN", "NT", "TN"])
+def test_gemm_f32_any_rows(gpu_ctx, layout, place):
+    """Small-integer operands (every sum exact in fp32, whatever its order),
+    with NaN around every row (padded) and before and after the tensors:
+    outputs and column sums bit for bit."""
+    torch = _torch()
+    gpu_ctx.reserve_workspace(64 << 20)
+    g = torch.Generator().manual_seed(11)
+
+    def ints(r, c):
+        ld = c + (3 if place == "padded" else 0)
+        off = 1 if place == "offset" else 64
+        v = torch.randint(-3, 4, (r, c), generator=g).float()
+        buf = torch.full((off + r * ld + 64,), float("nan"))
+        buf[off:off + r * ld].view(r, ld)[:, :c] = v
+        buf = buf.cuda()
+        return v.double(), buf[off:], ld
+
+    shapes = [(65, 67, 16 * t + x) for t in range(1, 10) for x in (0, 5)]
+    shapes += [(4, 4, 1), (5, 7, 15), (63, 4, 33), (129, 130, 64), (128, 66, 256),
+               (100, 201, 3000), (500, 1000, 1500), (1000, 1501, 400)]
+    for M, N, K in shapes:
+        if layout != O.TN and M <= 32:
+            continue  # (few rows: another kernel)
+        note(f"gemm_f32_any_rows {layout} {place} {M}x{N}x{K}")
+        a, A, lda = ints(*((K, M) if layout == O.TN else (M, K)))
+        b, B, ldb = ints(*((N, K) if layout == O.NT else (K, N)))
+        old, C, ldc = ints(M, N)
+        ref = (a.T if layout == O.TN else a) @ (b.T if layout == O.NT else b)
+
+        def got():
+            torch.cuda.synchronize()
+            return C[:M * ldc].view(M, ldc)[:, :N].cpu().double()
+
+        gpu_ctx.gemm(layout, M, N, K, A, lda, B, ldb, C, ldc, accumulate=True)
+        assert torch.equal(got(), ref + old)
+        if layout == O.TN:
+            cs, S, _ = ints(1, N)
+            gpu_ctx.gemm_dw(M, N, K, A, lda, B, ldb, C, ldc, colsum=S, colsum_accumulate=True)
+            assert torch.equal(got(), ref)
+            assert torch.equal(S[:N].cpu().double(), (cs + b.sum(0)).reshape(-1))
+        else:
+            zs, Zs, ldzs = ints(M, N)
+            gpu_ctx.gemm_bwd(layout, M, N, K, A, lda, B, ldb, C, ldc, act=O.ACT_RELU, Zs=Zs,
+                             ldzs=ldzs)
+            assert torch.equal(got(), torch.where(zs > 0, ref, torch.zeros_like(ref)))
+
+
 # --------------------------------------------------------- softmax + CE
 def check_softmax_ce(ctx, x, labels, scale=1.0):
     torch = _torch()
