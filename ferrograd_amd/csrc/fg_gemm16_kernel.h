@@ -42,6 +42,34 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// Vectors anywhere in 16-bit (fp32) tensors: the hardware takes unaligned
+// accesses.
+typedef u32x2 u32x2_u __attribute__((aligned(2)));
+typedef u32x4 u32x4_u4 __attribute__((aligned(4)));
+typedef f32x4 f32x4_u __attribute__((aligned(4)));
+
+// Eight 16-bit elements from p on, in one 16-byte load and, where the first
+// word also holds the element before p, a word more: a 16-byte load off a 4-byte
+// boundary takes two to three times as long.  raw: the words as loaded; the
+// elements once landed, by shift().
+struct Raw8 {
+    u32x4 v;
+    uint32_t v4;
+    __device__ __forceinline__ void load(const uint16_t *p) {
+        const uint32_t odd = (uint32_t)((uintptr_t)p >> 1) & 1u;
+        const uint32_t *w = reinterpret_cast<const uint32_t *>(p - odd);
+        v = *reinterpret_cast<const u32x4_u4 *>(w);
+        v4 = w[odd ? 4 : 3];
+    }
+    // odd: p's parity in elements.
+    __device__ __forceinline__ u32x4 shift(uint32_t odd) const {
+        u32x4 r;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            r[q] = __builtin_amdgcn_alignbit(q < 3 ? v[q + 1] : v4, v[q], 16 * odd);
+        return r;
+    }
+};
 
 struct Args {
     const uint16_t *A;
@@ -56,7 +84,6 @@ struct Args {
     int mode;  // 0 forward epilogue, 1 backward (act-derivative) epilogue
     int accumulate;
     int tiles_m, tiles_n;
-    int vec_out;  // C / Z / Zs rows and bias 8-byte aligned: 4-element epilogue I/O
     // TN on the pipelined path only: colsum[n] (=|+=) sum_k B[k][n] --
     // the bias gradient of the layer whose weight gradient this GEMM
     // computes -- summed in fp32 from the B tiles already in LDS by the
@@ -240,12 +267,12 @@ __device__ __forceinline__ void epi16_x4(const Args &p, f32x4 v, f32x4 bv, int r
         return x;
     };
     auto ld4 = [](const uint16_t *q) {
-        const u32x2 w = *reinterpret_cast<const u32x2 *>(q);
+        const u32x2 w = *reinterpret_cast<const u32x2_u *>(q);
         return f32x4{E::to_f((uint16_t)w[0]), E::to_f((uint16_t)(w[0] >> 16)),
                      E::to_f((uint16_t)w[1]), E::to_f((uint16_t)(w[1] >> 16))};
     };
     auto st4 = [](uint16_t *q, f32x4 x) {
-        *reinterpret_cast<u32x2 *>(q) = u32x2{pack2(E::from_f(x[0]), E::from_f(x[1])),
+        *reinterpret_cast<u32x2_u *>(q) = u32x2{pack2(E::from_f(x[0]), E::from_f(x[1])),
                                               pack2(E::from_f(x[2]), E::from_f(x[3]))};
     };
     v = rnd(v);
@@ -278,8 +305,8 @@ __device__ __forceinline__ void epi16_x4(const Args &p, f32x4 v, f32x4 bv, int r
 // its slot.  The slot's rows are N floats from a 256-byte aligned base.
 __device__ __forceinline__ void store_slice16(const Args &p, f32x4 v, int row, int col) {
     float *q = p.partial + (size_t)row * p.N + col;
-    if (p.N % 4 == 0) {
-        *reinterpret_cast<f32x4 *>(q) = v;
+    if (col + 4 <= p.N) {
+        *reinterpret_cast<f32x4_u *>(q) = v;
     } else {
 #pragma unroll 1
         for (int t = 0; t < 4 && col + t < p.N; ++t) q[t] = v[t];
@@ -308,10 +335,10 @@ __device__ __forceinline__ void store_tile16(const Args &p, const f32x16 (&acc)[
     static_assert(64 % G4 == 0 && 32 % RPP == 0, "epilogue lane mapping");
     const int c4 = (lane % G4) * 4, rr0 = lane / G4;
     const int col = c0 + c4;
-    const bool vec = p.vec_out && col + 4 <= p.N;
+    const bool vec = col + 4 <= p.N;
     f32x4 bv = {0.f, 0.f, 0.f, 0.f};
     if (p.mode == 0 && p.bias && vec) {
-        const u32x2 w = *reinterpret_cast<const u32x2 *>(p.bias + col);
+        const u32x2 w = *reinterpret_cast<const u32x2_u *>(p.bias + col);
         bv = f32x4{E::to_f((uint16_t)w[0]), E::to_f((uint16_t)(w[0] >> 16)),
                    E::to_f((uint16_t)w[1]), E::to_f((uint16_t)(w[1] >> 16))};
     }
@@ -354,7 +381,7 @@ __device__ __forceinline__ void store_tile16(const Args &p, const f32x16 (&acc)[
 
 // ------------------------------------------------ register epilogue
 // The pipelined kernels' epilogue when the workgroup's whole tile is in
-// bounds (and rows are 8-byte aligned): no LDS and no workgroup barrier.
+// bounds: no LDS and no workgroup barrier.
 // Accumulator registers 4k .. 4k+3 of lane (h, l32) hold rows 8k + 4h + 0..3
 // of column l32 of a 32x32 block; within each quad of lanes (l32 = 4a + e)
 // a 4x4 transpose by two DPP exchanges leaves lane e with row 8k + 4h + e,
@@ -448,8 +475,8 @@ __device__ __forceinline__ void store_direct16_k(const Args &p, const f32x16 (&a
         const int colh = col0 + 32 * h;  // the block this lane stores
         f32x4 bv0 = {0.f, 0.f, 0.f, 0.f}, bv1 = bv0;
         if constexpr (MODE == 0 && BIAS) {
-            bv0 = unpack4(BF, *reinterpret_cast<const u32x2 *>(p.bias + col0));
-            bv1 = unpack4(BF, *reinterpret_cast<const u32x2 *>(p.bias + col1));
+            bv0 = unpack4(BF, *reinterpret_cast<const u32x2_u *>(p.bias + col0));
+            bv1 = unpack4(BF, *reinterpret_cast<const u32x2_u *>(p.bias + col1));
         }
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
@@ -461,8 +488,8 @@ __device__ __forceinline__ void store_direct16_k(const Args &p, const f32x16 (&a
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const uint16_t *zq = p.Zs + (size_t)(rowb + 8 * k) * p.ldzs;
-                    zr0[k] = *reinterpret_cast<const u32x2 *>(zq + col0);
-                    zr1[k] = *reinterpret_cast<const u32x2 *>(zq + col1);
+                    zr0[k] = *reinterpret_cast<const u32x2_u *>(zq + col0);
+                    zr1[k] = *reinterpret_cast<const u32x2_u *>(zq + col1);
                 }
             }
 #pragma unroll 1
@@ -472,8 +499,8 @@ __device__ __forceinline__ void store_direct16_k(const Args &p, const f32x16 (&a
                 const int row = rowb + 8 * k;                     // this lane's row now
                 const int rowA = r0 + 32 * i + 8 * k + e, rowB = rowA + 4;
                 if constexpr (MODE == 2) {
-                    *reinterpret_cast<f32x4 *>(p.partial + (size_t)row * p.N + col0) = y0;
-                    *reinterpret_cast<f32x4 *>(p.partial + (size_t)row * p.N + col1) = y1;
+                    *reinterpret_cast<f32x4_u *>(p.partial + (size_t)row * p.N + col0) = y0;
+                    *reinterpret_cast<f32x4_u *>(p.partial + (size_t)row * p.N + col1) = y1;
                 } else {
                     f32x4 z0 = {0.f, 0.f, 0.f, 0.f}, z1 = z0, o0 = z0, o1 = z0;
                     if constexpr (kZs) {
@@ -482,8 +509,8 @@ __device__ __forceinline__ void store_direct16_k(const Args &p, const f32x16 (&a
                     }
                     if (p.accumulate) {
                         const uint16_t *cq = p.C + (size_t)row * p.ldc;
-                        o0 = unpack4(BF, *reinterpret_cast<const u32x2 *>(cq + col0));
-                        o1 = unpack4(BF, *reinterpret_cast<const u32x2 *>(cq + col1));
+                        o0 = unpack4(BF, *reinterpret_cast<const u32x2_u *>(cq + col0));
+                        o1 = unpack4(BF, *reinterpret_cast<const u32x2_u *>(cq + col1));
                     }
                     u32x2 zp0, zp1;
                     const u32x2 c0v = epi16_x4_k<BF, MODE, BIAS, ACT>(p, y0, bv0, z0, o0, &zp0);
@@ -492,8 +519,8 @@ __device__ __forceinline__ void store_direct16_k(const Args &p, const f32x16 (&a
                         const u32x2 send = h ? w0 : w1;
                         const u32x2 recv = {(uint32_t)__shfl_xor((int)send[0], 32),
                                             (uint32_t)__shfl_xor((int)send[1], 32)};
-                        *reinterpret_cast<u32x2 *>(base + (size_t)rowA * ld + colh) = h ? recv : w0;
-                        *reinterpret_cast<u32x2 *>(base + (size_t)rowB * ld + colh) = h ? w1 : recv;
+                        *reinterpret_cast<u32x2_u *>(base + (size_t)rowA * ld + colh) = h ? recv : w0;
+                        *reinterpret_cast<u32x2_u *>(base + (size_t)rowB * ld + colh) = h ? w1 : recv;
                     };
                     if (MODE == 0 && p.Z) xch(zp0, zp1, p.Z, p.ldz);
                     xch(c0v, c1v, p.C, p.ldc);
@@ -750,6 +777,13 @@ struct Pipe16Lds {
     static constexpr int elems = kBytes / 2;
 };
 
+// Register sets of a staged tile, i.e. tiles in flight.  A 128x128 tile of
+// BK 32 is an eighth of a microsecond of MFMAs, a load several times that: four
+// sets, with which one workgroup of these tiles a CU beat the larger direct
+// ones split over K (bf16 1024^3 NN / NT 19.5 / 18.8 -> 15.4 / 13.2 us, 2048^3
+// 35.8 / 32.6 -> 28.7 / 25.4).  The 256x256 tiles' registers hold two.
+constexpr int staged_sets16(int BM, int BN) { return BM * BN <= 128 * 128 ? 4 : 2; }
+
 // The kernel's LDS buffer of N 16-bit elements: one static array per N, so
 // bodies that ask for the same N in one launch share it.
 template <int N>
@@ -764,8 +798,10 @@ __device__ __forceinline__ uint16_t (&lds16_buffer())[N] {
 // KT: K need not be a multiple of BK (K % 8 == 0 where an operand is
 // k-contiguous): the tile loop runs the whole tiles, and the k past them go
 // into the accumulators from global memory at the end (the K tail below).
+// Staged tiles only: rows that are not whole aligned chunks too; ODD: rows may
+// start on odd elements.
 template <int BM, int BN, int BK, int WGM, int WGN, bool AK, bool BNC, bool BF, int LDSN = 0,
-          bool KT = false>
+          bool KT = false, bool ODD = false>
 __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
     using E = T16<BF>;
     constexpr int NW = WGM * WGN;
@@ -783,7 +819,12 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
     constexpr int kStages = PL::kStages;
     static_assert(LDSN == 0 || LDSN >= PL::elems, "LDS buffer too small");
     uint16_t(&lds)[LDSN ? LDSN : PL::elems] = lds16_buffer<LDSN ? LDSN : PL::elems>();
+    constexpr bool kAny = KT && kStaged;  // rows of any alignment
+    constexpr int kSets = staged_sets16(BM, BN);
+    static_assert(!ODD || kAny, "odd rows: staged tiles");
 
+    // This workgroup's K ends where the operands do.
+    const bool last = p.ksplit <= 0 || (by + 1) * p.ksplit >= p.K;
     if (p.ksplit > 0) {  // K slice by: offset operands, its own slot
         const int kb = by * p.ksplit;
         p.A += AK ? (size_t)kb : (size_t)kb * p.lda;
@@ -818,7 +859,9 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
     auto src_rc = [&](const uint16_t *base, int ld, int r0, int rmax, int k0, int pos, int R) {
         const int k = pos / (R / 8), pc = pos % (R / 8);
         const int c = pc ^ swz16_r(k);
-        return base + (size_t)(k0 + k) * ld + min(r0 + 8 * c, rmax - 8);
+        // (Rows of any length: a row's last chunk may end past it, in the next
+        // row.)
+        return base + (size_t)(k0 + k) * ld + min(r0 + 8 * c, kAny ? (rmax - 1) & ~7 : rmax - 8);
     };
     // Wave load q (0 .. kLoads-1) of tile kt into stage `stage`: this wave's
     // share of A first, then of B.
@@ -844,7 +887,7 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
     // Staged: wave load q of tile kt into registers, and from there to its
     // place in a stage (lane l's 16 bytes at element 8 l of the wave load's
     // 1 KiB run, as the direct loads would put them).
-    auto load_reg = [&](int kt, int q) {
+    auto src_of = [&](int kt, int q) {
         const int k0 = kt * BK;
         const uint16_t *src;
         if (q < kPerA) {
@@ -854,16 +897,37 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
             const int pos = (wave * kPerB + (q - kPerA)) * 64 + lane;
             src = BNC ? src_rc(p.B, p.ldb, n0, p.N, k0, pos, BN) : src_kc(p.B, p.ldb, n0, p.N, k0, pos);
         }
-        return *reinterpret_cast<const u32x4 *>(src);
+        return src;
     };
-    auto store_reg = [&](int stage, int q, const u32x4 &v) {
+    using Reg = typename std::conditional<ODD, Raw8, u32x4>::type;
+    auto load_reg = [&](int kt, int q) {
+        Reg r;
+        if constexpr (ODD) r.load(src_of(kt, q));
+        else if constexpr (kAny) r = *reinterpret_cast<const u32x4_u4 *>(src_of(kt, q));
+        else r = *reinterpret_cast<const u32x4 *>(src_of(kt, q));
+        return r;
+    };
+    // ODD: a chunk's parity is the same in every tile (BK is even).
+    uint32_t odd = 0;
+    if constexpr (ODD)
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q)
+            odd |= ((uint32_t)((uintptr_t)src_of(0, q) >> 1) & 1u) << q;
+    auto store_reg = [&](int stage, int q, const Reg &v) {
         uint16_t *sa = lds + stage * kStageSz;
         uint16_t *run = q < kPerA ? sa + (wave * kPerA + q) * 512
                                   : sa + kASz + (wave * kPerB + q - kPerA) * 512;
-        *reinterpret_cast<u32x4 *>(run + 8 * lane) = v;
+        if constexpr (ODD)
+            *reinterpret_cast<u32x4 *>(run + 8 * lane) = v.shift((odd >> q) & 1u);
+        else
+            *reinterpret_cast<u32x4 *>(run + 8 * lane) = v;
     };
 
-    const int nk = p.K / BK;
+    // A row-contiguous operand whose rows are not whole chunks leaves its last
+    // row to the K tail: a chunk past the end of that row would be past the
+    // operand's end.
+    const bool ragged = kAny && last && ((!AK && (p.M & 7)) || (BNC && (p.N & 7)));
+    const int nk = (p.K - (ragged ? 1 : 0)) / BK;
     constexpr bool kTN = !AK && BNC;
     ColSum16<BN, BK, 64 * NW, BF> cs;
     const bool do_cs = kTN && p.colsum && tile_m == 0;
@@ -919,7 +983,7 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
     // queues and hold up the MFMAs behind them.
     auto run_step = [&](const u32x4 (&ca)[TM], const u32x4 (&cb)[TN], const uint16_t *An,
                         const uint16_t *Bn, int un, u32x4 (&na)[TM], u32x4 (&nb)[TN], int u,
-                        bool ld, int kl, int slot, const u32x4 *Rw, u32x4 *Rl) {
+                        bool ld, int kl, int slot, const Reg *Rw, Reg *Rl) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int m = 0; m < (kMfma > kPieces ? kMfma : kPieces); ++m) {
@@ -954,8 +1018,9 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
     // out among the MFMAs of step u; ca / cb hold the operands of the next
     // step to multiply.
     u32x4 ca[TM], cb[TN];
-    auto tile = [&](int kt, int kl, int slot, const u32x4 *Rw, u32x4 *Rl) {
-        const uint16_t *As = lds + (kt % kStages) * kStageSz;
+    // st: kt, or a number equal to it modulo kStages.
+    auto tile = [&](int kt, int kl, int slot, const Reg *Rw, Reg *Rl, int st) {
+        const uint16_t *As = lds + (st % kStages) * kStageSz;
         const uint16_t *Bs = As + kASz;
 #pragma unroll
         for (int u = 0; u < NU - 1; ++u) {
@@ -984,7 +1049,7 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
         // Step 0 of tile kt+1 (past the last tile: a stage nothing uses,
         // read and discarded).
         u32x4 na[TM], nb[TN];
-        const uint16_t *An = lds + ((kt + 1) % kStages) * kStageSz;
+        const uint16_t *An = lds + ((st + 1) % kStages) * kStageSz;
         run_step(ca, cb, An, An + kASz, 0, na, nb, 0, false, 0, 0, Rw, Rl);
 #pragma unroll
         for (int i = 0; i < TM; ++i) ca[i] = na[i];
@@ -992,37 +1057,39 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
         for (int j = 0; j < TN; ++j) cb[j] = nb[j];
     };
     if constexpr (kStaged) {
-        // Tile t is loaded into register set t % 2 during tile t-2 and
+        // Tile t is loaded into register set t % kSets during tile t-kSets and
         // written from there to stage t % 2 during tile t-1 (the stage of
-        // tile t-2, free since the barrier that ended tile t-2); each write
-        // goes out right before the load that refills its registers.  Past
-        // the last tile, tile nk-1 is reloaded and written to the free
-        // stage, which nothing reads.  The kt loop is unrolled by two so
-        // that the register sets swap roles without copies.
+        // tile t-2, free since the barrier that ended tile t-2); the set of
+        // tile t is free from then on and refilled during tile t.  Past the
+        // last tile, tile nk-1 is reloaded and written to the free stage,
+        // which nothing reads.  The kt loop is unrolled by kSets so that the
+        // register sets swap roles without copies.
+        static_assert(kSets % 2 == 0, "stage parity");
         if (nk > 0) {
-            u32x4 R0[kLoads], R1[kLoads];
+            Reg R[kSets][kLoads];
 #pragma unroll
-            for (int q = 0; q < kLoads; ++q) R0[q] = load_reg(0, q);
+            for (int d = 0; d < kSets; ++d)
 #pragma unroll
-            for (int q = 0; q < kLoads; ++q) R1[q] = load_reg(min(1, nk - 1), q);
+                for (int q = 0; q < kLoads; ++q) R[d][q] = load_reg(min(d, nk - 1), q);
 #pragma unroll
-            for (int q = 0; q < kLoads; ++q) store_reg(0, q, R0[q]);
+            for (int q = 0; q < kLoads; ++q) store_reg(0, q, R[0][q]);
             wait_lgkm0();
             asm volatile("s_barrier" ::: "memory");
             frag(lds, lds + kASz, 0, ca, cb);
-            // Tile kt writes the set holding tile kt+1 and refills the other
-            // with tile kt+2; that set was loaded a whole tile ago.
+            // Tile kt (set d) writes the set holding tile kt+1, which was
+            // loaded kSets-1 tiles ago: all but the newest kSets-2 sets have
+            // landed.
+            auto turn = [&](int kt, auto dc) {
+                constexpr int d = decltype(dc)::value, w = (d + 1) % kSets;
+                wait_vmcnt<(kSets - 2) * kLoads * (ODD ? 2 : 1)>();
+                tile(kt, min(kt + kSets, nk - 1), (d + 1) % kStages, R[w], R[d], d);
+            };
             int kt = 0;
-            for (; kt + 1 < nk; kt += 2) {
-                wait_vmcnt<0>();
-                tile(kt, min(kt + 2, nk - 1), (kt + 1) % kStages, R1, R0);
-                wait_vmcnt<0>();
-                tile(kt + 1, min(kt + 3, nk - 1), kt % kStages, R0, R1);
-            }
-            if (kt < nk) {
-                wait_vmcnt<0>();
-                tile(kt, nk - 1, (kt + 1) % kStages, R1, R0);
-            }
+            for (; kt + kSets <= nk; kt += kSets)
+                each_of<kSets>([&](auto d) { turn(kt + d(), d); });
+            each_of<kSets - 1>([&](auto d) {
+                if (kt + d() < nk) turn(kt + d(), d);
+            });
         }
     } else {
         // Tile t goes to stage t % kStages.  The prologue issues tiles
@@ -1038,7 +1105,7 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
             asm volatile("s_barrier" ::: "memory");
             frag(lds, lds + kASz, 0, ca, cb);
             for (int kt = 0; kt < nk; ++kt)
-                tile(kt, min(kt + kAhead, nk - 1), (kt + kAhead) % kStages, nullptr, nullptr);
+                tile(kt, min(kt + kAhead, nk - 1), (kt + kAhead) % kStages, nullptr, nullptr, kt);
             wait_vmcnt<0>();  // the reloads past the last tile, before the LDS reuse
         }
     }
@@ -1061,14 +1128,16 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
             for (int j = 0; j < TN; ++j) bcol[j] = min(n0 + wn0 + 32 * j + l32, p.N - 1);
             auto eight = [&](const uint16_t *base, int ld, bool kc, int r, int k8) {
                 u32x4 v;
-                if (kc) {
-                    v = *reinterpret_cast<const u32x4 *>(base + (size_t)r * ld + min(k8, p.K - 8));
+                if (kc && (!kAny || ((p.K & 7) == 0 && !ODD))) {
+                    v = *reinterpret_cast<const u32x4_u4 *>(base + (size_t)r * ld +
+                                                            min(k8, p.K - 8));
                     if (k8 >= p.K) v = u32x4{0u, 0u, 0u, 0u};
                 } else {
                     uint16_t e[8];
 #pragma unroll
                     for (int t = 0; t < 8; ++t) {
-                        const uint16_t x = base[(size_t)min(k8 + t, p.K - 1) * ld + r];
+                        const int k = min(k8 + t, p.K - 1);
+                        const uint16_t x = kc ? base[(size_t)r * ld + k] : base[(size_t)k * ld + r];
                         e[t] = k8 + t < p.K ? x : (uint16_t)0;
                     }
                     v = u32x4{pack2(e[0], e[1]), pack2(e[2], e[3]), pack2(e[4], e[5]),
@@ -1110,7 +1179,7 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
     constexpr bool kDirect = TN % 2 == 0 && TM * TN <= 8;
     bool direct = false;
     if constexpr (kDirect)
-        direct = p.vec_out && m0 + BM <= p.M && n0 + BN <= p.N && (p.ksplit == 0 || p.N % 4 == 0);
+        direct = m0 + BM <= p.M && n0 + BN <= p.N;
     if (direct) {
         if constexpr (kDirect) store_direct16<BF, TM, TN>(p, acc, m0 + wm0, n0 + wn0, lane);
     } else {
@@ -1119,9 +1188,10 @@ __device__ __forceinline__ void gemm16_pipe_body(Args p, int bx, int by) {
     }
 }
 
-template <int BM, int BN, int BK, int WGM, int WGN, bool AK, bool BNC, bool BF, bool KT = false>
+template <int BM, int BN, int BK, int WGM, int WGN, bool AK, bool BNC, bool BF, bool KT = false,
+          bool ODD = false>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm16_pipe(Args p) {
-    gemm16_pipe_body<BM, BN, BK, WGM, WGN, AK, BNC, BF, 0, KT>(p, blockIdx.x, blockIdx.y);
+    gemm16_pipe_body<BM, BN, BK, WGM, WGN, AK, BNC, BF, 0, KT, ODD>(p, blockIdx.x, blockIdx.y);
 }
 
 // A large layer's weight gradient (TN, 256x256 tiles, 8 waves, BK 64, direct
@@ -1149,8 +1219,6 @@ void launch_pair16(Args a1, Args a2, hipStream_t st) {
     const int n1 = a1.tiles_m * a1.tiles_n, n2 = a2.tiles_m * a2.tiles_n;
     gemm16_pair_big<BF><<<n1 + n2, 512, 0, st>>>(a1, a2, n1);
 }
-// The pair's configurations (see launch_layout): dW on cfg 6, dX on cfg 8.
-constexpr int kPair16CfgW = 6, kPair16CfgX = 8;
 
 // The slots of a K-split GEMM summed in slot order (fp32), then the GEMM's
 // epilogue applied to each sum exactly as the kernel applies it to its own
@@ -1175,13 +1243,21 @@ __global__ __launch_bounds__(256) void sum_slices16(Args p, int splits) {
         }
     }
     const float *src = p.partial + (size_t)row * p.N + col;
-    if (p.vec_out && p.N % 4 == 0) {
-        f32x4 v = *reinterpret_cast<const f32x4 *>(src);
-#pragma unroll 1
-        for (int s = 1; s < splits; ++s) v += *reinterpret_cast<const f32x4 *>(src + s * slot);
+    if (col + 4 <= p.N) {
+        f32x4 v = *reinterpret_cast<const f32x4_u *>(src);
+        int s = 1;
+        for (; s + 4 <= splits; s += 4) {  // four slots' loads in flight
+            f32x4 x[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                x[q] = *reinterpret_cast<const f32x4_u *>(src + (s + q) * slot);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v += x[q];
+        }
+        for (; s < splits; ++s) v += *reinterpret_cast<const f32x4_u *>(src + s * slot);
         f32x4 bv = {0.f, 0.f, 0.f, 0.f};
         if (p.mode == 0 && p.bias) {
-            const u32x2 w = *reinterpret_cast<const u32x2 *>(p.bias + col);
+            const u32x2 w = *reinterpret_cast<const u32x2_u *>(p.bias + col);
             bv = f32x4{E::to_f((uint16_t)w[0]), E::to_f((uint16_t)(w[0] >> 16)),
                        E::to_f((uint16_t)w[1]), E::to_f((uint16_t)(w[1] >> 16))};
         }
@@ -1209,13 +1285,14 @@ void launch_sum16(const Args &a, int splits, hipStream_t st) {
     sum_slices16<BF><<<(unsigned)((threads + 255) / 256), 256, 0, st>>>(a, splits);
 }
 
-template <int BM, int BN, int WGM, int WGN, int BK, bool AK, bool BNC, bool BF, bool KT = false>
+template <int BM, int BN, int WGM, int WGN, int BK, bool AK, bool BNC, bool BF, bool KT = false,
+          bool ODD = false>
 void launch_pipe16(const Args &a0, hipStream_t st) {
     Args a = a0;
     a.tiles_m = (a.M + BM - 1) / BM;
     a.tiles_n = (a.N + BN - 1) / BN;
     const int splits = a.ksplit > 0 ? (a.K + a.ksplit - 1) / a.ksplit : 1;
-    gemm16_pipe<BM, BN, BK, WGM, WGN, AK, BNC, BF, KT>
+    gemm16_pipe<BM, BN, BK, WGM, WGN, AK, BNC, BF, KT, ODD>
         <<<dim3(a.tiles_m * a.tiles_n, splits), 64 * WGM * WGN, 0, st>>>(a);
     if (splits > 1) launch_sum16<BF>(a, splits, st);
 }
@@ -1230,60 +1307,56 @@ void launch_one(const Args &a0, hipStream_t st) {
 }
 
 // Tile configurations (BM x BN, waves, K depth):
-//   0: 256x256, 4 waves, BK 32     1: 256x256, 8 waves, BK 32
-//   2: 128x128, 4 waves, BK 32     3:  64x64,  4 waves, BK 32
-//   4: 256x128, 4 waves, BK 32     5: 256x256, 4 waves, BK 64
-//   6: 256x256, 8 waves, BK 64     7: 256x128, 4 waves, BK 64
-//   8: 256x128, 8 waves, BK 64      9: 8's tiles with a K tail (K % 64 != 0)
-// 64x64 is also the only element-load variant, for unaligned operands.
-constexpr int kNumCfgs = 10;
-constexpr int kCfgKTail16 = 9;
+//   0: 256x256, 8 waves, BK 32      1: 128x128, 4 waves, BK 32
+//   2: 256x256, 8 waves, BK 64      3: 256x128, 8 waves, BK 64
+//   4: 3's tiles with a K tail (K % 64 != 0)
+//   5, 6: 0's and 1's with a K tail and rows of any 4-byte alignment
+//   7, 8: and rows that start on odd elements
+//   9:  64x64, 4 waves, BK 32 (gemm16_mfma), for under 8 rows or columns
+enum : int {
+    kCfg256 = 0, kCfg128 = 1, kCfgBig = 2, kCfgMid = 3, kCfgMidTail = 4, kCfgAny256 = 5,
+    kCfgAny128 = 6, kCfgOdd256 = 7, kCfgOdd128 = 8, kCfgSmall = 9
+};
 
 // K depth of a configuration.
-inline int cfg_bk16(int cfg) { return cfg >= 5 ? 64 : 32; }
+inline int cfg_bk16(int cfg) { return cfg >= kCfgBig && cfg <= kCfgMidTail ? 64 : 32; }
+// Output tile.
+inline void cfg_tile16(int cfg, int &bm, int &bn) {
+    const bool t128 = cfg == kCfg128 || cfg == kCfgAny128 || cfg == kCfgOdd128;
+    const bool mid = cfg == kCfgMid || cfg == kCfgMidTail;
+    bm = cfg == kCfgSmall ? 64 : t128 ? 128 : 256;
+    bn = cfg == kCfgSmall ? 64 : t128 || mid ? 128 : 256;
+}
 
 template <bool AK, bool BNC, bool BF>
-void launch_layout(const Args &a, bool vec, bool pipe, int cfg, hipStream_t st) {
-    if (!vec) {
-        launch_one<64, 64, 2, 2, 32, AK, BNC, false, BF>(a, st);
-        return;
-    }
-    if (pipe && cfg != 3) {
-        switch (cfg) {
-            case 0: launch_pipe16<256, 256, 2, 2, 32, AK, BNC, BF>(a, st); break;
-            case 1: launch_pipe16<256, 256, 2, 4, 32, AK, BNC, BF>(a, st); break;
-            case 2: launch_pipe16<128, 128, 2, 2, 32, AK, BNC, BF>(a, st); break;
-            case 4: launch_pipe16<256, 128, 2, 2, 32, AK, BNC, BF>(a, st); break;
-            case 5: launch_pipe16<256, 256, 2, 2, 64, AK, BNC, BF>(a, st); break;
-            case 6: launch_pipe16<256, 256, 2, 4, 64, AK, BNC, BF>(a, st); break;
-            case 7: launch_pipe16<256, 128, 2, 2, 64, AK, BNC, BF>(a, st); break;
-            case kCfgKTail16: launch_pipe16<256, 128, 4, 2, 64, AK, BNC, BF, true>(a, st); break;
-            default: launch_pipe16<256, 128, 4, 2, 64, AK, BNC, BF>(a, st); break;
-        }
-        return;
-    }
+void launch_layout(const Args &a, bool vec, int cfg, hipStream_t st) {
     switch (cfg) {
-        case 0: launch_one<256, 256, 2, 2, 32, AK, BNC, true, BF>(a, st); break;
-        case 1: launch_one<256, 256, 2, 4, 32, AK, BNC, true, BF>(a, st); break;
-        case 2: launch_one<128, 128, 2, 2, 32, AK, BNC, true, BF>(a, st); break;
-        case 4: launch_one<256, 128, 2, 2, 32, AK, BNC, true, BF>(a, st); break;
-        case 5: launch_one<256, 256, 2, 2, 64, AK, BNC, true, BF>(a, st); break;
-        case 6: launch_one<256, 256, 2, 4, 64, AK, BNC, true, BF>(a, st); break;
-        case 7: launch_one<256, 128, 2, 2, 64, AK, BNC, true, BF>(a, st); break;
-        case 8:
-        case kCfgKTail16: launch_one<256, 128, 4, 2, 64, AK, BNC, true, BF>(a, st); break;
-        default: launch_one<64, 64, 2, 2, 32, AK, BNC, true, BF>(a, st); break;
+        case kCfg256: launch_pipe16<256, 256, 2, 4, 32, AK, BNC, BF>(a, st); break;
+        case kCfg128: launch_pipe16<128, 128, 2, 2, 32, AK, BNC, BF>(a, st); break;
+        case kCfgBig: launch_pipe16<256, 256, 2, 4, 64, AK, BNC, BF>(a, st); break;
+        case kCfgMid: launch_pipe16<256, 128, 4, 2, 64, AK, BNC, BF>(a, st); break;
+        case kCfgMidTail: launch_pipe16<256, 128, 4, 2, 64, AK, BNC, BF, true>(a, st); break;
+        case kCfgAny256: launch_pipe16<256, 256, 2, 4, 32, AK, BNC, BF, true>(a, st); break;
+        case kCfgAny128: launch_pipe16<128, 128, 2, 2, 32, AK, BNC, BF, true>(a, st); break;
+        case kCfgOdd256: launch_pipe16<256, 256, 2, 4, 32, AK, BNC, BF, true, true>(a, st); break;
+        case kCfgOdd128: launch_pipe16<128, 128, 2, 2, 32, AK, BNC, BF, true, true>(a, st); break;
+        default:
+            if (vec)
+                launch_one<64, 64, 2, 2, 32, AK, BNC, true, BF>(a, st);
+            else
+                launch_one<64, 64, 2, 2, 32, AK, BNC, false, BF>(a, st);
+            break;
     }
 }
 
 // Defined in k_gemm16_{bf16,f16}.hip.  layout: FG_NN / FG_NT / FG_TN.
-void launch_bf16(int layout, const Args &a, bool vec, bool pipe, int cfg, hipStream_t st);
-void launch_f16(int layout, const Args &a, bool vec, bool pipe, int cfg, hipStream_t st);
+void launch_bf16(int layout, const Args &a, bool vec, int cfg, hipStream_t st);
+void launch_f16(int layout, const Args &a, bool vec, int cfg, hipStream_t st);
 // sum_slices16 of a's slots.
 void launch_sum_bf16(const Args &a, int splits, hipStream_t st);
 void launch_sum_f16(const Args &a, int splits, hipStream_t st);
-// gemm16_pair_big: dW (TN, a1) and dX (NT, a2), both planned pipelined on
-// kPair16CfgW / kPair16CfgX without a K split.
+// gemm16_pair_big: dW (TN, a1) and dX (NT, a2), planned on kCfgBig and kCfgMid
+// without a K split.
 void launch_pair_bf16(const Args &a1, const Args &a2, hipStream_t st);
 void launch_pair_f16(const Args &a1, const Args &a2, hipStream_t st);
 

@@ -41,9 +41,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
-#include <utility>
-
 #include "fg_act.h"
 #include "fg_sched.h"
 
@@ -770,16 +767,6 @@ struct PipeLds {
     static constexpr int kEpi = WGM * WGN * 32 * (BN / WGN + 4);
     static constexpr int floats = (kStages * kStageSz > kEpi) ? kStages * kStageSz : kEpi;
 };
-
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>), in order.
-template <class F, int... I>
-__device__ __forceinline__ void each_of_seq(F f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void each_of(F f) {
-    each_of_seq(f, std::make_integer_sequence<int, N>{});
-}
 
 // Register sets of a staged tile, i.e. tiles in flight.  A 64x64 tile is a
 // quarter of a microsecond of MFMAs, less than a load takes, and often the only

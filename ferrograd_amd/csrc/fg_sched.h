@@ -1,9 +1,23 @@
-// fg_sched.h -- wait-count helpers shared by the MFMA GEMM main loops.
+// fg_sched.h -- wait-count and unrolling helpers shared by the MFMA GEMM main loops.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+#include <utility>
+
 namespace fg {
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>), in order.
+template <class F, int... I>
+__device__ __forceinline__ void each_of_seq(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void each_of(F f) {
+    each_of_seq(f, std::make_integer_sequence<int, N>{});
+}
+
 
 // s_waitcnt with vmcnt <= N and no wait on the other counters.
 template <int N>

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <iterator>
 
 #include "fg_gemm16_kernel.h"
 #include "fg_gemm_rows.h"
@@ -13,126 +14,143 @@ namespace {
 
 using fg::gemm16::Args;
 
-// Pipelined whole-tile kernel on (1) or off (0): a knob for measurement builds.
-#ifndef FG_GEMM16_PIPE
-#define FG_GEMM16_PIPE 1
-#endif
-constexpr bool kPipe16 = FG_GEMM16_PIPE != 0;
-
 int tiles(int M, int N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-// Tile configuration (indices as in fg_gemm16_kernel.h), from a measured
-// sweep on MI355X of every configuration of the pipelined kernel (TFLOP/s,
-// bf16, N(0,1) operands; fp16 within a few percent):
-//  * squares that give >= one 256x256 tile per CU: 256x256 with 8 waves and
-//    BK 64, direct loads, every layout: 1134-1162 / 1141-1171 / 1117-1145
-//    (NN / NT / TN) at 4096^3 and 995-1003 for the 4096x4096x2048 weight
-//    gradient, against 1115-1145 / 1143-1171 / 1117-1151 and 938-947 for
-//    the staged BK 32 tile, and 1070-1098 / 1075-1105 / 1050-1080 and 839-846
-//    for 4 waves (one per SIMD: each wave's waits idle its matrix unit).
-//    The direct loads are issued as inline assembly (lds_dma16): as builtins
-//    the compiler made every transposing LDS read wait for all of them in
-//    flight (933 / 714 / 600 then);
-//  * else 256x128 with 8 waves and BK 64 down to a quarter tile per CU: 956
-//    for the 2048x4096x4096 forward, 799-855 for its NT data gradient, 302
-//    for the 1000-wide head, where every smaller tile measured lower;
-//  * else 128x128, else 64x64.
-// The BK 64 tiles need K % 64 == 0; when only K % 32 == 0 holds, 256x256
-// with 8 waves and BK 32 or 128x128 keep the pipelined kernel.  Other K take
-// the 256x128 8-wave tiles where they give a quarter tile per CU: pipelined
-// with a K tail (plan16), or gemm16_mfma where the operands do not allow it.
-int pick_cfg16(int layout, int M, int N, int K, int cus) {
-    if (K % 64 == 0) {
-        if (tiles(M, N, 256, 256) >= cus) return 6;
-        if (tiles(M, N, 256, 128) >= cus / 4) return 8;
-    } else if (K % 32 == 0) {
-        if (tiles(M, N, 256, 256) >= cus) return 1;
-    } else if (tiles(M, N, 256, 128) >= cus / 4) {
-        return 8;  // gemm16_mfma: 529 against 453 for 128x128 (2048x4096x1000 NT)
-    }
-    if (tiles(M, N, 128, 128) >= cus / 4) return 2;
-    return 3;
+// How a call's rows lie: whole 16-byte chunks on 16-byte boundaries, on
+// 4-byte ones, or on odd elements.
+enum Rows { kRowsWhole = 0, kRowsEven = 1, kRowsOdd = 2 };
+// Of operands given by address and leading dimension (multiples of 8 with
+// aligned bases, and row-contiguous operands' row lengths too, are whole).
+Rows rows_of(int layout, int M, int N, const void *A, int lda, const void *B, int ldb) {
+    const uintptr_t ab = (uintptr_t)A | (uintptr_t)B;
+    const int ld = lda | ldb;
+    if ((ab & 3u) || (ld & 1)) return kRowsOdd;
+    const bool rc = (layout == FG_NT || N % 8 == 0) && (layout != FG_TN || M % 8 == 0);
+    return (ab & 15u) == 0 && ld % 8 == 0 && rc ? kRowsWhole : kRowsEven;
 }
 
-// K slices for a pipelined GEMM whose output tiles fill at most half the
-// CUs (the 1000-wide head and the 1024-wide layer's data gradient of a
-// batch-2048 MLP: 64 tiles of 256x128): enough slices to give every CU a
-// workgroup, each of whole K tiles and at least four of them.  Returns the
-// number of slices (1: no split) and their depth in ks.
-int split16(int cus, int M, int N, int K, int cfg, int &ks) {
-    ks = 0;
-    const int bk = fg::gemm16::cfg_bk16(cfg);
-    // the configurations' tiles (fg_gemm16_kernel.h)
-    const int bm = cfg == 2 ? 128 : cfg == 3 ? 64 : 256;
-    const int bn = (cfg == 2 || cfg == 4 || cfg >= 7) ? 128 : cfg == 3 ? 64 : 256;
-    const int t = tiles(M, N, bm, bn);
-    if (2 * t > cus || K < 8 * bk) return 1;
-    int s = std::min(cus / t, K / (4 * bk));
-    if (s < 2) return 1;
-    int k = (K + s - 1) / s;
-    k = (k + bk - 1) / bk * bk;  // whole K tiles per slice
-    s = (K + k - 1) / k;
-    if (s < 2) return 1;
-    ks = k;
-    return s;
+// Tile configuration and K slices of a pipelined call (M, N >= 8) by a model
+// of its time: a CU with n workgroups takes n tiles' time, a tile its k times
+// kRate (us per k per 64x64 of output, measured on MI355X, bf16, N(0,1)
+// operands, HIP events, 512^3 to 4096^3) and a fixed part that grows with it
+// (pipeline fill, output); slices cut the depth for a summing launch and the
+// slots' traffic.  With the fused column sums each slice also leaves N fp32
+// sums, after the output slots.  Modelled against measured (us, NN): 2048 x 1000
+// x 4096 on 128x128 tiles in two slices 33 / 33, on 256x128 in four 36 / 37; 2046
+// x 4094 x 4094 on 256x256 in two 100 / 100, unsplit 131 / 127.  The candidates'
+// order settles ties: the larger tiles first.
+//
+// Rows that are not whole chunks took one element a lane before (us): 2047 x
+// 4095 x 4093 NN 975 -> 116, NT 1363 -> 121, 777 x 1333 x 2049 120 -> 27, 300^3
+// 16.1 -> 10.8; 1000^3 (K not whole tiles) NN / NT / TN 58 / 35 / 102 -> 17 / 15 / 18.
+// Of the whole-row calls, those with under a 256x128 tile per CU changed tiles:
+// 1024^3 20.5 / 19.8 / 21.1 -> 15.4 / 13.2 / 17.2, 128 x 4096 x 4096 NN 87 -> 19.
+struct Rate16 {
+    int cfg;
+    float nn, nt, tn;
+};
+constexpr Rate16 kWhole[] = {{fg::gemm16::kCfgBig, 0.0017f, 0.0017f, 0.0017f},
+                             {fg::gemm16::kCfgMid, 0.0021f, 0.0021f, 0.0021f},
+                             {fg::gemm16::kCfgMidTail, 0.0022f, 0.0022f, 0.0022f},
+                             {fg::gemm16::kCfg256, 0.0018f, 0.0019f, 0.0024f},
+                             {fg::gemm16::kCfg128, 0.0026f, 0.0023f, 0.0032f},
+                             {fg::gemm16::kCfgAny256, 0.0018f, 0.0019f, 0.0024f},
+                             {fg::gemm16::kCfgAny128, 0.0026f, 0.0023f, 0.0032f},
+                             // (not pipelined, no slices or column sums: NN and
+                             // NT with K up to 512; 256^3 7.8 / 5.9 us, on
+                             // 128x128 tiles 9.0 / 6.4)
+                             {fg::gemm16::kCfgSmall, 0.010f, 0.005f, 1.0f}};
+constexpr Rate16 kEven[] = {{fg::gemm16::kCfgAny256, 0.0018f, 0.0020f, 0.0025f},
+                            {fg::gemm16::kCfgAny128, 0.0033f, 0.0036f, 0.0030f},
+                            // (one element a lane: 100 x 4000 x 100 NN 8.9 us,
+                            // on 128x128 tiles 10.5)
+                            {fg::gemm16::kCfgSmall, 0.030f, 0.022f, 1.0f}};
+constexpr Rate16 kOdd[] = {{fg::gemm16::kCfgOdd256, 0.0024f, 0.0026f, 0.0030f},
+                           {fg::gemm16::kCfgOdd128, 0.0041f, 0.0047f, 0.0037f},
+                           {fg::gemm16::kCfgSmall, 0.030f, 0.022f, 1.0f}};
+constexpr float kTileUs = 1.5f, kTileUnitUs = 0.4f;       // fixed, and per 64x64
+constexpr float kTailUs = 1.0f;                           // a K tail
+constexpr float kSumUs16 = 2.0f, kSumBytesPerUs16 = 6.0e6f;
+
+struct Choice16 {
+    int cfg = fg::gemm16::kCfgSmall, splits = 1, ks = 0;
+    float us = 1e30f;
+};
+Choice16 choose16(int layout, int M, int N, int K, int cus, Rows rows, bool colsum,
+                  uint64_t ws_bytes) {
+    using namespace fg::gemm16;
+    Choice16 best;
+    const Rate16 *r = rows == kRowsWhole ? kWhole : rows == kRowsEven ? kEven : kOdd;
+    const Rate16 *end = rows == kRowsWhole  ? std::end(kWhole)
+                        : rows == kRowsEven ? std::end(kEven)
+                                            : std::end(kOdd);
+    for (; r != end; ++r) {
+        // Whole K tiles, but for the tails': that of 256x128 takes k-contiguous
+        // rows eight at a time.
+        const int bk = cfg_bk16(r->cfg);
+        if (r->cfg == kCfgMidTail) {
+            if (K % bk == 0 || (layout != FG_TN && K % 8 != 0)) continue;
+        } else if (r->cfg < kCfgMidTail) {
+            if (K % bk != 0) continue;
+        }
+        if (r->cfg == kCfgSmall && K > 512) continue;
+        const float fixed = kTileUs + (K % bk != 0 && r->cfg != kCfgSmall ? kTailUs : 0.0f);
+        int bm, bn;
+        cfg_tile16(r->cfg, bm, bn);
+        const int64_t t = tiles(M, N, bm, bn);
+        const int units = (bm / 64) * (bn / 64);
+        const float rate = (layout == FG_NN ? r->nn : layout == FG_NT ? r->nt : r->tn) * units;
+        for (int s = 1; s <= 16; ++s) {
+            int ks = K;
+            if (s > 1) {
+                // At least eight K tiles in all and four a slice, whole ones;
+                // slices only while the CUs have under two tiles each.
+                if (r->cfg == kCfgSmall || K < 8 * bk || s > K / (4 * bk) ||
+                    t * s > 2 * (int64_t)cus)
+                    break;
+                ks = ((K + s - 1) / s + bk - 1) / bk * bk;
+                if ((K + ks - 1) / ks != s) continue;
+                if ((uint64_t)s * ((uint64_t)M * N + (colsum ? N : 0)) * sizeof(float) > ws_bytes)
+                    break;
+            }
+            float us = (float)((t * s + cus - 1) / cus) * (ks * rate + fixed + kTileUnitUs * units);
+            if (s > 1) us += kSumUs16 + (2 * s + 1) * (float)M * N * 4.0f / kSumBytesPerUs16;
+            if (us < 0.99f * best.us) best = Choice16{r->cfg, s, s > 1 ? ks : 0, us};
+        }
+    }
+    return best;
 }
 
 // The kernel choices of one call (operands as passed, colsum included).
 struct Plan16 {
-    bool vec = false, pipe = false;
     bool rows = false;  // the few-row kernel (fg_gemm_rows.h); then only splits and ks apply
-    int cfg = 3, splits = 1, ks = 0;
+    bool pipe = false;  // else gemm16_mfma, with 16-byte operand loads (vec) or not
+    bool vec = false;
+    int cfg = fg::gemm16::kCfgSmall, splits = 1, ks = 0;
 };
 Plan16 plan16(const fg_ctx *ctx, int layout, const Args &a) {
     Plan16 q;
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    // K slices go into the context's workspace when what is reserved holds
+    // them (it is never grown for this), summed by a second kernel in slot
+    // order -- deterministic, within the GEMM tolerance of the unsplit sum.
+    const uint64_t ws = ctx->ws ? ctx->ws_bytes : 0;
     // Few rows (up to 64), any alignment: bf16 16 x 4096 x 4096 97.5 -> 11.8 us,
     // 64 x 4096 x 4096 98.7 -> 17.0, 64 x 1000 x 2048 94.3 -> 12.2, 64 x 1001 x
     // 2049 99.8 -> 13.8, 40 x 300 x 333 19 -> 5.8 against the tiles below.
     if (!a.colsum && fg::rows::applies(layout, a.M, a.N, a.K)) {
         q.rows = true;
-        q.splits = fg::rows::split_of(cus, 2, a.M, a.N, a.K, ctx->ws ? ctx->ws_bytes : 0, q.ks);
+        q.splits = fg::rows::split_of(cus, 2, a.M, a.N, a.K, ws, q.ks);
         return q;
     }
-    // 16-byte operand loads need 16-byte aligned bases and leading
-    // dimensions that keep every row start aligned (multiples of 8
-    // elements); the bounds checks split per 8-element vector, so the
-    // extents themselves are free.
-    auto al = [](const void *p, unsigned m) { return (((uintptr_t)p) & (m - 1)) == 0; };
-    q.vec = al(a.A, 16) && al(a.B, 16) && a.lda % 8 == 0 && a.ldb % 8 == 0;
-#ifdef FG_GEMM16_FORCE_CFG  // tuning builds: one tile configuration for every shape
-    q.cfg = FG_GEMM16_FORCE_CFG;
-#else
-    q.cfg = pick_cfg16(layout, a.M, a.N, a.K, cus);
-#endif
-    // The pipelined kernel: whole K tiles, 16-byte chunks of 8 elements along
-    // each row-contiguous operand's rows (B of NN / TN, A of TN).
-    const bool rc_ok = (layout == FG_NT || a.N % 8 == 0) && (layout != FG_TN || a.M % 8 == 0);
-    q.pipe = kPipe16 && q.vec && rc_ok && a.K > 0 && a.K % fg::gemm16::cfg_bk16(q.cfg) == 0 &&
-             a.M >= 8 && a.N >= 8 && q.cfg != 3;
-    // K not a multiple of 32 on the 256x128 8-wave tiles (the 1000-deep data
-    // gradient of a 1000-wide head): the pipelined kernel over the whole
-    // tiles with the K tail from global memory, where each k-contiguous
-    // operand's rows hold whole 8-element chunks of k (K % 8 == 0).
-    if (!q.pipe && q.cfg == 8 && kPipe16 && q.vec && rc_ok && a.K > 0 && a.M >= 8 && a.N >= 8 &&
-        (layout == FG_TN || a.K % 8 == 0)) {
-        q.pipe = true;
-        q.cfg = fg::gemm16::kCfgKTail16;
-    }
-    // Few tiles and a long K: K slices into the context's workspace when
-    // what is reserved holds them (it is never grown for this), summed by a
-    // second kernel in slot order -- deterministic, within the GEMM
-    // tolerance of the unsplit sum.  With the fused column sums each slice
-    // also leaves N fp32 sums, after the output slots.
-    if (q.pipe && ctx->ws) {
-        int ks;
-        const int sl = split16(cus, a.M, a.N, a.K, q.cfg, ks);
-        const uint64_t need = (uint64_t)sl * ((uint64_t)a.M * a.N + (a.colsum ? a.N : 0));
-        if (sl > 1 && need * sizeof(float) <= ctx->ws_bytes) {
-            q.splits = sl;
-            q.ks = ks;
-        }
-    }
+    const Rows rows = rows_of(layout, a.M, a.N, a.A, a.lda, a.B, a.ldb);
+    q.vec = rows == kRowsWhole;
+    if (a.K <= 0 || a.M < 8 || a.N < 8) return q;
+    const Choice16 ch = choose16(layout, a.M, a.N, a.K, cus, rows, a.colsum != nullptr, ws);
+    q.pipe = ch.cfg != fg::gemm16::kCfgSmall;
+    q.cfg = ch.cfg;
+    q.splits = ch.splits;
+    q.ks = ch.ks;
     return q;
 }
 
@@ -149,13 +167,6 @@ int gemm16_check(fg_ctx *ctx, int dtype, int layout, const Args &a, const char *
     FG_REQUIRE(a.lda >= std::max(a_cols, 1) && a.ldb >= std::max(b_cols, 1) && a.ldc >= a.N,
                FG_ERR_SHAPE, "%s: leading dimension too small", who);
     return FG_OK;
-}
-
-// 8-byte epilogue I/O where C / Z / bias allow it.
-void set_vec_out(Args &a) {
-    auto al = [](const void *q, unsigned m) { return (((uintptr_t)q) & (m - 1)) == 0; };
-    a.vec_out = al(a.C, 8) && a.ldc % 4 == 0 && (!a.Z || (al(a.Z, 8) && a.ldz % 4 == 0)) &&
-                (!a.bias || al(a.bias, 8));
 }
 
 int gemm16_common(fg_ctx *ctx, int dtype, int layout, Args &a, const char *who) {
@@ -183,7 +194,6 @@ int gemm16_common(fg_ctx *ctx, int dtype, int layout, Args &a, const char *who) 
     FG_HIP(hipSetDevice(ctx->device));
     uint16_t *colsum = a.colsum;  // the bias gradient of fg_gemm_dw_x16, if any
     if (a.K == 0) a.A = a.B;  // loads are all masked; K=0 yields the epilogue of zero
-    set_vec_out(a);
     const Plan16 q = plan16(ctx, layout, a);
     // Only the pipelined kernel sums B's columns; elsewhere the separate
     // reduction runs after the GEMM (same result up to the order of the
@@ -202,9 +212,9 @@ int gemm16_common(fg_ctx *ctx, int dtype, int layout, Args &a, const char *who) 
                 fg::gemm16::launch_sum_f16(a, q.splits, ctx->stream);
         }
     } else if (dtype == FG_DTYPE_BF16)
-        fg::gemm16::launch_bf16(layout, a, q.vec, q.pipe, q.cfg, ctx->stream);
+        fg::gemm16::launch_bf16(layout, a, q.vec, q.cfg, ctx->stream);
     else
-        fg::gemm16::launch_f16(layout, a, q.vec, q.pipe, q.cfg, ctx->stream);
+        fg::gemm16::launch_f16(layout, a, q.vec, q.cfg, ctx->stream);
     FG_LAUNCH_CHECK(who);
     if (colsum && !q.pipe)
         return fg_bias_grad(ctx, dtype, a.K, a.N, a.B, a.ldb, colsum, a.colsum_accumulate);
@@ -254,11 +264,9 @@ Args dx_args16(int M, int N, int K, const void *A, int lda, const void *B, int l
 // Both pipelined on the pair's configurations, neither split.
 bool pairable16(fg_ctx *ctx, Args &w, Args &x) {
     if (w.M <= 0 || w.N <= 0 || w.K <= 0 || x.M <= 0 || x.N <= 0 || x.K <= 0) return false;
-    set_vec_out(w);
-    set_vec_out(x);
     const Plan16 qw = plan16(ctx, FG_TN, w), qx = plan16(ctx, FG_NT, x);
     return qw.pipe && qx.pipe && qw.splits == 1 && qx.splits == 1 &&
-           qw.cfg == fg::gemm16::kPair16CfgW && qx.cfg == fg::gemm16::kPair16CfgX;
+           qw.cfg == fg::gemm16::kCfgBig && qx.cfg == fg::gemm16::kCfgMid;
 }
 
 }  // namespace
@@ -331,7 +339,7 @@ int gemm16_dispatches(fg_ctx *ctx, int layout, int M, int N, int K, const void *
 
 // Workspace bytes a 16-bit GEMM of this shape splits K into when the
 // workspace holds them (0: it does not split), for planners that size a
-// workspace ahead.  Assumes the pipelined kernel (aligned operands).
+// workspace ahead.
 uint64_t gemm16_split_ws_bytes(int cus, int layout, int M, int N, int K, bool colsum) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     cus = cus > 0 ? cus : 256;
@@ -340,11 +348,13 @@ uint64_t gemm16_split_ws_bytes(int cus, int layout, int M, int N, int K, bool co
         const int sl = fg::rows::split_of(cus, 2, M, N, K, ~0ull, ks);
         return sl > 1 ? (uint64_t)sl * M * N * sizeof(float) : 0;
     }
-    const int cfg = pick_cfg16(layout, M, N, K, cus);
-    if (cfg == 3 || K % fg::gemm16::cfg_bk16(cfg) != 0) return 0;
-    int ks;
-    const int sl = split16(cus, M, N, K, cfg, ks);
-    return sl > 1 ? (uint64_t)sl * ((uint64_t)M * N + (colsum ? N : 0)) * sizeof(float) : 0;
+    if (M < 8 || N < 8) return 0;
+    // Dense rows from aligned bases.
+    const int lda = layout == FG_TN ? M : K, ldb = layout == FG_NT ? K : N;
+    const Choice16 ch = choose16(layout, M, N, K, cus, rows_of(layout, M, N, nullptr, lda, nullptr, ldb),
+                                 colsum, ~0ull);
+    return ch.splits > 1 ? (uint64_t)ch.splits * ((uint64_t)M * N + (colsum ? N : 0)) * sizeof(float)
+                         : 0;
 }
 }  // namespace fg
 

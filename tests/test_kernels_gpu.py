@@ -764,6 +764,66 @@ def test_gemm_f32_any_rows(gpu_ctx, layout, place):
             assert torch.equal(got(), torch.where(zs > 0, ref, torch.zeros_like(ref)))
 
 
+# 16-bit tiles on rows of any alignment, as test_gemm_f32_any_rows: K
+# remainders of the tile pipeline (1 to 6 tiles of 32 and a tail), rows that end
+# between chunks, even and odd leading dimensions, K slices, edges of tiles.
+@pytest.mark.parametrize("place", ["plain", "even", "odd", "offset"])
+@pytest.mark.parametrize("layout", [O.NN, O.NT, O.TN], ids=["NN", "NT", "TN"])
+@pytest.mark.parametrize("dtype", [1, 2], ids=["f16", "bf16"])
+def test_gemm_x16_any_rows(gpu_ctx, dtype, layout, place):
+    """Small-integer operands (sums exact in fp32 and every fp32 sum below the
+    types' first rounding reproduced by one), with NaN around every row (even:
+    ld + 2, odd: ld + 3) and the tensors: outputs and column sums bit for bit."""
+    torch = _torch()
+    dt = [None, torch.float16, torch.bfloat16][dtype]
+    gpu_ctx.reserve_workspace(64 << 20)
+    g = torch.Generator().manual_seed(13)
+
+    def ints(r, c):
+        ld = c + {"even": 2, "odd": 3}.get(place, 0)
+        off = 1 if place == "offset" else 64
+        v = torch.randint(-3, 4, (r, c), generator=g).to(dt)
+        buf = torch.full((off + r * ld + 64,), float("nan"), dtype=dt)
+        buf[off:off + r * ld].view(r, ld)[:, :c] = v
+        buf = buf.cuda()
+        return v.double(), buf[off:], ld
+
+    shapes = [(129, 130, 32 * t + x) for t in range(1, 7) for x in (0, 1, 18)]
+    shapes += [(72, 8, 1), (65, 9, 7), (257, 66, 256), (128, 256, 64), (100, 201, 3000),
+               (500, 1000, 1500), (600, 2001, 400), (2048, 2050, 300)]
+    for M, N, K in shapes:
+        note(f"gemm_x16_any_rows {dtype} {layout} {place} {M}x{N}x{K}")
+        a, A, lda = ints(*((K, M) if layout == O.TN else (M, K)))
+        b, B, ldb = ints(*((N, K) if layout == O.NT else (K, N)))
+        old, C, ldc = ints(M, N)
+        ref = ((a.T if layout == O.TN else a) @ (b.T if layout == O.NT else b)).to(dt)
+
+        def got():
+            torch.cuda.synchronize()
+            return C[:M * ldc].view(M, ldc)[:, :N].cpu()
+
+        gpu_ctx.gemm_x16(dtype, layout, M, N, K, A, lda, B, ldb, C, ldc, accumulate=True)
+        assert torch.equal(got(), (ref.double() + old).to(dt))
+        if layout == O.TN:
+            cs, S, _ = ints(1, N)
+            gpu_ctx.gemm_dw_x16(dtype, M, N, K, A, lda, B, ldb, C, ldc, colsum=S,
+                                colsum_accumulate=True)
+            assert torch.equal(got(), ref)
+            assert torch.equal(S[:N].cpu(), (cs + b.sum(0)).reshape(-1).to(dt))
+        else:
+            zs, Zs, ldzs = ints(M, N)
+            gpu_ctx.gemm_bwd_x16(dtype, layout, M, N, K, A, lda, B, ldb, C, ldc, act=O.ACT_RELU,
+                                 Zs=Zs, ldzs=ldzs)
+            assert torch.equal(got(), torch.where(zs > 0, ref, torch.zeros_like(ref)))
+            bias, Bi, _ = ints(1, N)
+            Z = torch.empty(M, N + 1, dtype=dt, device="cuda")
+            gpu_ctx.gemm_x16(dtype, layout, M, N, K, A, lda, B, ldb, C, ldc, bias=Bi,
+                             act=O.ACT_RELU, Z=Z, ldz=N + 1)
+            z = (ref.double() + bias).to(dt)
+            assert torch.equal(got(), z.clamp(min=0))
+            assert torch.equal(Z[:, :N].cpu(), z)
+
+
 # --------------------------------------------------------- softmax + CE
 def check_softmax_ce(ctx, x, labels, scale=1.0):
     torch = _torch()
