@@ -379,8 +379,15 @@ int launch_eltwise(fg_ctx *ctx, const EltProgram &p0) {
         if (regs <= 8) return launch_file<8, 2, true>(ctx, p);
         return launch_file<16, 1, true>(ctx, p);
     }
-    if (regs <= 4) return launch_file<4, 3, false>(ctx, p);
-    if (regs <= 8) return launch_file<8, 2, false>(ctx, p);
+    // Under 2^20 elements (the programs that are not compiled) a launch is a
+    // chain of latencies, not bandwidth: one quad per thread, three times the
+    // waves, whatever the registers.  tanh(a*b + c) and its backward, us a
+    // launch on 4 x 3 -> 16 x 1: 1000 x 777 7.24 -> 5.76, 300 x 1000 6.40 -> 4.76, 32
+    // x 64 5.08 -> 3.88 (on 4 x 1, read through select chains: 6.32, 5.24, 4.24).
+    if (p.n >= (uint64_t(1) << 20)) {
+        if (regs <= 4) return launch_file<4, 3, false>(ctx, p);
+        if (regs <= 8) return launch_file<8, 2, false>(ctx, p);
+    }
     return launch_file<16, 1, false>(ctx, p);
 }
 

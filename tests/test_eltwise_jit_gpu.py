@@ -70,6 +70,9 @@ def _loss_input(ops, x):
 # cases take input 3 as a row vector.
 CASES = {
     "tanh-partial": (_tanh_chain, 3, 37, 1025, "MEAN_SQUARED_ERROR", "f32"),
+    # Both sides of 2^20 elements, where the interpreter changes register files.
+    "tanh-under-2^20": (_tanh_chain, 3, 1023, 1025, "MEAN_SQUARED_ERROR", "f32"),
+    "tanh-2^20": (_tanh_chain, 3, 1024, 1024, "MEAN_SQUARED_ERROR", "f32"),
     "tanh-streaming": (_tanh_chain, 3, 1031, 4099, "MEAN_SQUARED_ERROR", "f32"),
     "wide-small": (_wide, 7, 9, 301, "MEAN_SQUARED_ERROR", "f32"),
     "wide-streaming": (_wide, 7, 1100, 4097, "MEAN_SQUARED_ERROR", "f32"),
