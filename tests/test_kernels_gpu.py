@@ -824,6 +824,30 @@ def test_gemm_x16_any_rows(gpu_ctx, dtype, layout, place):
             assert torch.equal(Z[:, :N].cpu(), z)
 
 
+@pytest.mark.parametrize("dtype", [0, 1, 2], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("pad", [0, 1, 2])
+def test_bias_grad_any_rows(gpu_ctx, dtype, pad):
+    """Column sums of small integers (exact in fp32) over rows of any length and
+    alignment, NaN between them: 1 to 63 row splits, columns at the edges of
+    the summing workgroups."""
+    torch = _torch()
+    dt = [torch.float32, torch.float16, torch.bfloat16][dtype]
+    g = torch.Generator().manual_seed(17)
+    for M, N in [(1, 1), (15, 3), (17, 63), (64, 65), (200, 257), (1000, 130)]:
+        ld = N + pad
+        v = torch.randint(-3, 4, (M, N), generator=g).to(dt)
+        buf = torch.full((M * ld + 9,), float("nan"), dtype=dt)
+        buf[pad:pad + M * ld].view(M, ld)[:, :N] = v
+        buf = buf.cuda()
+        old = torch.randint(-9, 10, (N,), generator=g).to(dt)
+        for acc in (False, True):
+            out = old.clone().cuda()
+            gpu_ctx.bias_grad(M, N, buf[pad:], ld, out, accumulate=acc, dtype=dtype)
+            torch.cuda.synchronize()
+            ref = v.double().sum(0) + (old.double() if acc else 0.0)
+            assert torch.equal(out.cpu(), ref.to(dt)), (M, N, acc)
+
+
 # --------------------------------------------------------- softmax + CE
 def check_softmax_ce(ctx, x, labels, scale=1.0):
     torch = _torch()
