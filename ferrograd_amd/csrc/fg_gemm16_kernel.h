@@ -9,8 +9,9 @@
 // as the reference's node values are, the bias-add node and the activation
 // node are each rounded to the storage type.
 //
-// Design of gemm16_mfma, the kernel for any shape (gfx950; the pipelined
-// kernel for whole tiles, gemm16_pipe, is described at its definition):
+// Design of gemm16_mfma, for products of under 8 rows or columns and small
+// ones of short K (gfx950; the pipelined kernel for everything else,
+// gemm16_pipe, is described at its definition):
 //  * Each MFMA consumes, per lane, 8 consecutive k of one row of A and of
 //    one column of B (16 bytes each).  Both operands are therefore kept in
 //    LDS k-contiguous, [row][k] with a row stride of BK+8 elements (16-byte
@@ -660,10 +661,11 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm16_mfma(Args p) {
 //    4e + q reads the 4 elements at (k0 + e, r0 + 4q .. + 3) and output lane
 //    l receives (k0 + 0..3, r0 + l) -- the layout measured on gfx950 with an
 //    in-bounds probe; the swizzle keeps the group's 4 k-rows on distinct banks.
-// Used when K % BK == 0, leading dimensions are multiples of 8 with 16-byte
-// aligned bases, and each row-contiguous operand's row length is a multiple
-// of 8 (edge chunks are clamped to the last valid one; they reach only
-// masked outputs).
+// Used from 8 rows and columns on.  Without a tail (KT) K % BK == 0, leading
+// dimensions are multiples of 8 with 16-byte aligned bases, and each
+// row-contiguous operand's row length is a multiple of 8 (edge chunks are
+// clamped to the last valid one; they reach only masked outputs); the tail's
+// staged tiles take any K and rows.
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 
 template <int BK>

@@ -12,12 +12,12 @@
 //  * 4 or 8 waves per workgroup; each wave owns a (TM*32)x(TN*32) block of
 //    C held in TM*TN 16-register MFMA accumulators (up to 256 registers,
 //    which the compiler places in AGPRs).
-//  * K is consumed in BK-deep tiles (16 or 32) staged through LDS.  Where
-//    whole K tiles and 16-byte alignment allow, gemm_f32_pipe runs a
-//    software pipeline over them (loads two tiles ahead, fragments
-//    double-buffered in registers, a fixed MFMA / LDS-read / load order,
-//    swizzled unpadded layout); otherwise gemm_f32_mfma stages them through
-//    registers into double-buffered LDS (the loads of tile t+1 in flight
+//  * K is consumed in BK-deep tiles (16 or 32) staged through LDS.  From 4
+//    rows and columns on gemm_f32_pipe runs a software pipeline over them
+//    (loads two or four tiles ahead, fragments double-buffered in registers,
+//    a fixed MFMA / LDS-read / load order, swizzled unpadded layout), for any
+//    K and alignment; thinner products, and prologues on other than whole
+//    aligned tiles, take gemm_f32_mfma, which stages them through registers into double-buffered LDS (the loads of tile t+1 in flight
 //    during the MFMAs of tile t).  One barrier per tile either way.
 //  * No operand is transposed on its way to LDS.  A k-contiguous operand is
 //    kept [row][k] (row stride BK+4 floats, conflict-free 16-byte reads) and
@@ -709,9 +709,9 @@ __device__ __forceinline__ void gemm_f32_mfma_body(GemmArgs p, int bx, int by) {
 }
 
 // ------------------------------------------------ pipelined variant
-// The same GEMM, software-pipelined over whole K tiles: used when every
-// 16-byte chunk of a tile is either in bounds or belongs only to outputs that
-// are masked (K % BK == 0 and the VEC alignment conditions).  Rows (or
+// The same GEMM, software-pipelined over whole K tiles (KT: and a last
+// partial one, and rows of any alignment).  Every 16-byte chunk of a tile is
+// either in bounds or belongs only to outputs that are masked.  Rows (or
 // columns) past the matrix edge are clamped to the last valid one, so every
 // load reads mapped memory; the values they bring only reach masked outputs.
 // Each wave loads its share of a tile as 16 bytes per lane; lane l's chunk of
@@ -1299,48 +1299,55 @@ void launch_one(const GemmArgs &a0, hipStream_t st) {
         <<<dim3(a.tiles_m * a.tiles_n, splits), 64 * WGM * WGN, 0, st>>>(a);
 }
 
-// Tile configurations (index: BM x BN, waves, K depth):
-//   0: 256x256, 4 waves, BK 16      1: 256x128, 4 waves, BK 16
-//   2: 128x256, 4 waves, BK 16      3: 128x128, 4 waves, BK 32
-//   4:  64x64,  4 waves, BK 16      5: 128x64,  4 waves, BK 32
-//   6: 256x256, 8 waves, BK 32      7: 256x128, 8 waves, BK 32
-// 64x64 is also the only scalar-load variant, for unaligned operands.
-constexpr int kNumCfgs = 8;
+// Tile configurations (BM x BN, waves, K depth).  Dropped once the choice was
+// by how the tiles fill the CUs, as no shape ran fastest on them: 256x256 with
+// 4 waves, 128x256, and outside TN 256x128 with 4 waves.
+enum : int {
+    kCfg256x128w4 = 0,  // 4 waves, BK 16 (TN)
+    kCfg128 = 1,        // 128x128, 4 waves, BK 32
+    kCfg64 = 2,         // 64x64, 4 waves, BK 16; also the element-load tile
+    kCfg128x64 = 3,     // 4 waves, BK 32
+    kCfg256 = 4,        // 256x256, 8 waves, BK 32 (whole aligned tiles only)
+    kCfg256x128 = 5,    // 8 waves, BK 32
+    kNumCfgs = 6
+};
 
 // K depth of a configuration.
-inline int cfg_bk(int cfg) { return (cfg == 3 || cfg >= 5) ? 32 : (cfg == 4 ? 16 : kBK); }
+inline int cfg_bk(int cfg) { return cfg == kCfg256x128w4 ? kBK : cfg == kCfg64 ? 16 : 32; }
 
-// Output tile of a configuration (the element-load variant is 64x64).
-inline void cfg_tile(int cfg, bool vec, int &bm, int &bn) {
-    static const int kBm[kNumCfgs] = {256, 256, 128, 128, 64, 128, 256, 256};
-    static const int kBn[kNumCfgs] = {256, 128, 256, 128, 64, 64, 256, 128};
-    bm = vec ? kBm[cfg] : 64;
-    bn = vec ? kBn[cfg] : 64;
+// Output tile of a configuration.
+inline void cfg_tile(int cfg, int &bm, int &bn) {
+    static const int kBm[kNumCfgs] = {256, 128, 64, 128, 256, 256};
+    static const int kBn[kNumCfgs] = {128, 128, 64, 64, 256, 128};
+    bm = kBm[cfg];
+    bn = kBn[cfg];
 }
 
 // Configuration used with a prologue: the 256x256 tiles load directly into
 // LDS, which leaves no point to scale a tile at, so they give way to the
 // 256x128 tile with the same waves.
-inline int pro_cfg(int cfg) { return cfg == 0 ? 1 : cfg == 6 ? 7 : cfg; }
+inline int pro_cfg(int cfg) { return cfg == kCfg256 ? kCfg256x128 : cfg; }
 
-// pipe: the VEC conditions hold (the host checks): the pipelined kernel with
-// the same tile shape, over whole K tiles, or (ktail, no prologue) with a
-// zero-filled last tile.  With PRO != 0 or ktail the host has mapped cfg
-// through pro_cfg (staged tiles).
+// pipe: the pipelined kernel, over whole K tiles of aligned rows, or (ktail,
+// no prologue, not kCfg256) of any K and rows; always vec.  Without it
+// gemm_f32_mfma: with a prologue and 16-byte loads (vec) any tile, else 64x64.
+// With PRO != 0 the host has mapped cfg through pro_cfg (staged tiles).
 template <bool AK, bool BNC, int PRO>
 void launch_layout(const GemmArgs &a, bool vec, bool pipe, bool ktail, int cfg, hipStream_t st) {
+    constexpr bool kTN = !AK && BNC;
     if (!vec) {
         launch_one<64, 64, 2, 2, 16, AK, BNC, false, PRO>(a, st);
         return;
     }
     if constexpr (PRO == kProNone) {
-        if (pipe && ktail) {
+        if (ktail) {
             switch (cfg) {
-                case 1: launch_pipe<256, 128, 2, 2, kBK, AK, BNC, PRO, true>(a, st); break;
-                case 2: launch_pipe<128, 256, 2, 2, kBK, AK, BNC, PRO, true>(a, st); break;
-                case 3: launch_pipe<128, 128, 2, 2, 32, AK, BNC, PRO, true>(a, st); break;
-                case 5: launch_pipe<128, 64, 2, 2, 32, AK, BNC, PRO, true>(a, st); break;
-                case 7: launch_pipe<256, 128, 4, 2, 32, AK, BNC, PRO, true>(a, st); break;
+                case kCfg256x128w4:
+                    if constexpr (kTN) launch_pipe<256, 128, 2, 2, kBK, AK, BNC, PRO, true>(a, st);
+                    break;
+                case kCfg128: launch_pipe<128, 128, 2, 2, 32, AK, BNC, PRO, true>(a, st); break;
+                case kCfg128x64: launch_pipe<128, 64, 2, 2, 32, AK, BNC, PRO, true>(a, st); break;
+                case kCfg256x128: launch_pipe<256, 128, 4, 2, 32, AK, BNC, PRO, true>(a, st); break;
                 default: launch_pipe<64, 64, 2, 2, 16, AK, BNC, PRO, true>(a, st); break;
             }
             return;
@@ -1348,34 +1355,31 @@ void launch_layout(const GemmArgs &a, bool vec, bool pipe, bool ktail, int cfg, 
     }
     if (pipe) {
         switch (cfg) {
-            case 0:
-                if constexpr (PRO == kProNone) launch_pipe<256, 256, 2, 2, kBK, AK, BNC, PRO>(a, st);
+            case kCfg256x128w4:
+                if constexpr (kTN) launch_pipe<256, 128, 2, 2, kBK, AK, BNC, PRO>(a, st);
                 break;
-            case 1: launch_pipe<256, 128, 2, 2, kBK, AK, BNC, PRO>(a, st); break;
-            case 2: launch_pipe<128, 256, 2, 2, kBK, AK, BNC, PRO>(a, st); break;
-            case 3: launch_pipe<128, 128, 2, 2, 32, AK, BNC, PRO>(a, st); break;
-            case 5: launch_pipe<128, 64, 2, 2, 32, AK, BNC, PRO>(a, st); break;
-            case 6:
+            case kCfg128: launch_pipe<128, 128, 2, 2, 32, AK, BNC, PRO>(a, st); break;
+            case kCfg128x64: launch_pipe<128, 64, 2, 2, 32, AK, BNC, PRO>(a, st); break;
+            case kCfg256:
                 if constexpr (PRO == kProNone) launch_pipe<256, 256, 2, 4, 32, AK, BNC, PRO>(a, st);
                 break;
-            case 7: launch_pipe<256, 128, 4, 2, 32, AK, BNC, PRO>(a, st); break;
+            case kCfg256x128: launch_pipe<256, 128, 4, 2, 32, AK, BNC, PRO>(a, st); break;
             default: launch_pipe<64, 64, 2, 2, 16, AK, BNC, PRO>(a, st); break;
         }
         return;
     }
-    switch (cfg) {
-        case 0:
-            if constexpr (PRO == kProNone) launch_one<256, 256, 2, 2, kBK, AK, BNC, true, PRO>(a, st);
-            break;
-        case 1: launch_one<256, 128, 2, 2, kBK, AK, BNC, true, PRO>(a, st); break;
-        case 2: launch_one<128, 256, 2, 2, kBK, AK, BNC, true, PRO>(a, st); break;
-        case 3: launch_one<128, 128, 2, 2, 32, AK, BNC, true, PRO>(a, st); break;
-        case 5: launch_one<128, 64, 2, 2, 32, AK, BNC, true, PRO>(a, st); break;
-        case 6:
-            if constexpr (PRO == kProNone) launch_one<256, 256, 2, 4, 32, AK, BNC, true, PRO>(a, st);
-            break;
-        case 7: launch_one<256, 128, 4, 2, 32, AK, BNC, true, PRO>(a, st); break;
-        default: launch_one<64, 64, 2, 2, 16, AK, BNC, true, PRO>(a, st); break;
+    if constexpr (PRO != kProNone) {
+        switch (cfg) {
+            case kCfg256x128w4:
+                if constexpr (kTN) launch_one<256, 128, 2, 2, kBK, AK, BNC, true, PRO>(a, st);
+                break;
+            case kCfg128: launch_one<128, 128, 2, 2, 32, AK, BNC, true, PRO>(a, st); break;
+            case kCfg128x64: launch_one<128, 64, 2, 2, 32, AK, BNC, true, PRO>(a, st); break;
+            case kCfg256x128: launch_one<256, 128, 4, 2, 32, AK, BNC, true, PRO>(a, st); break;
+            default: launch_one<64, 64, 2, 2, 16, AK, BNC, true, PRO>(a, st); break;
+        }
+    } else {
+        launch_one<64, 64, 2, 2, 16, AK, BNC, true, PRO>(a, st);
     }
 }
 

@@ -40,17 +40,26 @@ int tiles(int M, int N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn 
 // The candidates' order settles ties: the larger tiles first, which read
 // less from the L2s.
 struct Choice {
-    int cfg = 4, splits = 1, ks = 0;
+    int cfg = fg::gemm::kCfg64, splits = 1, ks = 0;
     float us = 0.0f;
 };
 struct Rate {
     int cfg;
     float us;
 };
+using fg::gemm::kCfg128;
+using fg::gemm::kCfg128x64;
+using fg::gemm::kCfg256;
+using fg::gemm::kCfg256x128;
+using fg::gemm::kCfg256x128w4;
+using fg::gemm::kCfg64;
 constexpr Rate kRates[3][5] = {
-    {{7, 0.0146f}, {6, 0.0145f}, {3, 0.0150f}, {5, 0.0153f}, {4, 0.0159f}},   // NN
-    {{7, 0.0146f}, {6, 0.0145f}, {3, 0.0150f}, {5, 0.0155f}, {4, 0.0159f}},   // NT
-    {{6, 0.0145f}, {1, 0.0152f}, {3, 0.0153f}, {5, 0.0150f}, {4, 0.0157f}}};  // TN
+    {{kCfg256x128, 0.0146f}, {kCfg256, 0.0145f}, {kCfg128, 0.0150f},
+     {kCfg128x64, 0.0153f}, {kCfg64, 0.0159f}},  // NN
+    {{kCfg256x128, 0.0146f}, {kCfg256, 0.0145f}, {kCfg128, 0.0150f},
+     {kCfg128x64, 0.0155f}, {kCfg64, 0.0159f}},  // NT
+    {{kCfg256, 0.0145f}, {kCfg256x128w4, 0.0152f}, {kCfg128, 0.0153f},
+     {kCfg128x64, 0.0150f}, {kCfg64, 0.0157f}}};  // TN
 // The summing launch: its own time, and the rate at which it and the GEMM
 // move the slots.
 constexpr float kSumUs = 2.0f, kSumBytesPerUs = 4.0e6f;
@@ -63,10 +72,10 @@ Choice choose(int layout, int M, int N, int K, int cus, bool aligned, bool colsu
     best.us = 1e30f;
     for (const Rate &r : kRates[layout]) {
         int bm, bn;
-        fg::gemm::cfg_tile(r.cfg, true, bm, bn);
+        fg::gemm::cfg_tile(r.cfg, bm, bn);
         const int bk = fg::gemm::cfg_bk(r.cfg);
         if (one_cfg >= 0 && r.cfg != one_cfg) continue;
-        if (r.cfg == 6 && (!aligned || K % bk != 0 || (layout != FG_TN && K < 4096))) continue;
+        if (r.cfg == kCfg256 && (!aligned || K % bk != 0 || (layout != FG_TN && K < 4096))) continue;
         const int64_t t = tiles(M, N, bm, bn);
         const float unit = r.us * (bm / 64) * (bn / 64);
         for (int s = 1; s <= 16; ++s) {
@@ -158,8 +167,9 @@ void set_choice(const fg_ctx *ctx, GemmArgs &a, const Choice &ch) {
 
 // The kernel choices of one GEMM call (sets a.vec_out, and a.partial /
 // a.ksplit when K is split): the skinny kernel (skinny; then nothing else
-// applies), 16-byte operand loads (vec), the pipelined kernel (pipe) and
-// whether its last K tile is partial (ktail), the tile configuration and the
+// applies), the few-row kernel (rows; then only the splits), 16-byte operand
+// loads (vec), the pipelined kernel (pipe), whether its rows are whole 16-byte
+// chunks (aligned) and whether it takes any K and rows (ktail), the tile configuration and the
 // number of K slices.  pro: the prologue code (fg::gemm::kPro*), whose
 // tensor Pz must meet the same 16-byte conditions as the operand it scales.
 void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &rows, bool &vec,
@@ -208,10 +218,10 @@ void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &rows, b
     aligned = vec;
     if (chunks && pro == fg::gemm::kProNone) vec = true;
     Choice ch;
-    if (vec) {
+    if (chunks ? vec : vec && pro != fg::gemm::kProNone) {
         ch = choose(layout, a.M, a.N, a.K, cus, aligned, a.colsum != nullptr, ctx->ws_bytes);
     } else {  // the element-load kernel's tile
-        ch = choose(layout, a.M, a.N, a.K, cus, true, a.colsum != nullptr, ctx->ws_bytes, 4);
+        ch = choose(layout, a.M, a.N, a.K, cus, true, a.colsum != nullptr, ctx->ws_bytes, kCfg64);
     }
     if (pro != fg::gemm::kProNone) ch.cfg = fg::gemm::pro_cfg(ch.cfg);
     set_choice(ctx, a, ch);
@@ -317,11 +327,11 @@ int gemm_common(fg_ctx *ctx, int layout, GemmArgs &a, const char *who,
 int pair_kind(const Planned &P) {
     if (P.empty || P.rows || P.pro != fg::gemm::kProNone) return -1;
     if (P.skinny) return fg::gemm::kPairSkinny;
-    if (P.pipe && P.cfg == 4) return P.ktail ? fg::gemm::kPairTail : fg::gemm::kPairPipe;
+    if (P.pipe && P.cfg == kCfg64) return P.ktail ? fg::gemm::kPairTail : fg::gemm::kPairPipe;
     if (P.pipe && !P.ktail && P.splits == 1 &&
-        ((P.layout == FG_TN && P.cfg == 6) || (P.layout == FG_NT && P.cfg == 7)))
+        ((P.layout == FG_TN && P.cfg == kCfg256) || (P.layout == FG_NT && P.cfg == kCfg256x128)))
         return fg::gemm::kPairBig;
-    if (P.pipe && P.cfg == 5) return P.ktail ? fg::gemm::kPairMidTail : fg::gemm::kPairMid;
+    if (P.pipe && P.cfg == kCfg128x64) return P.ktail ? fg::gemm::kPairMidTail : fg::gemm::kPairMid;
     return -1;
 }
 
@@ -593,7 +603,7 @@ void join(const fg_ctx *ctx, Planned &P1, Planned &P2) {
     if (tiles(P1.a.M, P1.a.N, 64, 64) < cus || tiles(P2.a.M, P2.a.N, 64, 64) < cus) return;
     auto cost = [&](const Planned &P, int cfg, float &granule) {
         int bm, bn;
-        fg::gemm::cfg_tile(cfg, true, bm, bn);
+        fg::gemm::cfg_tile(cfg, bm, bn);
         float r = 0.0f;
         for (const Rate &q : kRates[P.layout])
             if (q.cfg == cfg) r = q.us;
@@ -608,7 +618,7 @@ void join(const fg_ctx *ctx, Planned &P1, Planned &P2) {
     const float apart = alone(P1) + alone(P2) + kSumUs;
     int best = -1;
     float us = apart;
-    for (int cfg : {5, 4}) {
+    for (int cfg : {kCfg128x64, kCfg64}) {
         float g1, g2;
         // (On average half of the larger tile's time is left at the end.)
         const float t = cost(P1, cfg, g1) + cost(P2, cfg, g2);

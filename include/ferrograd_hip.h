@@ -76,8 +76,9 @@ int fg_ctx_stream(fg_ctx *ctx, void **stream);
 /* Pre-size the context's scratch workspace so later direct-kernel calls
  * (and graph capture) never allocate.  A GEMM of few output tiles and a long
  * K splits K into this workspace when it already holds the slices (fp32 or
- * fp32 sums of a 16-bit GEMM, M x N floats per slice); it is never grown for
- * that, so a larger workspace can change which GEMMs split. */
+ * fp32 sums of a 16-bit GEMM, M x N floats per slice, and N more with the
+ * fused column sums); it is never grown for that, so a larger workspace can
+ * change which GEMMs split. */
 int fg_ctx_reserve_workspace(fg_ctx *ctx, uint64_t bytes);
 /* GpuBackend::sync / is_ready (rocm/mod.rs:398-400). */
 int fg_sync(fg_ctx *ctx);
@@ -223,10 +224,9 @@ int fg_gemm_dw_f32(fg_ctx *ctx, int M, int N, int K, const float *d_A, int lda,
  * operand, colsum included): C as fg_gemm_x16 in the TN layout; colsum[n]
  * (=|+=) sum_k B[k][n] summed in fp32 and rounded to dtype once (with
  * colsum_accumulate: round(colsum + sum)). Shapes off the pipelined
- * path (K not a multiple of the tile depth, unaligned rows) take the GEMM
- * plus fg_bias_grad's reduction: the same values up to the order of the
- * fp32 sums. Replaces the 16-bit dB lowering (matmul/mod.rs:85-94) and the
- * bias add's backward, which the reference lacks (binary.rs:53-63). */
+ * path (M or N under 8) take the GEMM plus fg_bias_grad's reduction: the
+ * same values up to the order of the fp32 sums. Replaces the 16-bit dB
+ * lowering (matmul/mod.rs:85-94) and the bias add's backward, which the reference lacks (binary.rs:53-63). */
 int fg_gemm_dw_x16(fg_ctx *ctx, int dtype, int M, int N, int K, const void *d_A, int lda,
                    const void *d_B, int ldb, void *d_C, int ldc, int accumulate,
                    void *d_colsum, int colsum_accumulate);
