@@ -91,7 +91,7 @@ struct Args {
     // workgroups of the first tile row, rounded to the storage type once.
     uint16_t *colsum;
     int colsum_accumulate;
-    // K split (pipelined kernel only, never with colsum): workgroup row s
+    // K split (pipelined and few-row kernels): workgroup row s
     // (blockIdx.y) multiplies K elements [s * ksplit, (s + 1) * ksplit) and
     // writes its fp32 sums, without epilogue, into the M x N slot s of
     // partial (row length N); sum_slices16 then adds the slots in slot order
