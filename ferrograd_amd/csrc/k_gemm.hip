@@ -289,10 +289,22 @@ void launch_reduce(fg_ctx *ctx, const GemmArgs &a, int splits) {
     splitk_reduce<<<fg::reduce_blocks(ctx, a.M, a.N), kThreads, 0, ctx->stream>>>(a, splits);
 }
 
+// Before slices go to the workspace: a summing launch held over the ones there
+// now (of an earlier GEMM of the same launch group) goes out first, and the hold
+// passes to the sum of the new ones.
+int claim_slices(fg_ctx *ctx) {
+    if (ctx->pending_splits <= 0) return FG_OK;
+    const int rc = fg::launch_pending_reduce(ctx);
+    if (rc == FG_OK) ctx->defer_reduce = true;
+    return rc;
+}
+
 // reduce: launch the summing kernel of a split GEMM (false: its consumer
 // sums the slices).
 int gemm_launch(fg_ctx *ctx, const Planned &P, const char *who, bool reduce = true) {
     if (P.empty) return FG_OK;
+    if (P.splits > 1)
+        if (const int rc = claim_slices(ctx)) return rc;
     if (P.skinny) {
         fg::gemm::launch_skinny(P.a, P.layout, ctx->stream);
         FG_LAUNCH_CHECK(who);
@@ -718,6 +730,8 @@ int gemm_dw_dx_f32(fg_ctx *ctx, int M1, int N1, int K1, const float *A1, int lda
     if (!plan_pair(ctx, dw_args(M1, N1, K1, A1, lda1, B1, ldb1, C1, ldc1, acc1, colsum, colsum_acc),
                    dx_args(M2, N2, K2, A2, lda2, B2, ldb2, act, Zs, ldzs, C2, ldc2, acc2), P1, P2))
         return separate();
+    if (P1.splits > 1 || P2.splits > 1)
+        if (const int rc = claim_slices(ctx)) return rc;
     int x1, n1, x2, n2;
     pair_grid(P1, x1, n1);
     pair_grid(P2, x2, n2);
@@ -825,6 +839,8 @@ int gemm_dw_dw_dx_f32(fg_ctx *ctx, int M0, int N0, int K0, const float *A0, int 
         fg::clear_error();
         return separate();
     }
+    if (P1.splits > 1 || P2.splits > 1)
+        if (const int rc = claim_slices(ctx)) return rc;
     int x0, n0, x1, n1, x2, n2;
     pair_grid(P0, x0, n0);
     pair_grid(P1, x1, n1);

@@ -861,6 +861,24 @@ def test_captured_sgd_fused_paths_at_other_shapes(ctx, dims, B, act):
             st.plan.close()
 
 
+@pytest.mark.parametrize("dims,B", [([64, 512, 10], 512), ([32, 1024, 10], 1024),
+                                    ([128, 512, 3], 512)],
+                         ids=["64-512-10-b512", "32-1024-10-b1024", "128-512-3-b512"])
+def test_captured_sgd_both_first_layer_gradients_split(ctx, dims, B):
+    """The first layer's dW (with the bias gradient) and dX both split K, one
+    after the other, in the backward's last launch group: the slices of the
+    second take the workspace that held the first's, whose sum must be out by
+    then.  Captured steps against eager ones bit for bit, and the oracle."""
+    G = api()
+    _, _, _, st = build_mlp(ctx, dims, B, "relu", G.Optim.sgd())
+    desc = st.plan.describe()
+    st.plan.close()
+    last = desc.split("backward(ce-fused)")[1].split("optim:")[0].strip().splitlines()[-2:]
+    assert all("[K split: slices + summing kernel]" in l for l in last), desc
+    assert "the backward's last summing launch shares the SGD launch" in desc, desc
+    test_captured_sgd_fused_paths_at_other_shapes(ctx, dims, B, "relu")
+
+
 @pytest.mark.parametrize("act", ["relu", "gelu"])
 @pytest.mark.parametrize("seeded", [True, False], ids=["seed", "mse"])
 def test_linear_root_activation_backward(ctx, act, seeded):
