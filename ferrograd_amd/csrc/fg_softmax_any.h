@@ -162,6 +162,77 @@ __device__ __forceinline__ float sum_over(float v, float *sm) {
     return v;
 }
 
+// The sum over a wave's row of per-lane sums part[i] (those of the lane's i-th
+// chunk): each of the NV added over the lanes, then the NV in order, as NV waves
+// of one chunk a thread add them -- chains of a chunk, the six steps and NV, not of
+// a lane's whole share of the row.  With NV > 1 the first steps halve the values a
+// lane carries (lanes of bit 32, then 16, keep the upper ones).
+template <int NV>
+__device__ __forceinline__ float sum_chunks(const float (&part)[NV]) {
+    static_assert(NV == 1 || NV == 2 || NV == 4, "one-wave rows");
+    const int lane = threadIdx.x & 63;
+    float v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = part[i];
+    int o = 32;
+#pragma unroll
+    for (int n = NV / 2; n > 0; n /= 2, o >>= 1) {
+        const bool up = (lane & o) != 0;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const float keep = up ? v[i + n] : v[i], give = up ? v[i] : v[i + n];
+            v[i] = keep + __shfl_xor(give, o);
+        }
+    }
+#pragma unroll
+    for (; o > 0; o >>= 1) v[0] += __shfl_xor(v[0], o);
+    if constexpr (NV == 1) return v[0];
+    auto of = [&](int i) {  // the i-th chunks' sum
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[0]), i * (64 / NV)));
+    };
+    float s = of(0);
+#pragma unroll
+    for (int i = 1; i < NV; ++i) s += of(i);
+    return s;
+}
+
+// A row's sum over the NV chunks a thread of NW waves holds, added an element at a
+// time: a sum per chunk (in two halves where a chunk has eight elements), on one
+// wave, which holds a larger share of the row a lane, added by sum_chunks, else by
+// the thread.  fp32 on four waves: one running sum a thread.  In fp32 rows of up
+// to 8192 columns on 16-byte boundaries are so added in the order of one float4 a
+// thread on four waves.
+template <int DT, int NV, int NW>
+struct RowSum {
+    static constexpr bool kEach = NW == 1, kRunning = DT == kF32 && NW == 4;
+    float s[kEach ? NV : 1], lo = 0.0f, hi = 0.0f;
+    __device__ __forceinline__ explicit RowSum(float first) {
+#pragma unroll
+        for (int i = 1; i < (kEach ? NV : 1); ++i) s[i] = 0.0f;
+        s[0] = first;
+    }
+    __device__ __forceinline__ void add(int i, int e, float v) {
+        if constexpr (kRunning || (kEach && DT == kF32)) {
+            s[kEach ? i : 0] += v;
+        } else {
+            if (e % 4 == 0) (e ? hi : lo) = v;
+            else (e > 4 ? hi : lo) += v;
+            if (e == Io<DT>::E - 1) s[kEach ? i : 0] += Io<DT>::E > 4 ? lo + hi : lo;
+        }
+    }
+    __device__ __forceinline__ float over(float *sm) {
+        if constexpr (kEach) return sum_chunks<NV>(s);
+        else return sum_over<NW>(s[0], sm);
+    }
+};
+
+// What a label's column gets: the probability rounded, then less one.
+__device__ __forceinline__ float label_grad(float scale, float e, float inv) {
+#pragma clang fp contract(off)
+    const float p = e * inv;
+    return scale * (p - 1.0f);
+}
+
 // Threads of a workgroup whose rows take NW waves each (one wave a row:
 // four rows a workgroup).
 constexpr int threads_of(int NW) { return NW == 1 ? 256 : NW * 64; }
@@ -232,21 +303,21 @@ void softmax_any(const typename Io<DT>::T *x, int ldx,
     if constexpr (!kHold) repack(w);
     float ex[kHold ? NV * E : 1];
     vs = sp.single(t) >= 0 ? exp_below<DT>(vs, m) : 0.0f;
-    float s = vs;
+    RowSum<DT, NV, NW> sum(vs);
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const float p = exp_below<DT>(IO::get(w[i], e), m);
             if constexpr (kHold) ex[i * E + e] = p;
-            s += p;
+            sum.add(i, e, p);
         }
     // The label's logit, in the thread that writes its column and before any
     // thread stores (out may be x).
     const bool mine = tc >= 0 && t == sp.owner(tc, NT);
     float xt = 0.0f;
     if (mine) xt = IO::load1(xr, tc);
-    s = sum_over<NW>(s, ssum);
+    const float s = sum.over(ssum);
     if (t == 0) {
         if (NW > 1 && argmax) argmax[r] = (uint32_t)sarg;
         // A label outside [0, C) has no logit; report NaN rather than read.
@@ -274,7 +345,7 @@ void softmax_any(const typename Io<DT>::T *x, int ldx,
         auto *orow = out + (size_t)r * ldo;
         write(orow, scale);
         // Then, over it, the label's column.
-        if (mine) IO::store1(orow, tc, scale * (exp_below<DT>(xt, m) * inv - 1.0f));
+        if (mine) IO::store1(orow, tc, label_grad(scale, exp_below<DT>(xt, m), inv));
     }
     if (probs) write(probs + (size_t)r * ldp, 1.0f);
 }
@@ -322,10 +393,12 @@ __global__ __launch_bounds__(kLongNW * 64) void softmax_long(
         }
         // Nothing above -inf yet: only a NaN counts.
         const float base = m == -INFINITY ? 0.0f : m;
+        float step = 0.0f;
 #pragma unroll
         for (int i = 0; i < kStep; ++i)
 #pragma unroll
-            for (int e = 0; e < E; ++e) s += exp_below<DT>(IO::get(w[i], e), base);
+            for (int e = 0; e < E; ++e) step += exp_below<DT>(IO::get(w[i], e), base);
+        s += step;
     }
     const float lm = fmaxf(m, vs);
     const float mr = max_over<kLongNW>(lm, smax);
@@ -387,7 +460,7 @@ __global__ __launch_bounds__(kLongNW * 64) void softmax_long(
                                             reinterpret_cast<u32x4 *>(prow + sp.head) + j);
         }
     }
-    if (out && mine) IO::store1(orow, tc, scale * (exp_below<DT>(xt, mr) * inv - 1.0f));
+    if (out && mine) IO::store1(orow, tc, label_grad(scale, exp_below<DT>(xt, mr), inv));
 }
 
 // dx (=|+=) y * (dy - sum(dy * y)), y and dy held in registers.
@@ -415,12 +488,12 @@ __global__ __launch_bounds__(threads_of(NW)) void softmax_bwd_any(
     const int cs = sp.single(t);
     const float ys = cs >= 0 ? IO::load1(y + base, cs) : 0.0f;
     const float ds = cs >= 0 ? IO::load1(dy + base, cs) : 0.0f;
-    float dot = ds * ys;
+    RowSum<DT, NV, NW> sum(ds * ys);
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (int e = 0; e < E; ++e) dot += IO::get(wd[i], e) * IO::get(wy[i], e);
-    dot = sum_over<NW>(dot, ssum);
+        for (int e = 0; e < E; ++e) sum.add(i, e, IO::get(wd[i], e) * IO::get(wy[i], e));
+    const float dot = sum.over(ssum);
     if constexpr (DT != kF32) {
         repack(wy);
         repack(wd);
@@ -467,8 +540,10 @@ __global__ __launch_bounds__(kLongNW * 64) void softmax_bwd_long(
 #pragma unroll 2
     for (int j = t; j < sp.nb; j += NT) {
         const u32x4 wy = yb[j], wd = db[j];
+        float chunk = 0.0f;
 #pragma unroll
-        for (int e = 0; e < E; ++e) dot += IO::get(wd, e) * IO::get(wy, e);
+        for (int e = 0; e < E; ++e) chunk += IO::get(wd, e) * IO::get(wy, e);
+        dot += chunk;
     }
     dot = sum_over<kLongNW>(dot, ssum);
     auto *xr = dx + base;

@@ -1159,3 +1159,28 @@ def test_device_rng_matches_host(gpu_ctx):
     hx = fa.rng_normal(9, 6, (n,))
     assert np.mean(host(x) == hx) > 0.999
     assert np.max(np.abs(host(x) - hx)) < 1e-5
+
+
+def test_softmax_row_sum_order(gpu_ctx):
+    """A one-wave row's sum (fp32, 1024 columns) adds its chunks' sums, not one
+    long chain a lane: with 256 columns at the maximum and the rest 15.5 below
+    it (1.9e-7 each, under half a unit of a lane's first four), a chain loses
+    all of the rest.  Chunk sums and the six steps are exact but for units of
+    the small ones; the three sums added to the first, 1 / s and the product
+    round by half a unit each.  And the label's gradient is the rounded
+    probability less one."""
+    torch = _torch()
+    R, C = 6, 1024
+    x = torch.full((R, C), -15.5)
+    x[:, :256] = 0.0
+    x[3:] += 2.0
+    y, d, loss = empty((R, C)), empty((R, C)), empty((R,))
+    lab = torch.arange(0, 32 * R, 32, dtype=torch.int32)
+    xd = x.cuda()
+    gpu_ctx.softmax(xd, R, C, y)
+    gpu_ctx.softmax_ce(xd, C, lab.cuda(), R, C, 1.0, row_loss=loss, dlogits=d, ldd=C)
+    torch.cuda.synchronize()
+    p = torch.softmax(x.double(), 1)
+    assert ((y.cpu().double() - p).abs() <= 5 * 2.0 ** -24 * p)[:, :256].all()
+    cols = lab.long()[:, None]
+    assert torch.equal(d.cpu().gather(1, cols), y.cpu().gather(1, cols) - 1.0)
