@@ -1314,7 +1314,7 @@ void launch_one(const Args &a0, hipStream_t st) {
 //   4: 3's tiles with a K tail (K % 64 != 0)
 //   5, 6: 0's and 1's with a K tail and rows of any 4-byte alignment
 //   7, 8: and rows that start on odd elements
-//   9:  64x64, 4 waves, BK 32 (gemm16_mfma), for under 8 rows or columns
+//   9:  64x64, 4 waves, BK 32 (gemm16_mfma): under 8 rows or columns, short K
 enum : int {
     kCfg256 = 0, kCfg128 = 1, kCfgBig = 2, kCfgMid = 3, kCfgMidTail = 4, kCfgAny256 = 5,
     kCfgAny128 = 6, kCfgOdd256 = 7, kCfgOdd128 = 8, kCfgSmall = 9

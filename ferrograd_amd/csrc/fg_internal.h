@@ -114,8 +114,9 @@ int noalloc_init(int device);
 // Bytes of workspace fg_bias_grad needs for an M x N reduction on a device
 // with `cus` compute units (the partial sums of its row splits).
 uint64_t bias_grad_ws_bytes(int cus, int M, int N);
-// Workspace bytes of the K slices a 16-bit GEMM of this shape takes when the
-// workspace holds them (0: no split); colsum: with the fused column sums.
+// Workspace bytes a 16-bit GEMM of this shape uses when the workspace holds
+// them (K slices, or a column-sum reduction's partial sums; 0: none); colsum:
+// with the fused column sums.
 uint64_t gemm16_split_ws_bytes(int cus, int layout, int M, int N, int K, bool colsum);
 // Dispatches of one 16-bit GEMM call (no launch; colsum: the fused bias
 // gradient of fg_gemm_dw_x16 is asked).

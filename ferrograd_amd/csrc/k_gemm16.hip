@@ -29,16 +29,19 @@ Rows rows_of(int layout, int M, int N, const void *A, int lda, const void *B, in
     return (ab & 15u) == 0 && ld % 8 == 0 && rc ? kRowsWhole : kRowsEven;
 }
 
-// Tile configuration and K slices of a pipelined call (M, N >= 8) by a model
-// of its time: a CU with n workgroups takes n tiles' time, a tile its k times
-// kRate (us per k per 64x64 of output, measured on MI355X, bf16, N(0,1)
-// operands, HIP events, 512^3 to 4096^3) and a fixed part that grows with it
-// (pipeline fill, output); slices cut the depth for a summing launch and the
-// slots' traffic.  With the fused column sums each slice also leaves N fp32
-// sums, after the output slots.  Modelled against measured (us, NN): 2048 x 1000
-// x 4096 on 128x128 tiles in two slices 33 / 33, on 256x128 in four 36 / 37; 2046
-// x 4094 x 4094 on 256x256 in two 100 / 100, unsplit 131 / 127.  The candidates'
-// order settles ties: the larger tiles first.
+// Tile configuration and K slices of a call (M, N >= 8) by a model of its time,
+// measured on MI355X (256 CUs, bf16, N(0,1) operands, HIP events, K from 1 to
+// 4096).  Pipelined tiles: a CU with n workgroups takes n tiles' time, a tile its
+// k times kRate (us per k per 64x64 of output), a fixed part that grows with it
+// (pipeline fill, output), its K tail, and more where its output has edges; slices
+// cut the depth for a summing launch and the slots' traffic.  That a CU's
+// workgroups take their tiles one after the other is how the matrix units' time
+// adds up; tiles of unaligned rows, which wait for loads, overlap more than that,
+// so their kRate is a mean over the sizes.  With the fused column sums each slice
+// also leaves N fp32 sums, after the output slots.  Modelled against measured (us,
+// NN): 2048 x 1000 x 4096 on 128x128 tiles in two slices 33 / 33, on 256x128 in
+// four 36 / 37; 2046 x 4094 x 4094 on 256x256 in two 100 / 100, unsplit 131 / 127.
+// The candidates' order settles ties: the larger tiles first.
 //
 // Rows that are not whole chunks took one element a lane before (us): 2047 x
 // 4095 x 4093 NN 975 -> 116, NT 1363 -> 121, 777 x 1333 x 2049 120 -> 27, 300^3
@@ -55,22 +58,52 @@ constexpr Rate16 kWhole[] = {{fg::gemm16::kCfgBig, 0.0017f, 0.0017f, 0.0017f},
                              {fg::gemm16::kCfg256, 0.0018f, 0.0019f, 0.0024f},
                              {fg::gemm16::kCfg128, 0.0026f, 0.0023f, 0.0032f},
                              {fg::gemm16::kCfgAny256, 0.0018f, 0.0019f, 0.0024f},
-                             {fg::gemm16::kCfgAny128, 0.0026f, 0.0023f, 0.0032f},
-                             // (not pipelined, no slices or column sums: NN and
-                             // NT with K up to 512; 256^3 7.8 / 5.9 us, on
-                             // 128x128 tiles 9.0 / 6.4)
-                             {fg::gemm16::kCfgSmall, 0.010f, 0.005f, 1.0f}};
+                             {fg::gemm16::kCfgAny128, 0.0026f, 0.0023f, 0.0032f}};
 constexpr Rate16 kEven[] = {{fg::gemm16::kCfgAny256, 0.0018f, 0.0020f, 0.0025f},
-                            {fg::gemm16::kCfgAny128, 0.0033f, 0.0036f, 0.0030f},
-                            // (one element a lane: 100 x 4000 x 100 NN 8.9 us,
-                            // on 128x128 tiles 10.5)
-                            {fg::gemm16::kCfgSmall, 0.030f, 0.022f, 1.0f}};
+                            {fg::gemm16::kCfgAny128, 0.0033f, 0.0036f, 0.0030f}};
 constexpr Rate16 kOdd[] = {{fg::gemm16::kCfgOdd256, 0.0024f, 0.0026f, 0.0030f},
-                           {fg::gemm16::kCfgOdd128, 0.0041f, 0.0047f, 0.0037f},
-                           {fg::gemm16::kCfgSmall, 0.030f, 0.022f, 1.0f}};
-constexpr float kTileUs = 1.5f, kTileUnitUs = 0.4f;       // fixed, and per 64x64
-constexpr float kTailUs = 1.0f;                           // a K tail
+                           {fg::gemm16::kCfgOdd128, 0.0041f, 0.0047f, 0.0037f}};
+constexpr float kTileUs = 1.5f, kTileUnitUs = 0.4f;  // fixed, and per 64x64
 constexpr float kSumUs16 = 2.0f, kSumBytesPerUs16 = 6.0e6f;
+
+// A pipelined tile's K tail of r elements, which is loaded one element at a time:
+// where rows are odd and k-contiguous it shows (1023 x 1021 NN, 128x128 tiles:
+// 12.2 us for K = 2, 15.8 for 32, 14.4 for 33).
+float tail_us(int layout, Rows rows, int units, int r) {
+    const float per_k = rows != kRowsOdd || layout == FG_TN ? 0.006f : 0.03f;
+    return r > 0 ? 0.5f + per_k * units * r : 0.0f;
+}
+// A pipelined tile's output where the row length is not whole groups of four
+// (written one element at a time, by rows: 1024 x 1024 x 64 NN 7.2 us, 1023 x
+// 1021 x 65 14.9) or a tile reaches past the output.
+float edge_us(int M, int N, int bm, int bn, int units) {
+    if (N % 4 != 0)
+        return (units == 4 ? 7.5f : units == 16 ? 16.0f : 8.0f) * std::min(M, bm) / bm;
+    return M % bm != 0 || N % bn != 0 ? 0.3f * units : 0.0f;
+}
+// The 64x64 tiles that are not pipelined (kCfgSmall; n a CU, several of them at
+// once), without slices; K up to 512, from where the others were faster.  The column
+// sums are a reduction of their own then.  They win where K is too short for a
+// pipeline to pay (us, against 128x128 tiles): TN 297 x 407 x 32 10 / 26, 512 x
+// 57 x 11 9.4 / 16.9, NN 1146 x 137 x 128 13.8 / 24.7, 1024 x 1024 x 64 5.3 /
+// 7.2; at K = 256 NN / TN 1024^2 8.3 / 8.8, 10.7 / 8.8.
+float small_us(int layout, int M, int N, int K, Rows rows, int64_t n, bool colsum) {
+    const bool vec = rows == kRowsWhole;
+    float one, many;  // us per k: a CU's only tile, and each of several
+    if (layout == FG_NT) {
+        one = vec ? 0.008f : 0.034f;
+        many = vec ? 0.006f : 0.034f;
+    } else if (layout == FG_NN) {
+        one = vec && N % 64 == 0 ? 0.012f : 0.036f;
+        many = vec && N % 64 == 0 ? 0.010f : 0.034f;
+    } else {
+        const bool whole = vec && M % 64 == 0 && N % 64 == 0;
+        one = whole ? 0.030f : 0.042f;
+        many = whole ? 0.012f : 0.032f;
+    }
+    return std::max(0, K - 32) * std::max(one, n * many) + 0.2f + 1.2f * n +
+           (layout == FG_TN ? (vec ? 1.0f : 2.0f) : 0.0f) + (colsum ? 5.0f : 0.0f);
+}
 
 struct Choice16 {
     int cfg = fg::gemm16::kCfgSmall, splits = 1, ks = 0;
@@ -84,6 +117,9 @@ Choice16 choose16(int layout, int M, int N, int K, int cus, Rows rows, bool cols
     const Rate16 *end = rows == kRowsWhole  ? std::end(kWhole)
                         : rows == kRowsEven ? std::end(kEven)
                                             : std::end(kOdd);
+    // A row-contiguous operand of ragged rows leaves its last row to the tail.
+    const bool ragged = rows != kRowsWhole &&
+                        ((layout == FG_TN && M % 8 != 0) || (layout != FG_NT && N % 8 != 0));
     for (; r != end; ++r) {
         // Whole K tiles, but for the tails': that of 256x128 takes k-contiguous
         // rows eight at a time.
@@ -93,30 +129,37 @@ Choice16 choose16(int layout, int M, int N, int K, int cus, Rows rows, bool cols
         } else if (r->cfg < kCfgMidTail) {
             if (K % bk != 0) continue;
         }
-        if (r->cfg == kCfgSmall && K > 512) continue;
-        const float fixed = kTileUs + (K % bk != 0 && r->cfg != kCfgSmall ? kTailUs : 0.0f);
         int bm, bn;
         cfg_tile16(r->cfg, bm, bn);
         const int64_t t = tiles(M, N, bm, bn);
         const int units = (bm / 64) * (bn / 64);
         const float rate = (layout == FG_NN ? r->nn : layout == FG_NT ? r->nt : r->tn) * units;
+        const int tail = K - (K - (ragged ? 1 : 0)) / bk * bk;
+        const float fixed = kTileUs + kTileUnitUs * units + tail_us(layout, rows, units, tail) +
+                            edge_us(M, N, bm, bn, units);
         for (int s = 1; s <= 16; ++s) {
             int ks = K;
             if (s > 1) {
                 // At least eight K tiles in all and four a slice, whole ones;
                 // slices only while the CUs have under two tiles each.
-                if (r->cfg == kCfgSmall || K < 8 * bk || s > K / (4 * bk) ||
-                    t * s > 2 * (int64_t)cus)
-                    break;
+                if (K < 8 * bk || s > K / (4 * bk) || t * s > 2 * (int64_t)cus) break;
                 ks = ((K + s - 1) / s + bk - 1) / bk * bk;
                 if ((K + ks - 1) / ks != s) continue;
                 if ((uint64_t)s * ((uint64_t)M * N + (colsum ? N : 0)) * sizeof(float) > ws_bytes)
                     break;
             }
-            float us = (float)((t * s + cus - 1) / cus) * (ks * rate + fixed + kTileUnitUs * units);
+            const int k = s > 1 ? ks : K - tail;  // (a slice has a tail only if it is the last)
+            float us = (float)((t * s + cus - 1) / cus) * (k * rate + fixed);
             if (s > 1) us += kSumUs16 + (2 * s + 1) * (float)M * N * 4.0f / kSumBytesPerUs16;
             if (us < 0.99f * best.us) best = Choice16{r->cfg, s, s > 1 ? ks : 0, us};
         }
+    }
+    // Its column sums only where the workspace holds their partial sums already:
+    // a call never grows it for a choice that it need not make.
+    if (K <= 512 && (!colsum || fg::bias_grad_ws_bytes(cus, K, N) <= ws_bytes)) {
+        const float us = small_us(layout, M, N, K, rows, (tiles(M, N, 64, 64) + cus - 1) / cus,
+                                  colsum);
+        if (us < 0.99f * best.us) best = Choice16{kCfgSmall, 1, 0, us};
     }
     return best;
 }
@@ -337,9 +380,9 @@ int gemm16_dispatches(fg_ctx *ctx, int layout, int M, int N, int K, const void *
     return q.splits > 1 ? 2 : 1;
 }
 
-// Workspace bytes a 16-bit GEMM of this shape splits K into when the
-// workspace holds them (0: it does not split), for planners that size a
-// workspace ahead.
+// Workspace bytes a 16-bit GEMM of this shape uses when the workspace holds
+// them (its K slices, or the column sums' partial sums off the pipelined kernel;
+// 0: none), for planners that size a workspace ahead.
 uint64_t gemm16_split_ws_bytes(int cus, int layout, int M, int N, int K, bool colsum) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     cus = cus > 0 ? cus : 256;
@@ -348,11 +391,14 @@ uint64_t gemm16_split_ws_bytes(int cus, int layout, int M, int N, int K, bool co
         const int sl = fg::rows::split_of(cus, 2, M, N, K, ~0ull, ks);
         return sl > 1 ? (uint64_t)sl * M * N * sizeof(float) : 0;
     }
-    if (M < 8 || N < 8) return 0;
+    // Off the pipelined kernel the column sums are a reduction of their own.
+    const uint64_t reduce = colsum ? bias_grad_ws_bytes(cus, K, N) : 0;
+    if (M < 8 || N < 8) return reduce;
     // Dense rows from aligned bases.
     const int lda = layout == FG_TN ? M : K, ldb = layout == FG_NT ? K : N;
     const Choice16 ch = choose16(layout, M, N, K, cus, rows_of(layout, M, N, nullptr, lda, nullptr, ldb),
                                  colsum, ~0ull);
+    if (ch.cfg == fg::gemm16::kCfgSmall) return reduce;
     return ch.splits > 1 ? (uint64_t)ch.splits * ((uint64_t)M * N + (colsum ? N : 0)) * sizeof(float)
                          : 0;
 }

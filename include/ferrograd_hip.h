@@ -223,9 +223,10 @@ int fg_gemm_dw_f32(fg_ctx *ctx, int M, int N, int K, const float *d_A, int lda,
 /* The same for 16-bit tensors (dtype FG_DTYPE_F16 / FG_DTYPE_BF16 for every
  * operand, colsum included): C as fg_gemm_x16 in the TN layout; colsum[n]
  * (=|+=) sum_k B[k][n] summed in fp32 and rounded to dtype once (with
- * colsum_accumulate: round(colsum + sum)). Shapes off the pipelined
- * path (M or N under 8) take the GEMM plus fg_bias_grad's reduction: the
- * same values up to the order of the fp32 sums. Replaces the 16-bit dB
+ * colsum_accumulate: round(colsum + sum)). Off the pipelined path (M or N
+ * under 8, and short K where the workspace holds the reduction's partial sums)
+ * it takes the GEMM plus fg_bias_grad's reduction: the same values up to the
+ * order of the fp32 sums. Replaces the 16-bit dB
  * lowering (matmul/mod.rs:85-94) and the bias add's backward, which the reference lacks (binary.rs:53-63). */
 int fg_gemm_dw_x16(fg_ctx *ctx, int dtype, int M, int N, int K, const void *d_A, int lda,
                    const void *d_B, int ldb, void *d_C, int ldc, int accumulate,

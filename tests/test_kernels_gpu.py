@@ -824,6 +824,59 @@ def test_gemm_x16_any_rows(gpu_ctx, dtype, layout, place):
             assert torch.equal(Z[:, :N].cpu(), z)
 
 
+@pytest.mark.parametrize("reserved", [0, 64 << 20], ids=["no-workspace", "workspace"])
+@pytest.mark.parametrize("dtype", [1, 2], ids=["f16", "bf16"])
+def test_gemm_x16_short_k(dtype, reserved):
+    """K around the lengths where the 64x64 tiles, the pipelined tiles and their
+    K tails take over from each other, each call captured on a context that holds
+    no workspace (and must not ask for one then) or enough: small-integer operands,
+    outputs and column sums bit for bit."""
+    torch = _torch()
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import ferrograd_amd as fa
+
+    dt = [None, torch.float16, torch.bfloat16][dtype]
+    g = torch.Generator().manual_seed(19)
+    before = torch.cuda.current_stream()
+    ctx, st = fa.torch_context(0)
+    try:
+        if reserved:
+            ctx.reserve_workspace(reserved)
+        for M, N in ((100, 99), (16, 1216), (512, 57), (130, 256), (300, 407)):
+            for K in (1, 2, 3, 31, 32, 33, 96, 129, 250, 512, 513):
+                for layout in (O.NN, O.NT, O.TN):
+                    if layout != O.TN and M <= 64:
+                        continue  # (few rows: another kernel)
+                    note(f"gemm_x16_short_k {dtype} {reserved} {layout} {M}x{N}x{K}")
+                    a = torch.randint(-2, 3, (K, M) if layout == O.TN else (M, K), generator=g)
+                    b = torch.randint(-2, 3, (N, K) if layout == O.NT else (K, N), generator=g)
+                    ref = ((a.T if layout == O.TN else a).double() @
+                           (b.T if layout == O.NT else b).double())
+                    A, B = a.to(dt).cuda(), b.to(dt).cuda()
+                    C = torch.zeros(M, N, dtype=dt, device="cuda")
+                    S = torch.zeros(N, dtype=dt, device="cuda")
+                    lda, ldb = A.shape[1], B.shape[1]
+                    torch.cuda.synchronize()
+                    graph = torch.cuda.CUDAGraph()
+                    with torch.cuda.graph(graph, stream=st):
+                        if layout == O.TN:
+                            ctx.gemm_dw_x16(dtype, M, N, K, A, lda, B, ldb, C, N, colsum=S)
+                        else:
+                            ctx.gemm_x16(dtype, layout, M, N, K, A, lda, B, ldb, C, N)
+                    for _ in range(2):
+                        C.zero_(), S.zero_()
+                        graph.replay()
+                        torch.cuda.synchronize()
+                        assert torch.equal(C.cpu(), ref.to(dt))
+                        if layout == O.TN:
+                            assert torch.equal(S.cpu(), b.double().sum(0).to(dt))
+    finally:
+        torch.cuda.set_stream(before)
+        ctx.sync()
+        ctx.close()
+
+
 @pytest.mark.parametrize("dtype", [0, 1, 2], ids=["f32", "f16", "bf16"])
 @pytest.mark.parametrize("pad", [0, 1, 2])
 def test_bias_grad_any_rows(gpu_ctx, dtype, pad):
