@@ -73,9 +73,10 @@ float tail_us(int layout, Rows rows, int units, int r) {
     const float per_k = rows != kRowsOdd || layout == FG_TN ? 0.006f : 0.03f;
     return r > 0 ? 0.5f + per_k * units * r : 0.0f;
 }
-// A pipelined tile's output where the row length is not whole groups of four
-// (written one element at a time, by rows: 1024 x 1024 x 64 NN 7.2 us, 1023 x
-// 1021 x 65 14.9) or a tile reaches past the output.
+// What the last of a launch's tiles take longer where the row length is not whole
+// groups of four (written one element at a time, by rows: 1024 x 1024 x 64 NN 7.2
+// us, 1023 x 1021 x 65 14.9) or a tile reaches past the output.  A slice's fp32
+// sums have no such edges, the summing launch's are spread over all CUs.
 float edge_us(int M, int N, int bm, int bn, int units) {
     if (N % 4 != 0)
         return (units == 4 ? 7.5f : units == 16 ? 16.0f : 8.0f) * std::min(M, bm) / bm;
@@ -89,6 +90,7 @@ float edge_us(int M, int N, int bm, int bn, int units) {
 // 7.2; at K = 256 NN / TN 1024^2 8.3 / 8.8, 10.7 / 8.8.
 float small_us(int layout, int M, int N, int K, Rows rows, int64_t n, bool colsum) {
     const bool vec = rows == kRowsWhole;
+    const bool whole = vec && M % 64 == 0 && N % 64 == 0;
     float one, many;  // us per k: a CU's only tile, and each of several
     if (layout == FG_NT) {
         one = vec ? 0.008f : 0.034f;
@@ -97,12 +99,11 @@ float small_us(int layout, int M, int N, int K, Rows rows, int64_t n, bool colsu
         one = vec && N % 64 == 0 ? 0.012f : 0.036f;
         many = vec && N % 64 == 0 ? 0.010f : 0.034f;
     } else {
-        const bool whole = vec && M % 64 == 0 && N % 64 == 0;
         one = whole ? 0.030f : 0.042f;
         many = whole ? 0.012f : 0.032f;
     }
     return std::max(0, K - 32) * std::max(one, n * many) + 0.2f + 1.2f * n +
-           (layout == FG_TN ? (vec ? 1.0f : 2.0f) : 0.0f) + (colsum ? 5.0f : 0.0f);
+           (layout == FG_TN ? (whole ? 1.0f : vec ? 3.0f : 2.0f) : 0.0f) + (colsum ? 5.0f : 0.0f);
 }
 
 struct Choice16 {
@@ -135,8 +136,7 @@ Choice16 choose16(int layout, int M, int N, int K, int cus, Rows rows, bool cols
         const int units = (bm / 64) * (bn / 64);
         const float rate = (layout == FG_NN ? r->nn : layout == FG_NT ? r->nt : r->tn) * units;
         const int tail = K - (K - (ragged ? 1 : 0)) / bk * bk;
-        const float fixed = kTileUs + kTileUnitUs * units + tail_us(layout, rows, units, tail) +
-                            edge_us(M, N, bm, bn, units);
+        const float fixed = kTileUs + kTileUnitUs * units + tail_us(layout, rows, units, tail);
         for (int s = 1; s <= 16; ++s) {
             int ks = K;
             if (s > 1) {
@@ -150,7 +150,8 @@ Choice16 choose16(int layout, int M, int N, int K, int cus, Rows rows, bool cols
             }
             const int k = s > 1 ? ks : K - tail;  // (a slice has a tail only if it is the last)
             float us = (float)((t * s + cus - 1) / cus) * (k * rate + fixed);
-            if (s > 1) us += kSumUs16 + (2 * s + 1) * (float)M * N * 4.0f / kSumBytesPerUs16;
+            us += s > 1 ? kSumUs16 + (2 * s + 1) * (float)M * N * 4.0f / kSumBytesPerUs16
+                        : edge_us(M, N, bm, bn, units);
             if (us < 0.99f * best.us) best = Choice16{r->cfg, s, s > 1 ? ks : 0, us};
         }
     }
