@@ -1315,6 +1315,9 @@ enum : int {
 // K depth of a configuration.
 inline int cfg_bk(int cfg) { return cfg == kCfg256x128w4 ? kBK : cfg == kCfg64 ? 16 : 32; }
 
+// Waves of a configuration.
+inline int cfg_waves(int cfg) { return cfg == kCfg256 || cfg == kCfg256x128 ? 8 : 4; }
+
 // Output tile of a configuration.
 inline void cfg_tile(int cfg, int &bm, int &bn) {
     static const int kBm[kNumCfgs] = {256, 128, 64, 128, 256, 256};

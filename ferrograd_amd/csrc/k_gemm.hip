@@ -28,10 +28,15 @@ int tiles(int M, int N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn 
 // Tile configuration (indices as in fg_gemm_kernel.h) and K slices of a call,
 // by a model of its time.  Every configuration multiplies at nearly the same
 // rate per CU once a CU has a workgroup (measured on MI355X, 256 CUs, N(0,1)
-// operands, HIP events: kRate, us per k per 64x64 of output, from 1024^3 to
+// operands, HIP events: kRates, us per k per 64x64 of output, from 1024^3 to
 // 4096^3 products in each layout), so what tells them apart is how their
-// tiles fill the CUs: a CU with n workgroups takes n tiles' time.  K slices cut
-// the tiles' depth, for a summing launch and the slots' traffic.  Modelled
+// tiles fill the CUs (a CU with n workgroups takes n tiles' time) and, where K is
+// short, the output a CU writes (kOutUs) and, where it has edges or rows lie
+// unaligned, a wave's part of a tile, written in slower steps (kRaggedUs: 300 x
+// 3998 x 64 NN on 128x64 tiles 12.6 us, 64x64 8.8; 2047 x 4095 x 31 on 256x128
+// 27.6, 64x64 20.1).  K slices cut the tiles' depth, for a summing launch, the slots'
+// traffic and, past 16, kSlotUs a slot (56 x 32 x 65536 NN in 16 / 32 / 64 / 96 / 128 / 256
+// slices 69 / 40 / 28 / 25.5 / 25.6 / 33 us).  Modelled
 // against measured (us, NN): 1536^3 on 128x64 tiles 102 / 102, 64x64 77 / 77;
 // 777 x 1333 x 2049 on 64x64 tiles 70 / 71, in four slices 56 / 57.  Against the
 // choice by thresholds on the tile counts before: 1536^3 96 -> 76, 777 x
@@ -60,12 +65,22 @@ constexpr Rate kRates[3][5] = {
      {kCfg128x64, 0.0155f}, {kCfg64, 0.0159f}},  // NT
     {{kCfg256, 0.0145f}, {kCfg256x128w4, 0.0152f}, {kCfg128, 0.0153f},
      {kCfg128x64, 0.0150f}, {kCfg64, 0.0157f}}};  // TN
-// The summing launch: its own time, and the rate at which it and the GEMM
-// move the slots.
-constexpr float kSumUs = 2.0f, kSumBytesPerUs = 4.0e6f;
+// Per 64x64 of a CU's output (128x64 tiles: measured apart), and per 64x64 that
+// four waves hold of a tile with edges or unaligned rows.
+constexpr float kOutUs = 0.55f, kOut128x64Us = 0.7f, kRaggedUs = 1.5f;
+// The summing launch: its own time, what a slot past the sixteenth adds to it, and
+// the rate at which it and the GEMM move the slots.
+constexpr float kSumUs = 2.0f, kSlotUs = 0.09f, kSumBytesPerUs = 4.0e6f;
+constexpr int kMaxSlices = 256;
 
-// one_cfg: only that configuration (-1: any).  A K that is not whole tiles
-// (or rows unaligned: !aligned) takes the staged tiles, not 256x256.
+// What the slices of a product add: the summing launch and the slots' traffic.
+float slices_us(int M, int N, int s) {
+    return kSumUs + kSlotUs * std::max(0, s - 16) + (2 * s + 1) * (float)M * N * 4.0f / kSumBytesPerUs;
+}
+
+// one_cfg: only that configuration (-1: any), on the kernel that is not
+// pipelined, which takes twice as long per k.  A K that is not whole tiles (or
+// rows unaligned: !aligned) takes the staged tiles, not 256x256.
 Choice choose(int layout, int M, int N, int K, int cus, bool aligned, bool colsum,
               uint64_t ws_bytes, int one_cfg = -1) {
     Choice best;
@@ -77,21 +92,27 @@ Choice choose(int layout, int M, int N, int K, int cus, bool aligned, bool colsu
         if (one_cfg >= 0 && r.cfg != one_cfg) continue;
         if (r.cfg == kCfg256 && (!aligned || K % bk != 0 || (layout != FG_TN && K < 4096))) continue;
         const int64_t t = tiles(M, N, bm, bn);
-        const float unit = r.us * (bm / 64) * (bn / 64);
-        for (int s = 1; s <= 16; ++s) {
-            int ks = K;
+        const int units = (bm / 64) * (bn / 64);
+        const float unit = r.us * units * (one_cfg >= 0 ? 2.0f : 1.0f);
+        const float out = (r.cfg == kCfg128x64 ? kOut128x64Us : kOutUs) * units;
+        const float ragged = aligned && M % bm == 0 && N % bn == 0
+                                 ? 0.0f
+                                 : kRaggedUs * units * 4.0f / fg::gemm::cfg_waves(r.cfg);
+        // (Every count up to 16, then in steps.)
+        for (int n = 1; n <= kMaxSlices; n += n < 16 ? 1 : n / 8) {
+            int s = n, ks = K;
             if (s > 1) {
                 // At least eight K tiles in all and four a slice, whole ones;
                 // slices only while the CUs have under four tiles each.
                 // (A weight gradient of a narrow head stays one launch.)
                 if ((colsum && N < 64) || K < 8 * bk || s > K / (4 * bk) || t * s > 4 * (int64_t)cus) break;
                 ks = ((K + s - 1) / s + bk - 1) / bk * bk;
-                if ((K + ks - 1) / ks != s) continue;
+                s = (K + ks - 1) / ks;
                 if ((uint64_t)s * ((uint64_t)M * N + (colsum ? N : 0)) * sizeof(float) > ws_bytes)
                     break;
             }
-            float us = (float)((t * s + cus - 1) / cus) * ks * unit;
-            if (s > 1) us += kSumUs + (2 * s + 1) * (float)M * N * 4.0f / kSumBytesPerUs;
+            float us = (float)((t * s + cus - 1) / cus) * (ks * unit + out) + ragged;
+            if (s > 1) us += slices_us(M, N, s);
             if (us < 0.99f * best.us) best = Choice{r.cfg, s, s > 1 ? ks : 0, us};
         }
     }

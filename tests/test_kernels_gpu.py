@@ -764,6 +764,32 @@ def test_gemm_f32_any_rows(gpu_ctx, layout, place):
             assert torch.equal(got(), torch.where(zs > 0, ref, torch.zeros_like(ref)))
 
 
+@pytest.mark.parametrize("layout", [O.NN, O.NT, O.TN], ids=["NN", "NT", "TN"])
+def test_gemm_f32_deep_k(gpu_ctx, layout):
+    """Few outputs of a K so deep that it takes more than 16 slices (odd counts of
+    them, a last slice of any length): small-integer operands, outputs and column
+    sums bit for bit."""
+    torch = _torch()
+    gpu_ctx.reserve_workspace(64 << 20)
+    g = torch.Generator().manual_seed(23)
+    for M, N, K in ((56, 64, 40000), (130, 70, 20011), (64, 200, 65536), (256, 64, 9001)):
+        note(f"gemm_f32_deep_k {layout} {M}x{N}x{K}")
+        a = torch.randint(-3, 4, (K, M) if layout == O.TN else (M, K), generator=g).float()
+        b = torch.randint(-3, 4, (N, K) if layout == O.NT else (K, N), generator=g).float()
+        ref = ((a.T if layout == O.TN else a).double() @
+               (b.T if layout == O.NT else b).double()).float()
+        A, B = a.cuda(), b.cuda()
+        C, S = empty((M, N)), empty((N,))
+        gpu_ctx.gemm(layout, M, N, K, A, A.shape[1], B, B.shape[1], C, N)
+        torch.cuda.synchronize()
+        assert torch.equal(C.cpu(), ref)
+        if layout == O.TN:
+            gpu_ctx.gemm_dw(M, N, K, A, M, B, N, C, N, colsum=S)
+            torch.cuda.synchronize()
+            assert torch.equal(C.cpu(), ref)
+            assert torch.equal(S.cpu().double(), b.double().sum(0))
+
+
 # 16-bit tiles on rows of any alignment, as test_gemm_f32_any_rows: K
 # remainders of the tile pipeline (1 to 6 tiles of 32 and a tail), rows that end
 # between chunks, even and odd leading dimensions, K slices, edges of tiles.
