@@ -620,12 +620,69 @@ bool pairable(const Planned &P1, const Planned &P2) {
     return fg::gemm::pair_exclusive(k1) || fg::gemm::pair_exclusive(k2) ? k1 == k2 : true;
 }
 
+// dW and dX of a layer on the 64x64 tiles, of which dX splits K: the slices each
+// would take alone are not those that the two should take together.  dW's tiles
+// fill the CUs that dX's leave, so dX takes fewer slices, and dW none (two split
+// GEMMs do not pair: their slices take the same workspace), where the one launch
+// and dX's sum are then shorter (us: 448 x 1024 x 448 20.1 -> 16.4, 640 x 2992 x
+// 88 26.8 -> 20.2; before dW's column sums split K they took 16.7 and 22.3).
+void share_slices(const fg_ctx *ctx, Planned &W, Planned &X) {
+    auto small = [](const Planned &P) {
+        return !P.empty && !P.skinny && !P.rows && P.pipe && P.cfg == kCfg64 &&
+               P.pro == fg::gemm::kProNone;
+    };
+    if (!small(W) || !small(X) || X.splits <= 1) return;
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, bk = fg::gemm::cfg_bk(kCfg64);
+    const int tw = tiles(W.a.M, W.a.N, 64, 64), tx = tiles(X.a.M, X.a.N, 64, 64);
+    auto tile_us = [](const Planned &P, int k) {
+        float r = 0.0f;
+        for (const Rate &q : kRates[P.layout])
+            if (q.cfg == kCfg64) r = q.us;
+        return k * r + kOutUs;
+    };
+    auto alone = [&](const Planned &P, int t) {
+        const int n = (t * P.splits + cus - 1) / cus;
+        return n * tile_us(P, P.splits > 1 ? P.a.ksplit : P.a.K) +
+               (P.splits > 1 ? slices_us(P.a.M, P.a.N, P.splits) : 0.0f);
+    };
+    // In one launch, dW unsplit, dX in s slices of ks: one round of workgroups, or
+    // the CUs' share of the work and on average half of the deeper tile's time.
+    auto together = [&](int s, int ks) {
+        const float w = tile_us(W, W.a.K), x = tile_us(X, ks), deep = std::max(w, x);
+        const float share = (tw * w + tx * s * x) / cus + 0.5f * deep;
+        return (tw + tx * s <= cus ? deep : std::max(deep, share)) +
+               (s > 1 ? slices_us(X.a.M, X.a.N, s) : 0.0f);
+    };
+    float us = W.splits > 1 ? alone(W, tw) + alone(X, tx) + kSumUs
+                            : together(X.splits, X.a.ksplit);
+    int best = 0, best_ks = 0;
+    us *= 0.9f;  // (else as each would alone, to the same bits)
+    for (int s = 1; s <= X.splits; ++s) {
+        const int ks = s > 1 ? ((X.a.K + s - 1) / s + bk - 1) / bk * bk : X.a.K;
+        if ((X.a.K + ks - 1) / ks != s) continue;
+        const float t = together(s, ks);
+        if (t < us) {
+            us = t;
+            best = s;
+            best_ks = ks;
+        }
+    }
+    if (best == 0) return;
+    W.splits = 1;
+    W.a.ksplit = 0;
+    W.a.partial = W.a.colsum_partial = nullptr;
+    X.splits = best;
+    X.a.ksplit = best > 1 ? best_ks : 0;
+    if (best == 1) X.a.partial = nullptr;
+}
+
 // Two unsplit pipelined GEMMs of different kinds (dW and dX of a layer) on the
 // 64x64 or the 128x64 tiles both, where one launch of all their tiles is
 // shorter than the two they would take alone: the tiles of the second fill the
 // CUs that the last of the first leave (and their bits are those of any tile:
 // each output sums its K in the same order).
 void join(const fg_ctx *ctx, Planned &P1, Planned &P2) {
+    share_slices(ctx, P1, P2);
     auto plain = [](const Planned &P) {
         return !P.empty && !P.skinny && !P.rows && P.pipe && P.splits == 1 &&
                P.pro == fg::gemm::kProNone;
@@ -729,8 +786,9 @@ namespace fg {
 // A layer's weight gradient dW (=|+=) X^T.dZ with dbias (=|+=) the column
 // sums of dZ (as fg_gemm_dw_f32) and its data gradient dX (=|+=)
 // (dZ.W^T) * act'(Zs) (as fg_gemm_bwd_f32, NT): independent GEMMs, one
-// launch when both take small 256-thread kernels, else one after the other.
-// The same results, bit for bit, either way.
+// launch when both take small 256-thread kernels, else one after the other:
+// the results of the two calls, bit for bit, unless share_slices cut K for the
+// two together.
 int gemm_dw_dx_f32(fg_ctx *ctx, int M1, int N1, int K1, const float *A1, int lda1,
                    const float *B1, int ldb1, float *C1, int ldc1, int acc1, float *colsum,
                    int colsum_acc, int M2, int N2, int K2, const float *A2, int lda2,

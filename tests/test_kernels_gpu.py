@@ -790,6 +790,31 @@ def test_gemm_f32_deep_k(gpu_ctx, layout):
             assert torch.equal(S.cpu().double(), b.double().sum(0))
 
 
+@pytest.mark.parametrize("dims", [(448, 1024, 448), (640, 2992, 88), (512, 512, 64), (64, 256, 784),
+                                  (300, 700, 130), (67, 378, 2229)],
+                         ids=lambda d: "x".join(map(str, d)))
+def test_matmul_bwd_slices(gpu_ctx, dims):
+    """dW (+ dbias) and dX whose K splits, together or apart: small-integer
+    operands, every gradient bit for bit, with and without accumulation."""
+    torch = _torch()
+    gpu_ctx.reserve_workspace(64 << 20)
+    M, N, K = dims
+    g = torch.Generator().manual_seed(29)
+    x, w, dz, zs, dx0, dw0, db0 = (torch.randint(-3, 4, s, generator=g).float() for s in
+                                   ((M, K), (K, N), (M, N), (M, K), (M, K), (K, N), (N,)))
+    X, W, dZ, Zs = (t.cuda() for t in (x, w, dz, zs))
+    dw, db = (x.T.double() @ dz.double()).float(), dz.double().sum(0).float()
+    dx = torch.where(zs > 0, (dz.double() @ w.T.double()).float(), torch.zeros(M, K))
+    for acc in (False, True):
+        dX, dW, dB = dx0.cuda(), dw0.cuda(), db0.cuda()
+        gpu_ctx.matmul_bwd(M, N, K, X, K, W, N, dZ, N, dX, K, dW, N, dbias=dB, act=O.ACT_RELU,
+                           Zs=Zs, ldzs=K, accumulate=acc)
+        torch.cuda.synchronize()
+        assert torch.equal(dW.cpu(), dw + dw0 if acc else dw)
+        assert torch.equal(dB.cpu(), db + db0 if acc else db)
+        assert torch.equal(dX.cpu(), dx + dx0 if acc else dx)
+
+
 # 16-bit tiles on rows of any alignment, as test_gemm_f32_any_rows: K
 # remainders of the tile pipeline (1 to 6 tiles of 32 and a tail), rows that end
 # between chunks, even and odd leading dimensions, K slices, edges of tiles.
