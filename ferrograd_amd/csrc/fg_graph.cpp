@@ -2435,7 +2435,8 @@ FG_API int fg_plan_describe(const fg_plan *p, char *buf, size_t len, size_t *nee
                                          L.kind == LK_GEMM && L.sExtra != kNone);
         return fg::gemm_f32_dispatches(wc, L.sExtra != kNone ? FG_TN : L.layout, L.M, L.N, L.K,
                                        p->ptr(L.sA), L.lda, p->ptr(L.sB), L.ldb,
-                                       L.kind == LK_GEMM && L.sExtra != kNone);
+                                       L.kind == LK_GEMM && L.sExtra != kNone,
+                                       L.kind == LK_GEMM_BWD);
     };
     // Dispatches of a forward chain (L and the next launch X).
     auto chain_dispatches = [&](const Launch &L, const Launch &X) {
@@ -2562,6 +2563,7 @@ FG_API int fg_plan_describe(const fg_plan *p, char *buf, size_t len, size_t *nee
             };
             std::vector<fg::ByteRange> held = {slot_range(H->sC)};
             if (H->kind == LK_GEMM_BWD && H->act != FG_ACT_NONE) held.push_back(slot_range(H->sZ));
+            if (H->kind == LK_GEMM && H->sExtra != kNone) held.push_back(slot_range(H->sExtra));
             bool shared = true;
             for (const fg::ByteRange &o : optim_ranges(*p))
                 for (const fg::ByteRange &q : held) shared = shared && !q.overlaps(o);

@@ -178,9 +178,10 @@ bool eltwise_jit_selected(const EltProgram &p);
 int eltwise_jit(fg_ctx *ctx, const EltProgram &p, int live, bool prepare_only, bool *launched);
 void eltwise_count_interpreted();
 // Kernel dispatches of one fp32 GEMM call with these operands (2 when K is
-// split: the slices, then the summing epilogue), for plan descriptions.
+// split: the slices, then the summing epilogue), for plan descriptions.  bwd: a
+// data gradient (fg_gemm_bwd_f32).
 int gemm_f32_dispatches(fg_ctx *ctx, int layout, int M, int N, int K, const void *A, int lda,
-                        const void *B, int ldb, bool colsum);
+                        const void *B, int ldb, bool colsum, bool bwd = false);
 // A layer's dW (TN, fused column sums) and dX (NT, act'(Zs)) GEMMs, in one
 // launch when both take small kernels (k_gemm.hip), and its dispatch count.
 int gemm_dw_dx_f32(fg_ctx *ctx, int M1, int N1, int K1, const float *A1, int lda1,

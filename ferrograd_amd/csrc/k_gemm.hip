@@ -452,9 +452,10 @@ void pending_reduce_ranges(const fg_ctx *ctx, ByteRange out[4]) {
 }
 
 int gemm_f32_dispatches(fg_ctx *ctx, int layout, int M, int N, int K, const void *A, int lda,
-                        const void *B, int ldb, bool colsum) {
+                        const void *B, int ldb, bool colsum, bool bwd) {
     if (!ctx || M <= 0 || N <= 0) return 1;  // no workspace (or nothing to do): no split
     GemmArgs a{};
+    a.mode = bwd ? 1 : 0;
     a.A = static_cast<const float *>(A);
     a.B = static_cast<const float *>(B);
     a.M = M;
@@ -969,7 +970,7 @@ int gemm_dw_dx_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A1, i
                           const void *B1, int ldb1, int M2, int N2, int K2, const void *A2,
                           int lda2, const void *B2, int ldb2) {
     const int sep = gemm_f32_dispatches(ctx, FG_TN, M1, N1, K1, A1, lda1, B1, ldb1, true) +
-                    gemm_f32_dispatches(ctx, FG_NT, M2, N2, K2, A2, lda2, B2, ldb2, false);
+                    gemm_f32_dispatches(ctx, FG_NT, M2, N2, K2, A2, lda2, B2, ldb2, false, true);
     if (!ctx || M1 <= 0 || N1 <= 0 || K1 <= 0 || M2 <= 0 || N2 <= 0 || K2 <= 0) return sep;
     // Dummy aligned outputs: only the operands' alignment enters the choice.
     float *c = reinterpret_cast<float *>(256);

@@ -861,6 +861,27 @@ def test_captured_sgd_fused_paths_at_other_shapes(ctx, dims, B, act):
             st.plan.close()
 
 
+def test_describe_counts_a_lone_data_gradient(ctx):
+    """The data gradient of a layer whose weights need none (16 rows, 100x700
+    weights) is a GEMM of its own on the tiles, K split: the description counts its
+    two launches."""
+    G = api()
+    graph, meta = new_graph(G.MEAN_SQUARED_ERROR, G.Optim.sgd())
+    B, k, n = meta.new_field(), meta.new_field(), meta.new_field()
+    with graph.define_ops() as ops:
+        x = ops.input([B, k])
+        W = ops.input([k, n], requires_grad=False)
+        ops.matmul(x, W)
+    st = ctx.alloc_tensors(graph, graph.compute_saved_nodes(), [G.f32_bits(1e-3), 16, 100, 700])
+    try:
+        desc = st.plan.describe()
+    finally:
+        st.plan.close()
+    bwd = desc.split("backward(seed)")[1].split("optim:")[0]
+    line = [l for l in bwd.splitlines() if "gemm NT 16x100x700" in l]
+    assert len(line) == 1 and "[K split: slices + summing kernel]" in line[0], desc
+
+
 @pytest.mark.parametrize("dims,B", [([64, 512, 10], 512), ([32, 1024, 10], 1024),
                                     ([128, 512, 3], 512)],
                          ids=["64-512-10-b512", "32-1024-10-b1024", "128-512-3-b512"])
