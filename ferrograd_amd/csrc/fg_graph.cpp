@@ -2438,13 +2438,20 @@ FG_API int fg_plan_describe(const fg_plan *p, char *buf, size_t len, size_t *nee
                                        L.kind == LK_GEMM && L.sExtra != kNone,
                                        L.kind == LK_GEMM_BWD);
     };
-    // Dispatches of a forward chain (L and the next launch X).
+    // Dispatches of a forward chain (L and the next launch X), and whether X sums
+    // L's slices.
+    bool chained = false;
     auto chain_dispatches = [&](const Launch &L, const Launch &X) {
+        chained = false;
         if (!wc) return gemm_dispatches(L) + gemm_dispatches(X);
         return fg::gemm_fwd_chain_dispatches(
             wc, L.M, L.N, L.K, p->ptr(L.sA), L.lda, p->ptr(L.sB), L.ldb, p->ptr(L.sBias),
             p->ptr(L.sC), L.ldc, p->ptr(L.sZ), L.ldz, X.M, X.N, X.K, p->ptr(X.sA), X.lda,
-            p->ptr(X.sB), X.ldb);
+            p->ptr(X.sB), X.ldb, &chained);
+    };
+    auto chains = [&](const Launch &L, const Launch &X) {
+        chain_dispatches(L, X);
+        return chained;
     };
     auto add = [&](const char *title, const std::vector<Launch> &v) {
         s += std::string(title) + ": " + std::to_string(v.size()) + " launches\n";
@@ -2452,14 +2459,12 @@ FG_API int fg_plan_describe(const fg_plan *p, char *buf, size_t len, size_t *nee
             const Launch &L = v[i];
             s += "  " + L.desc;
             const int nd = gemm_dispatches(L);
-            if (nd == 3) {  // a 16-bit dW off the pipelined kernel
+            if (L.chain_next && i + 1 < v.size() && chains(L, v[i + 1]))
+                s += " [K split: slices, summed by the next launch]";
+            else if (nd == 3)  // a 16-bit dW off the pipelined kernel
                 s += " [GEMM + column-sum reduction]";
-            } else if (nd > 1) {
-                const bool summed_by_next = L.chain_next && i + 1 < v.size() &&
-                                            chain_dispatches(L, v[i + 1]) == 2;
-                s += summed_by_next ? " [K split: slices, summed by the next launch]"
-                                    : " [K split: slices + summing kernel]";
-            }
+            else if (nd > 1)
+                s += " [K split: slices + summing kernel]";
             s += "\n";
         }
     };
@@ -2525,8 +2530,8 @@ FG_API int fg_plan_describe(const fg_plan *p, char *buf, size_t len, size_t *nee
     int k_loss = kernels(p->loss);
     // A captured SGD step may finish the loss in the head GEMM, and then the
     // head's data gradient too, its dW joining the next pair's launch.
-    if (const int hc = head_loss_chain(*p); hc >= 0 && wc &&
-                                            chain_dispatches(p->fwd[hc], p->fwd[hc + 1]) == 2) {
+    if (const int hc = head_loss_chain(*p);
+        hc >= 0 && wc && chains(p->fwd[hc], p->fwd[hc + 1])) {
         k_loss = 0;
         s += "(captured step: the head GEMM finishes the loss; its mean runs in the SGD launch)\n";
         if (head_bwd_fusable(*p, bwd, hc)) {

@@ -224,7 +224,7 @@ int gemm_fwd_chain_f32(fg_ctx *ctx, int M1, int N1, int K1, const float *A1, int
 int gemm_fwd_chain_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A1, int lda1,
                               const void *B1, int ldb1, const void *bias1, void *C1, int ldc1,
                               void *Z1, int ldz1, int M2, int N2, int K2, const void *A2, int lda2,
-                              const void *B2, int ldb2);
+                              const void *B2, int ldb2, bool *chained);
 }  // namespace fg
 
 #define FG_HIP(call)                                                     \

@@ -869,11 +869,13 @@ int gemm_fwd_chain_f32(fg_ctx *ctx, int M1, int N1, int K1, const float *A1, int
     return FG_OK;
 }
 
-// Dispatches of gemm_fwd_chain_f32 for these operands (no launch).
+// Dispatches of gemm_fwd_chain_f32 for these operands (no launch), and whether
+// GEMM 2's kernel sums GEMM 1's slices.
 int gemm_fwd_chain_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A1, int lda1,
                               const void *B1, int ldb1, const void *bias1, void *C1, int ldc1,
                               void *Z1, int ldz1, int M2, int N2, int K2, const void *A2, int lda2,
-                              const void *B2, int ldb2) {
+                              const void *B2, int ldb2, bool *chained) {
+    *chained = false;
     const int sep = gemm_f32_dispatches(ctx, FG_NN, M1, N1, K1, A1, lda1, B1, ldb1, false) +
                     gemm_f32_dispatches(ctx, FG_NN, M2, N2, K2, A2, lda2, B2, ldb2, false);
     if (!ctx || M1 <= 0 || N1 <= 0 || M2 <= 0 || N2 <= 0) return sep;
@@ -884,7 +886,8 @@ int gemm_fwd_chain_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A
     plan_quiet(ctx, FG_NN, a1, P1);
     plan_quiet(ctx, FG_NN, fwd_args(M2, N2, K2, (const float *)A2, lda2, (const float *)B2, ldb2,
                                     nullptr, FG_ACT_NONE, nullptr, N2, nullptr, 0, 0), P2);
-    return chainable(P1, P2) ? 2 : sep;
+    *chained = chainable(P1, P2);
+    return *chained ? 2 : sep;
 }
 
 // A small head's weight gradient (with its bias gradient; TN) beside a

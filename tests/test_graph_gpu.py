@@ -882,6 +882,17 @@ def test_describe_counts_a_lone_data_gradient(ctx):
     assert len(line) == 1 and "[K split: slices + summing kernel]" in line[0], desc
 
 
+def test_describe_head_without_a_chain(ctx):
+    """A first layer too short in K to split (96 inputs) is not chained to the head,
+    whose kernel then does not finish the loss: the description says so."""
+    G = api()
+    _, _, _, st = build_mlp(ctx, [96, 64, 12], 48, "relu", G.Optim.sgd())
+    desc = st.plan.describe()
+    st.plan.close()
+    assert "summed by the next launch" not in desc, desc
+    assert "the head GEMM finishes the loss" not in desc, desc
+
+
 @pytest.mark.parametrize("dims,B", [([64, 512, 10], 512), ([32, 1024, 10], 1024),
                                     ([128, 512, 3], 512)],
                          ids=["64-512-10-b512", "32-1024-10-b1024", "128-512-3-b512"])
