@@ -193,9 +193,10 @@ void set_choice(const fg_ctx *ctx, GemmArgs &a, const Choice &ch) {
 // chunks (aligned) and whether it takes any K and rows (ktail), the tile configuration and the
 // number of K slices.  pro: the prologue code (fg::gemm::kPro*), whose
 // tensor Pz must meet the same 16-byte conditions as the operand it scales.
+// few_rows false: not the few-row kernel.
 void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &rows, bool &vec,
                bool &pipe, bool &ktail, bool &aligned, int &cfg, int &splits,
-               int pro = fg::gemm::kProNone) {
+               int pro = fg::gemm::kProNone, bool few_rows = true) {
     skinny = use_skinny(ctx, a, pro);
     vec = pipe = ktail = rows = aligned = false;
     cfg = 0;
@@ -215,7 +216,7 @@ void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &rows, b
     auto al16 = [](const void *q) { return (((uintptr_t)q) & 15u) == 0; };
     a.vec_out = al16(a.C) && a.ldc % 4 == 0 && (!a.Z || (al16(a.Z) && a.ldz % 4 == 0)) &&
                 (!a.bias || al16(a.bias));
-    rows = use_rows(layout, a, pro);
+    rows = few_rows && use_rows(layout, a, pro);
     if (rows) {
         int ks;
         splits = fg::rows::split_of(cus, 4, a.M, a.N, a.K, ctx->ws_bytes, ks);
@@ -771,6 +772,21 @@ bool chainable(const Planned &P1, const Planned &P2) {
            b.K == a.N && b.M == a.M;
 }
 
+// As chainable, with GEMM 1 on the tiles if it is the few-row kernel, unsplit, that
+// keeps it from a chain: what that kernel saves (32 x 256 x 784 9.9 -> 8.3 us with
+// the tiles' sum) is less than the launches that a step's head needs without the
+// chain.  P1 is left as planned otherwise.
+bool chain_plan(fg_ctx *ctx, Planned &P1, const Planned &P2) {
+    if (chainable(P1, P2)) return true;
+    if (!P1.rows || P1.splits > 1) return false;
+    Planned T = P1;
+    plan_gemm(ctx, T.layout, T.a, T.skinny, T.rows, T.vec, T.pipe, T.ktail,
+              T.aligned, T.cfg, T.splits, T.pro, false);
+    if (!chainable(T, P2)) return false;
+    P1 = T;
+    return true;
+}
+
 // The kernel choices alone, for counting dispatches: no validation, no error
 // message, operands not bound yet taken as 16-byte aligned.
 void plan_quiet(fg_ctx *ctx, int layout, const GemmArgs &a0, Planned &P) {
@@ -854,7 +870,7 @@ int gemm_fwd_chain_f32(fg_ctx *ctx, int M1, int N1, int K1, const float *A1, int
         gemm_prepare(ctx, FG_NN, fwd_args(M2, N2, K2, A2, lda2, B2, ldb2, bias2, act2, C2, ldc2,
                                           Z2, ldz2, acc2),
                      "fg_gemm_f32", fg::gemm::kProNone, P2) ||
-        !chainable(P1, P2)) {
+        !chain_plan(ctx, P1, P2)) {
         fg::clear_error();
         return separate();
     }
@@ -886,7 +902,7 @@ int gemm_fwd_chain_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A
     plan_quiet(ctx, FG_NN, a1, P1);
     plan_quiet(ctx, FG_NN, fwd_args(M2, N2, K2, (const float *)A2, lda2, (const float *)B2, ldb2,
                                     nullptr, FG_ACT_NONE, nullptr, N2, nullptr, 0, 0), P2);
-    *chained = chainable(P1, P2);
+    *chained = chain_plan(ctx, P1, P2);
     return *chained ? 2 : sep;
 }
 

@@ -893,6 +893,20 @@ def test_describe_head_without_a_chain(ctx):
     assert "the head GEMM finishes the loss" not in desc, desc
 
 
+@pytest.mark.parametrize("k1", [256, 784, 900, 1024, 1500, 4096])
+@pytest.mark.parametrize("B", [8, 17, 32])
+def test_captured_sgd_small_batches_chain(ctx, B, k1):
+    """Two-layer MLPs at batches of the few-row kernel, with first layers that it
+    takes unsplit (K under 1024) and in slices: the head's kernel sums the first
+    layer's slices and finishes the loss, as at larger batches."""
+    G = api()
+    _, _, _, st = build_mlp(ctx, [k1, 256, 10], B, "relu", G.Optim.sgd())
+    desc = st.plan.describe()
+    st.plan.close()
+    assert "the head GEMM finishes the loss" in desc, desc
+    test_captured_sgd_fused_paths_at_other_shapes(ctx, [k1, 256, 10], B, "relu")
+
+
 @pytest.mark.parametrize("dims,B", [([64, 512, 10], 512), ([32, 1024, 10], 1024),
                                     ([128, 512, 3], 512)],
                          ids=["64-512-10-b512", "32-1024-10-b1024", "128-512-3-b512"])
