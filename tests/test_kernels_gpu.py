@@ -1288,3 +1288,41 @@ def test_softmax_row_sum_order(gpu_ctx):
     assert ((y.cpu().double() - p).abs() <= 5 * 2.0 ** -24 * p)[:, :256].all()
     cols = lab.long()[:, None]
     assert torch.equal(d.cpu().gather(1, cols), y.cpu().gather(1, cols) - 1.0)
+
+
+@pytest.mark.parametrize("C,active", [(2048, 1024), (32768, 8192), (131072, 8192)])
+@pytest.mark.parametrize("dtype", [1, 2], ids=["f16", "bf16"])
+def test_softmax_exponential_16bit(gpu_ctx, dtype, C, active):
+    """The fp32 row loss of 16-bit rows shows the exponential's own error: one
+    logit 0, `active` of -D, the rest -inf, so that all sums but a few are exact and
+    the loss is log(1 + active exp(-D)), for 64 D around 8.  In units of 2^-24: 1.5
+    for the exponential, half a unit for each of at most 3 sums and of the loss, 2
+    for the logarithm."""
+    torch = _torch()
+    dt = [None, torch.float16, torch.bfloat16][dtype]
+    D = (torch.arange(64) / 32 + 7).to(dt)
+    x = torch.full((64, C), float("-inf"), dtype=dt)
+    x[:, :active] = -D[:, None]
+    x[:, C - 5] = 0.0
+    lab = torch.full((64,), C - 5, dtype=torch.int32).cuda()
+    loss, d = empty((64,)), torch.empty(64, C, dtype=dt, device="cuda")
+    gpu_ctx.softmax_ce(x.cuda(), C, lab, 64, C, 1.0, row_loss=loss, dlogits=d, ldd=C, dtype=dtype)
+    torch.cuda.synchronize()
+    ref = torch.log1p(active * torch.exp(-D.double()))
+    err = (loss.cpu().double() - ref).abs().max().item() * 2.0 ** 24
+    assert err <= 5.5, err
+
+
+def test_softmax_bf16_subnormal(gpu_ctx):
+    """Probabilities under 2^-126 keep bf16's subnormal values: within one unit of
+    them (the fp32 value rounds once before)."""
+    torch = _torch()
+    x = torch.full((64, 2048), -88.0, dtype=torch.bfloat16)
+    x -= torch.arange(64, dtype=torch.bfloat16)[:, None] / 16
+    x[:, 7] = 0.0
+    y = torch.empty(64, 2048, dtype=torch.bfloat16, device="cuda")
+    gpu_ctx.softmax(x.cuda(), 64, 2048, y, dtype=2)
+    torch.cuda.synchronize()
+    p = torch.softmax(x.double(), 1)
+    assert p[:, 0].min() > 2.0 ** -133 and p[:, 0].max() < 2.0 ** -126
+    assert ((y.cpu().double() - p).abs() <= 2.0 ** -133)[:, 8:].all()
