@@ -9,20 +9,22 @@
 // 16), as rows of equal length and equally aligned tensors do.  Outputs may
 // be the inputs themselves.
 //
-// What bounds it: HBM, by holding a row in registers so that it is read and
-// written once.  Waves per row and chunks per thread (with_kind in k_softmax.hip, measured over
-// 1, 2, 4, 8 and 16 chunks on 1, 4, 8 and 16 waves, HIP events): the fewest
-// waves that hold the row without spilling, one wave a row up to 256 chunks
-// (no workgroup barrier; 16384 x 1000 fp32 24.2 us against 27.5 on four
-// waves and 31.7 for the 256-thread kernel before), and never so many
-// registers that only one row fits a CU: 16 chunks on 16 waves read and wrote
-// at 3.1-4.4 TB/s against 4.3-4.5 for the two-pass kernel below.
+// What bounds it: HBM in fp32, the vector unit in 16 bits from where a row's
+// exponentials are taken twice (NV > 4), by holding a row in registers so that it
+// is read and written once.  Waves per row and chunks per thread (with_kind in
+// k_softmax.hip, measured over 1, 2, 4, 8 and 16 chunks on 1, 4, 8 and 16 waves,
+// HIP events): the fewest waves that hold the row in the registers that let two
+// rows share a CU, one wave a row up to 256 chunks (no workgroup barrier; 16384 x
+// 1000 fp32 24.2 us against 27.5 on four waves and 31.7 for the 256-thread kernel
+// before).  8 chunks on 16 waves need 1 (fp32) and 3 (16 bits) registers more than
+// that and spill them, which costs less than a row alone on its CU: 16 chunks on 16
+// waves read and wrote at 3.1-4.4 TB/s against 4.3-4.5 for the two-pass kernel below.
 // Against the kernels before (float4 rows aligned and in whole chunks; one
 // element a lane, two passes and two expf an element otherwise), us:
-//   CE fp32  8192 x 32000  359.8 -> 358.0   2048 x 2048   7.8 -> 6.9
-//            2000 x 10001   58.6 ->  29.6   2000 x 50257  358 -> 187
-//   CE bf16  2048 x 50257  300.1 ->  83.5   8192 x 32000  470 -> 178
-//            4000 x 10001  102.0 ->  31.1   1500 x 131072 721 -> 183
+//   CE fp32  2048 x 2048   7.8 -> 6.9     2000 x 10001   58.6 -> 29.6
+//            2000 x 50257  358 -> 187
+//   CE bf16  2048 x 50257  292 -> 92      8192 x 32000   465 -> 190
+//            4000 x 10001  99.4 -> 34     1500 x 131072  721 -> 181
 //   backward fp32 8192 x 32000 1063 -> 521  bf16 2048 x 50257 455 -> 113
 #pragma once
 
@@ -85,7 +87,7 @@ struct Io {
 // 2^-24: at most 1.37 off, 0.45 rms, as expf (1.35, 0.44); the exponential of
 // (x - m) log2(e) rounded to fp32 is 2.7 off at -2, 8 at -8, 16 at -20, which
 // shows in the fp32 row loss and below 2^-126 gives zeros.  2048 x 50257 CE bf16 /
-// f16: 81 us with that, 94 / 105, with expf 111 / 128.
+// f16: 81 us with that, 92 / 92, with expf 111 / 128.
 template <int DT>
 __device__ __forceinline__ float exp_below(float x, float m) {
     if constexpr (DT == kF32) {
@@ -315,14 +317,20 @@ void softmax_any(const typename Io<DT>::T *x, int ldx,
     float ex[kHold ? NV * E : 1];
     vs = sp.single(t) >= 0 ? exp_below<DT>(vs, m) : 0.0f;
     RowSum<DT, NV, NW> sum(vs);
+    // Where exponentials are taken twice, a wave leaves out the chunks of which it
+    // holds none: 4000 x 10001 bf16 / f16 42 / 49 us, now 34 / 40.  (Held ones: no
+    // faster, 8192 x 2048 12.6 / 14.4 against 16.)
+    const int first = __builtin_amdgcn_readfirstlane(t) & ~63;
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
+    for (int i = 0; i < NV; ++i) {
+        if (!kHold && first + i * NT >= sp.nb) break;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const float p = exp_below<DT>(IO::get(w[i], e), m);
             if constexpr (kHold) ex[i * E + e] = p;
             sum.add(i, e, p);
         }
+    }
     // The label's logit, in the thread that writes its column and before any
     // thread stores (out may be x).
     const bool mine = tc >= 0 && t == sp.owner(tc, NT);
