@@ -49,9 +49,13 @@ inline Split split_of(int cus, int M, int N) {
 
 // DT: element type of dZ (fg_half.h codes).  Rows of any alignment are read (and
 // written) 4 elements at a time: with one element a lane where they were not
-// 16-byte (8-byte) aligned, dZ and its sums for 1000 x 2003 fp32 took 9.1 us, now 8.3; 50 x 101 5.1, now 3.9.  PACT != kActNone (fp32 only):
-// the rows summed are dZ * act'(Pz) (Pz[M][N], row stride ldp), i.e. the bias gradient below an activation whose
-// derivative was not applied yet; with `out` (fp32, row stride ldo) the scaled rows are also written there, so one pass
+// 16-byte (8-byte) aligned, dZ and its sums for 1000 x 2003 fp32 took 9.1 us, now
+// 8.3; 50 x 101 5.1, now 3.9.  16-bit rows that start on odd elements cost these
+// 8-byte loads up to 15 % (bf16 16384 x 8190 91 us against 79, 8192 x 4096 17.6
+// both).  PACT != kActNone (fp32
+// only): the rows summed are dZ * act'(Pz) (Pz[M][N], row stride ldp), i.e. the
+// bias gradient below an activation whose derivative was not applied yet; with
+// `out` (fp32, row stride ldo) the scaled rows are also written there, so one pass
 // materialises dZ = dC * act'(Pz) and sums its columns.
 template <int DT, int PACT = kActNone>
 __global__ __launch_bounds__(kThreads) void bias_grad_partial(const void *__restrict__ dZ, int M,

@@ -640,13 +640,11 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm16_mfma(Args p) {
 // chunk of wave load li landing at element 512 li + 8 l of the operand's
 // stage area; the source of each chunk is chosen so that the stage ends up
 // in the swizzled layout below.  Two ways to move the chunks:
-//  * staged (BK 32 tiles but 256x256 with 4 waves): global loads into
-//    registers, two register sets alternating by tile parity, written to a
-//    two-stage LDS ring by ds_write_b128 one tile later;
-//  * direct (BK 64 tiles, and 256x256 with 4 waves, whose accumulators leave
-//    no room for two register sets): global_load_lds_dwordx4 (inline
-//    assembly, lds_dma16) straight into an LDS ring of up to four stages,
-//    as many as fit -- three for 256x128 tiles, whose two tiles in flight
+//  * staged (BK 32 tiles): global loads into registers, staged_sets16 register
+//    sets in turn, written to a two-stage LDS ring by ds_write_b128 a tile
+//    before they are multiplied;
+//  * direct (BK 64 tiles): global_load_lds_dwordx4 (inline assembly,
+//    lds_dma16) straight into an LDS ring of up to four stages, as many as fit -- three for 256x128 tiles, whose two tiles in flight
 //    ran their NT data gradient 917-922 -> 944-948 TF at 2048x4096x4096
 //    (bf16 c5 step 2.066-2.070 -> 2.037-2.042 ms).
 // A BK of 32 or 64 is only 1-2 thousand MFMA cycles per SIMD, so the barrier
@@ -760,15 +758,14 @@ struct ColSum16 {
 };
 
 // LDS of the pipelined kernel, in 16-bit elements: its stages (staged
-// loads -- global -> registers -> ds_write -- for BK 32 tiles but 256x256
-// with 4 waves (256 accumulator registers): two; direct-to-LDS loads: up to
-// four, as many as fit in the 160 KiB of LDS) or the epilogue's fp32
-// staging, whichever is larger.
+// loads -- global -> registers -> ds_write -- for BK 32 tiles: two;
+// direct-to-LDS loads: up to four, as many as fit in the 160 KiB of LDS) or
+// the epilogue's fp32 staging, whichever is larger.
 template <int BM, int BN, int BK, int WGM, int WGN>
 struct Pipe16Lds {
     static constexpr int kNW = WGM * WGN;
     static constexpr int kStageSz = BM * BK + BN * BK;  // elements
-    static constexpr bool kStaged = BK == 32 && !(BM == 256 && BN == 256 && kNW == 4);
+    static constexpr bool kStaged = BK == 32;
     static constexpr int kStages = kStaged                             ? 2
                                    : 4 * kStageSz * 2 <= 160 * 1024   ? 4
                                    : 3 * kStageSz * 2 <= 160 * 1024 ? 3
@@ -783,7 +780,8 @@ struct Pipe16Lds {
 // BK 32 is an eighth of a microsecond of MFMAs, a load several times that: four
 // sets, with which one workgroup of these tiles a CU beat the larger direct
 // ones split over K (bf16 1024^3 NN / NT 19.5 / 18.8 -> 15.4 / 13.2 us, 2048^3
-// 35.8 / 32.6 -> 28.7 / 25.4).  The 256x256 tiles' registers hold two.
+// 35.8 / 32.6 -> 28.7 / 25.4).  The 256x256 tiles' registers hold two (f16 TN of odd
+// rows spills three).
 constexpr int staged_sets16(int BM, int BN) { return BM * BN <= 128 * 128 ? 4 : 2; }
 
 // The kernel's LDS buffer of N 16-bit elements: one static array per N, so

@@ -1428,9 +1428,9 @@ void launch_skinny_pre(const GemmArgs &a, const GemmArgs &pre, hipStream_t st,
 // with a K tail or unaligned rows) pair with each other; the others only with
 // their own kind (the two kPairMid kinds with each other), both bodies then
 // sharing one LDS buffer:
-// kPairBig: the 8-wave pipelined tiles of large layers, dW on 256x256 (cfg
-// 6, TN) with dX on 256x128 (cfg 7, NT), 512 threads;
-// kPairMid: both on the 4-wave 128x64 pipelined tiles (cfg 5), 256 threads;
+// kPairBig: the 8-wave pipelined tiles of large layers, dW on kCfg256 (TN)
+// with dX on kCfg256x128 (NT), 512 threads;
+// kPairMid: both on the pipelined tiles of kCfg128x64, 256 threads;
 // kPairMidTail: the same with a K tail or unaligned rows.
 enum : int {
     kPairSkinny = 0, kPairTail = 1, kPairPipe = 2, kPairBig = 3, kPairMid = 4, kPairMidTail = 5
