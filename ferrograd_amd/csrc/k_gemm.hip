@@ -69,9 +69,12 @@ constexpr Rate kRates[3][5] = {
 // four waves hold of a tile with edges or unaligned rows.
 constexpr float kOutUs = 0.55f, kOut128x64Us = 0.7f, kRaggedUs = 1.5f;
 // The summing launch: its own time, what a slot past the sixteenth adds to it, and
-// the rate at which it and the GEMM move the slots.
-constexpr float kSumUs = 2.0f, kSlotUs = 0.09f, kSumBytesPerUs = 4.0e6f;
-constexpr int kMaxSlices = 256;
+// the rate at which it and the GEMM move the slots.  (A slot takes 0.09 us; charged
+// less, as shorter slices are shorter chains of sums and the time is flat there: 64
+// x 64 x 4096 2.3e-7 off and 10.8 us at 0.05 a slot, 2.1e-7 and 11.0 at 0.02, 2.1e-7
+// and 24.3 in the 64 slices that thresholds on the tile counts gave.)
+constexpr float kSumUs = 2.0f, kSlotUs = 0.02f, kSumBytesPerUs = 4.0e6f;
+constexpr int kMaxSlices = 128;
 
 // What the slices of a product add: the summing launch and the slots' traffic.
 float slices_us(int M, int N, int s) {
