@@ -23,7 +23,7 @@
 // element a lane, two passes and two expf an element otherwise), us:
 //   CE fp32  2048 x 2048   7.8 -> 6.9     2000 x 10001   58.6 -> 29.6
 //            2000 x 50257  358 -> 187
-//   CE bf16  2048 x 50257  292 -> 90      8192 x 32000   465 -> 182
+//   CE bf16  2048 x 50257  292 -> 87      8192 x 32000   465 -> 182
 //            4000 x 10001  99.4 -> 32     1500 x 131072  721 -> 179
 //   backward fp32 8192 x 32000 1063 -> 521  bf16 2048 x 50257 455 -> 113
 #pragma once
@@ -93,18 +93,30 @@ struct Io {
 // 2^-24: at most 1.37 off, 0.45 rms, as expf (1.35, 0.44); the exponential of
 // (x - m) log2(e) rounded to fp32 is 2.7 off at -2, 8 at -8, 16 at -20, which
 // shows in the fp32 row loss and below 2^-126 gives zeros.  2048 x 50257 CE bf16 /
-// f16: 81 us with that, 90 / 92, with expf 111 / 128.
-template <int DT>
+// f16: 81 us with that, 87 / 92, with expf 111 / 128.
+//
+// The power is bounded, so that -inf leaves a remainder of -inf, and NaN stays in
+// the remainder: by the conversion, which saturates, or in its own step where the
+// exponentials are HELD (the conversion's form took 101 registers for 61 there: CE
+// 8192 x 2048 bf16 14.7 us for 12.0; elsewhere 4 % less time).
+template <int DT, bool HELD = false>
 __device__ __forceinline__ float exp_below(float x, float m) {
     if constexpr (DT == kF32) {
         return expf(x - m);
     } else {
         constexpr float kLog2e = 1.44269502e+00f, kLog2eLow = 1.92596303e-08f;
         const float d = x - m;
-        // (Bounded, so that the remainder of -inf is -inf; NaN stays in it.)
-        const float e = fmaxf(__builtin_rintf(d * kLog2e), -200.0f);
+        int k;
+        float e;
+        if constexpr (HELD) {
+            e = fmaxf(__builtin_rintf(d * kLog2e), -200.0f);
+            k = (int)e;
+        } else {
+            asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(k) : "v"(d * kLog2e));
+            e = (float)k;
+        }
         const float f = __builtin_fmaf(d, kLog2eLow, __builtin_fmaf(d, kLog2e, -e));
-        return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)e);
+        return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), k);
     }
 }
 
@@ -321,7 +333,7 @@ void softmax_any(const typename Io<DT>::T *x, int ldx,
     }
     if constexpr (!kHold) repack(w);
     float ex[kHold ? NV * E : 1];
-    vs = sp.single(t) >= 0 ? exp_below<DT>(vs, m) : 0.0f;
+    vs = sp.single(t) >= 0 ? exp_below<DT, kHold>(vs, m) : 0.0f;
     RowSum<DT, NV, NW> sum(vs);
     // Where exponentials are taken twice, a wave leaves out the chunks of which it
     // holds none: 4000 x 10001 bf16 / f16 42 / 49 us, now 34 / 40.  (Held ones: no
@@ -332,7 +344,7 @@ void softmax_any(const typename Io<DT>::T *x, int ldx,
         if (!kHold && first + i * NT >= sp.nb) break;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const float p = exp_below<DT>(IO::get(w[i], e), m);
+            const float p = exp_below<DT, kHold>(IO::get(w[i], e), m);
             if constexpr (kHold) ex[i * E + e] = p;
             sum.add(i, e, p);
         }
@@ -362,7 +374,7 @@ void softmax_any(const typename Io<DT>::T *x, int ldx,
             float d[E];
 #pragma unroll
             for (int e = 0; e < E; ++e)
-                d[e] = g * ((kHold ? ex[i * E + e] : exp_below<DT>(IO::get(w[i], e), m)) * inv);
+                d[e] = g * ((kHold ? ex[i * E + e] : exp_below<DT, kHold>(IO::get(w[i], e), m)) * inv);
             __builtin_nontemporal_store(IO::pack(d), at16(db, j));
         }
     };
@@ -370,7 +382,7 @@ void softmax_any(const typename Io<DT>::T *x, int ldx,
         auto *orow = out + (size_t)r * ldo;
         write(orow, scale);
         // Then, over it, the label's column.
-        if (mine) IO::store1(orow, tc, label_grad(scale, exp_below<DT>(xt, m), inv));
+        if (mine) IO::store1(orow, tc, label_grad(scale, exp_below<DT, kHold>(xt, m), inv));
     }
     if (probs) write(probs + (size_t)r * ldp, 1.0f);
 }
