@@ -102,8 +102,10 @@ float small_us(int layout, int M, int N, int K, Rows rows, int64_t n, bool colsu
         one = whole ? 0.030f : 0.042f;
         many = whole ? 0.012f : 0.032f;
     }
+    // (TN's operands are both transposed; partial tiles show from a third K tile on.)
+    const float tn = whole || (vec && K <= 64) ? 1.0f : vec ? 3.0f : 2.0f;
     return std::max(0, K - 32) * std::max(one, n * many) + 0.2f + 1.2f * n +
-           (layout == FG_TN ? (whole ? 1.0f : vec ? 3.0f : 2.0f) : 0.0f) + (colsum ? 5.0f : 0.0f);
+           (layout == FG_TN ? tn : 0.0f) + (colsum ? 5.0f : 0.0f);
 }
 
 struct Choice16 {
