@@ -40,7 +40,8 @@ int tiles(int M, int N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn 
 // against measured (us, NN): 1536^3 on 128x64 tiles 102 / 102, 64x64 77 / 77;
 // 777 x 1333 x 2049 on 64x64 tiles 70 / 71, in four slices 56 / 57.  Against the
 // choice by thresholds on the tile counts before: 1536^3 96 -> 76, 777 x
-// 1333 x 2049 74 -> 67, 512 x 1024 x 2048 46 -> 23, 2100 x 4096 x 1000 252 -> 166;
+// 1333 x 2049 74 -> 67, 512 x 1024 x 2048 46 -> 23 (where the workspace holds the
+// slices; a plan's holds 1 MiB of them), 2100 x 4096 x 1000 252 -> 166;
 // TN with column sums (not split before) 500 x 1000 x 3000 67 -> 34.
 // The candidates' order settles ties: the larger tiles first, which read
 // less from the L2s.
@@ -172,8 +173,9 @@ bool use_skinny(fg_ctx *ctx, const GemmArgs &a, int pro) {
 // 18.7, 32 x 1000 x 4096 19.0 -> 11.4, 32 x 256 x 784 9.9 -> 8.3), and up to 64
 // where reading B outweighs the fp32 matrix units' time (64 x 4096 x 4096 67.5
 // -> 40.4, 48 x 4096 x 1024 16.4 -> 14.6; but 64 x 1001 x 1001 16.5 -> 18.9, 64 x
-// 256 x 784 10.5 -> 14.4).  A data gradient of a small layer (under 2^20
-// weights) stays with the tiles, in one launch with its weight gradient.
+// 256 x 784 10.5 -> 14.4).  Each alone: a first layer that a head's kernel sums stays
+// on the tiles (chain_plan), and a data gradient of a small layer (under 2^20
+// weights) too, in one launch with its weight gradient.
 bool use_rows(int layout, const GemmArgs &a, int pro) {
     const int64_t nk = (int64_t)a.N * a.K;
     return pro == fg::gemm::kProNone && !a.colsum &&
@@ -987,10 +989,12 @@ int gemm_dw_dw_dx_dispatches(fg_ctx *ctx, int M0, int N0, int K0, const void *A0
 }
 
 // Dispatches of gemm_dw_dx_f32 for these shapes: 1 (+1 per split GEMM) when
-// the two pair, else the sum of the two calls'.  No launch.
+// the two pair, else the sum of the two calls'.  splits (may be NULL): the K
+// slices of each where they pair, else 0 and 0.  No launch.
 int gemm_dw_dx_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A1, int lda1,
                           const void *B1, int ldb1, int M2, int N2, int K2, const void *A2,
-                          int lda2, const void *B2, int ldb2) {
+                          int lda2, const void *B2, int ldb2, int *splits) {
+    if (splits) splits[0] = splits[1] = 0;
     const int sep = gemm_f32_dispatches(ctx, FG_TN, M1, N1, K1, A1, lda1, B1, ldb1, true) +
                     gemm_f32_dispatches(ctx, FG_NT, M2, N2, K2, A2, lda2, B2, ldb2, false, true);
     if (!ctx || M1 <= 0 || N1 <= 0 || K1 <= 0 || M2 <= 0 || N2 <= 0 || K2 <= 0) return sep;
@@ -1003,6 +1007,10 @@ int gemm_dw_dx_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A1, i
                                    FG_ACT_NONE, nullptr, 0, c, N2, 0), P2);
     join(ctx, P1, P2);
     if (!pairable(P1, P2)) return sep;
+    if (splits) {
+        splits[0] = P1.splits;
+        splits[1] = P2.splits;
+    }
     return 1 + (P1.splits > 1) + (P2.splits > 1);
 }
 }  // namespace fg
