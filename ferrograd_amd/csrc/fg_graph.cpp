@@ -2453,29 +2453,12 @@ FG_API int fg_plan_describe(const fg_plan *p, char *buf, size_t len, size_t *nee
         chain_dispatches(L, X);
         return chained;
     };
-    // K slices of a GEMM (1: none) as it is launched: in a pair (W, X) that runs as
-    // one launch those that the two take together, else its own call's.
-    auto pair_splits = [&](const Launch &W, const Launch &X, int sp[2]) {
-        sp[0] = sp[1] = 0;
-        if (wc && W.dtype == FG_DTYPE_F32)
-            fg::gemm_dw_dx_dispatches(wc, W.M, W.N, W.K, p->ptr(W.sA), W.lda, p->ptr(W.sB), W.ldb,
-                                      X.M, X.N, X.K, p->ptr(X.sA), X.lda, p->ptr(X.sB), X.ldb, sp);
-        return sp[0] > 0;
-    };
-    // Dispatches of launch i of v, its summing launch included.
-    auto launch_dispatches = [&](const std::vector<Launch> &v, size_t i) {
-        int sp[2];
-        if (v[i].pair_next && i + 1 < v.size() && pair_splits(v[i], v[i + 1], sp))
-            return 1 + (sp[0] > 1);
-        if (i > 0 && v[i - 1].pair_next && pair_splits(v[i - 1], v[i], sp)) return 1 + (sp[1] > 1);
-        return gemm_dispatches(v[i]);
-    };
     auto add = [&](const char *title, const std::vector<Launch> &v) {
         s += std::string(title) + ": " + std::to_string(v.size()) + " launches\n";
         for (size_t i = 0; i < v.size(); ++i) {
             const Launch &L = v[i];
             s += "  " + L.desc;
-            const int nd = launch_dispatches(v, i);
+            const int nd = gemm_dispatches(L);
             if (L.chain_next && i + 1 < v.size() && chains(L, v[i + 1]))
                 s += " [K split: slices, summed by the next launch]";
             else if (nd == 3)  // a 16-bit dW off the pipelined kernel
@@ -2570,14 +2553,14 @@ FG_API int fg_plan_describe(const fg_plan *p, char *buf, size_t len, size_t *nee
     // A captured SGD step runs the backward's last summing launch beside the
     // SGD update (run_optim), when the two touch disjoint memory.
     if (!adam && wc && !p->opt_inputs.empty() && !bwd.empty()) {
-        const size_t last = bwd.size() - 1;
+        const Launch &X = bwd.back();
+        const Launch *L = bwd.size() >= 2 && bwd[bwd.size() - 2].pair_next ? &bwd[bwd.size() - 2]
+                                                                           : nullptr;
         // (fp32 summing passes only: a 16-bit split sums within its own call)
-        auto held = [&](size_t i) {
-            return bwd[i].dtype == FG_DTYPE_F32 && launch_dispatches(bwd, i) > 1;
+        auto held = [&](const Launch *G) {
+            return G && G->dtype == FG_DTYPE_F32 && gemm_dispatches(*G) > 1;
         };
-        const Launch *H = held(last) ? &bwd[last]
-                          : last > 0 && bwd[last - 1].pair_next && held(last - 1) ? &bwd[last - 1]
-                                                                                  : nullptr;
+        const Launch *H = held(&X) ? &X : held(L) ? L : nullptr;
         if (H) {
             auto slot_range = [&](int slot) {
                 const uintptr_t b0 = (uintptr_t)p->ptr(slot);

@@ -191,8 +191,7 @@ int gemm_dw_dx_f32(fg_ctx *ctx, int M1, int N1, int K1, const float *A1, int lda
                    int ldc2, int acc2);
 int gemm_dw_dx_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A1, int lda1,
                           const void *B1, int ldb1, int M2, int N2, int K2, const void *A2,
-                          int lda2, const void *B2, int ldb2,
-                          int *splits = nullptr);
+                          int lda2, const void *B2, int ldb2);
 // The skinny kernel's largest N (output columns).
 int gemm_skinny_max_n();
 // A small head's dW (+ dbias, TN) beside a layer's dW and dX, in one launch

@@ -76,16 +76,26 @@ constexpr float kOutUs = 0.55f, kOut128x64Us = 0.7f, kRaggedUs = 1.5f;
 // and 24.3 in the 64 slices that thresholds on the tile counts gave.)
 constexpr float kSumUs = 2.0f, kSlotUs = 0.02f, kSumBytesPerUs = 4.0e6f;
 constexpr int kMaxSlices = 128;
+// With column sums a slot is charged what it takes: unsplit is what the accuracy was.
+constexpr float kSlotColUs = 0.09f;
+// What a weight gradient's slices must gain to be worth its pair.
+constexpr float kPairGain = 1.25f;
 
 // What the slices of a product add: the summing launch and the slots' traffic.
-float slices_us(int M, int N, int s) {
-    return kSumUs + kSlotUs * std::max(0, s - 16) + (2 * s + 1) * (float)M * N * 4.0f / kSumBytesPerUs;
+float slices_us(int M, int N, int s, float slot_us = kSlotUs) {
+    return kSumUs + slot_us * std::max(0, s - 16) +
+           (2 * s + 1) * (float)M * N * 4.0f / kSumBytesPerUs;
 }
 
+// grad: a layer's weight gradient with its column sums, which mostly runs in one
+// launch with its data gradient and must not take other slices there than alone (the
+// same bits).  Two split GEMMs do not pair (one workspace), so it splits only where
+// that takes a fifth off (us for the two: 640 x 2992 x 88 27.4 -> 25.8; over 334 drawn
+// layers 1 % less than where any gain splits it).
 // one_cfg: only that configuration (-1: any), on the kernel that is not
 // pipelined, which takes twice as long per k.  A K that is not whole tiles (or
 // rows unaligned: !aligned) takes the staged tiles, not 256x256.
-Choice choose(int layout, int M, int N, int K, int cus, bool aligned, bool colsum,
+Choice choose(int layout, int M, int N, int K, int cus, bool aligned, bool colsum, bool grad,
               uint64_t ws_bytes, int one_cfg = -1) {
     Choice best;
     best.us = 1e30f;
@@ -102,6 +112,8 @@ Choice choose(int layout, int M, int N, int K, int cus, bool aligned, bool colsu
         const float ragged = aligned && M % bm == 0 && N % bn == 0
                                  ? 0.0f
                                  : kRaggedUs * units * 4.0f / fg::gemm::cfg_waves(r.cfg);
+        Choice mine;
+        mine.us = 1e30f;
         // (Every count up to 16, then in steps.)
         for (int n = 1; n <= kMaxSlices; n += n < 16 ? 1 : n / 8) {
             int s = n, ks = K;
@@ -116,9 +128,11 @@ Choice choose(int layout, int M, int N, int K, int cus, bool aligned, bool colsu
                     break;
             }
             float us = (float)((t * s + cus - 1) / cus) * (ks * unit + out) + ragged;
-            if (s > 1) us += slices_us(M, N, s);
-            if (us < 0.99f * best.us) best = Choice{r.cfg, s, s > 1 ? ks : 0, us};
+            if (s > 1) us += slices_us(M, N, s, colsum ? kSlotColUs : kSlotUs);
+            if (s > 1 && grad && colsum) us *= kPairGain;
+            if (us < mine.us) mine = Choice{r.cfg, s, s > 1 ? ks : 0, us};
         }
+        if (mine.us < 0.99f * best.us) best = mine;
     }
     return best;
 }
@@ -198,10 +212,10 @@ void set_choice(const fg_ctx *ctx, GemmArgs &a, const Choice &ch) {
 // chunks (aligned) and whether it takes any K and rows (ktail), the tile configuration and the
 // number of K slices.  pro: the prologue code (fg::gemm::kPro*), whose
 // tensor Pz must meet the same 16-byte conditions as the operand it scales.
-// few_rows false: not the few-row kernel.
+// few_rows false: not the few-row kernel.  alone: a gradient that runs in no pair.
 void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &rows, bool &vec,
                bool &pipe, bool &ktail, bool &aligned, int &cfg, int &splits,
-               int pro = fg::gemm::kProNone, bool few_rows = true) {
+               int pro = fg::gemm::kProNone, bool few_rows = true, bool alone = false) {
     skinny = use_skinny(ctx, a, pro);
     vec = pipe = ktail = rows = aligned = false;
     cfg = 0;
@@ -244,11 +258,13 @@ void plan_gemm(fg_ctx *ctx, int layout, GemmArgs &a, bool &skinny, bool &rows, b
     const bool chunks = fg::gemm::kPipe && a.K > 0 && a.M >= 4 && a.N >= 4;
     aligned = vec;
     if (chunks && pro == fg::gemm::kProNone) vec = true;
+    const bool grad = !alone && a.colsum;
     Choice ch;
     if (chunks ? vec : vec && pro != fg::gemm::kProNone) {
-        ch = choose(layout, a.M, a.N, a.K, cus, aligned, a.colsum != nullptr, ctx->ws_bytes);
+        ch = choose(layout, a.M, a.N, a.K, cus, aligned, a.colsum != nullptr, grad, ctx->ws_bytes);
     } else {  // the element-load kernel's tile
-        ch = choose(layout, a.M, a.N, a.K, cus, true, a.colsum != nullptr, ctx->ws_bytes, kCfg64);
+        ch = choose(layout, a.M, a.N, a.K, cus, true, a.colsum != nullptr, grad, ctx->ws_bytes,
+                    kCfg64);
     }
     if (pro != fg::gemm::kProNone) ch.cfg = fg::gemm::pro_cfg(ch.cfg);
     set_choice(ctx, a, ch);
@@ -277,7 +293,7 @@ struct Planned {
 };
 
 int gemm_prepare(fg_ctx *ctx, int layout, const GemmArgs &a0, const char *who, int pro,
-                 Planned &P) {
+                 Planned &P, bool alone = false) {
     FG_REQUIRE(ctx, FG_ERR_INVALID_ARGUMENT, "%s: ctx is NULL", who);
     FG_REQUIRE(layout >= FG_NN && layout <= FG_TN, FG_ERR_INVALID_ARGUMENT, "%s: bad layout %d",
                who, layout);
@@ -301,7 +317,8 @@ int gemm_prepare(fg_ctx *ctx, int layout, const GemmArgs &a0, const char *who, i
                a.ldb, a.ldc);
     FG_HIP(hipSetDevice(ctx->device));
     if (a.K == 0) a.A = a.B;  // loads are all masked; K=0 yields the epilogue of zero
-    plan_gemm(ctx, layout, a, P.skinny, P.rows, P.vec, P.pipe, P.ktail, P.aligned, P.cfg, P.splits, pro);
+    plan_gemm(ctx, layout, a, P.skinny, P.rows, P.vec, P.pipe, P.ktail, P.aligned, P.cfg, P.splits, pro,
+              true, alone);
     return FG_OK;
 }
 
@@ -355,9 +372,9 @@ int gemm_launch(fg_ctx *ctx, const Planned &P, const char *who, bool reduce = tr
 }
 
 int gemm_common(fg_ctx *ctx, int layout, GemmArgs &a, const char *who,
-                int pro = fg::gemm::kProNone) {
+                int pro = fg::gemm::kProNone, bool alone = false) {
     Planned P;
-    const int rc = gemm_prepare(ctx, layout, a, who, pro, P);
+    const int rc = gemm_prepare(ctx, layout, a, who, pro, P, alone);
     if (rc) return rc;
     return gemm_launch(ctx, P, who);
 }
@@ -536,7 +553,7 @@ namespace {
 // prologue, B is scaled by act'(Pz) on load and the sums are of the scaled B.
 int gemm_dw(fg_ctx *ctx, int M, int N, int K, const float *d_A, int lda, const float *d_B,
             int ldb, float *d_C, int ldc, int accumulate, float *d_colsum, int colsum_accumulate,
-            const float *d_Pz, int ldp, int pro, const char *who) {
+            const float *d_Pz, int ldp, int pro, const char *who, bool alone = false) {
     GemmArgs a{};
     a.A = d_A;
     a.B = d_B;
@@ -564,7 +581,7 @@ int gemm_dw(fg_ctx *ctx, int M, int N, int K, const float *d_A, int lda, const f
         if (M == 0) return FG_OK;
         a.colsum = nullptr;
     }
-    return gemm_common(ctx, FG_TN, a, who, pro);
+    return gemm_common(ctx, FG_TN, a, who, pro, alone);
 }
 }  // namespace
 
@@ -627,85 +644,30 @@ bool pairable(const Planned &P1, const Planned &P2) {
     return fg::gemm::pair_exclusive(k1) || fg::gemm::pair_exclusive(k2) ? k1 == k2 : true;
 }
 
-// dW and dX of a layer on the 64x64 tiles, of which dX splits K: the slices each
-// would take alone are not those that the two should take together.  dW's tiles
-// fill the CUs that dX's leave, so dX takes fewer slices, and dW none (two split
-// GEMMs do not pair: their slices take the same workspace), where the one launch
-// and dX's sum are then shorter (us: 448 x 1024 x 448 20.1 -> 16.4, 640 x 2992 x
-// 88 26.8 -> 20.2; before dW's column sums split K they took 16.7 and 22.3).
-void share_slices(const fg_ctx *ctx, Planned &W, Planned &X) {
-    auto small = [](const Planned &P) {
-        return !P.empty && !P.skinny && !P.rows && P.pipe && P.cfg == kCfg64 &&
-               P.pro == fg::gemm::kProNone;
-    };
-    if (!small(W) || !small(X) || X.splits <= 1) return;
-    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, bk = fg::gemm::cfg_bk(kCfg64);
-    const int tw = tiles(W.a.M, W.a.N, 64, 64), tx = tiles(X.a.M, X.a.N, 64, 64);
-    auto tile_us = [](const Planned &P, int k) {
-        float r = 0.0f;
-        for (const Rate &q : kRates[P.layout])
-            if (q.cfg == kCfg64) r = q.us;
-        return k * r + kOutUs;
-    };
-    auto alone = [&](const Planned &P, int t) {
-        const int n = (t * P.splits + cus - 1) / cus;
-        return n * tile_us(P, P.splits > 1 ? P.a.ksplit : P.a.K) +
-               (P.splits > 1 ? slices_us(P.a.M, P.a.N, P.splits) : 0.0f);
-    };
-    // In one launch, dW unsplit, dX in s slices of ks: one round of workgroups, or
-    // the CUs' share of the work and on average half of the deeper tile's time.
-    auto together = [&](int s, int ks) {
-        const float w = tile_us(W, W.a.K), x = tile_us(X, ks), deep = std::max(w, x);
-        const float share = (tw * w + tx * s * x) / cus + 0.5f * deep;
-        return (tw + tx * s <= cus ? deep : std::max(deep, share)) +
-               (s > 1 ? slices_us(X.a.M, X.a.N, s) : 0.0f);
-    };
-    float us = W.splits > 1 ? alone(W, tw) + alone(X, tx) + kSumUs
-                            : together(X.splits, X.a.ksplit);
-    int best = 0, best_ks = 0;
-    us *= 0.9f;  // (else as each would alone, to the same bits)
-    for (int s = 1; s <= X.splits; ++s) {
-        const int ks = s > 1 ? ((X.a.K + s - 1) / s + bk - 1) / bk * bk : X.a.K;
-        if ((X.a.K + ks - 1) / ks != s) continue;
-        const float t = together(s, ks);
-        if (t < us) {
-            us = t;
-            best = s;
-            best_ks = ks;
-        }
-    }
-    if (best == 0) return;
-    W.splits = 1;
-    W.a.ksplit = 0;
-    W.a.partial = W.a.colsum_partial = nullptr;
-    X.splits = best;
-    X.a.ksplit = best > 1 ? best_ks : 0;
-    if (best == 1) X.a.partial = nullptr;
-}
-
-// Two unsplit pipelined GEMMs of different kinds (dW and dX of a layer) on the
-// 64x64 or the 128x64 tiles both, where one launch of all their tiles is
+// Two pipelined GEMMs of different kinds, one of them split at most (dW and dX of
+// a layer), on the 64x64 or the 128x64 tiles both, in the slices they have, where one launch of all their tiles is
 // shorter than the two they would take alone: the tiles of the second fill the
 // CUs that the last of the first leave (and their bits are those of any tile:
 // each output sums its K in the same order).
 void join(const fg_ctx *ctx, Planned &P1, Planned &P2) {
-    share_slices(ctx, P1, P2);
     auto plain = [](const Planned &P) {
-        return !P.empty && !P.skinny && !P.rows && P.pipe && P.splits == 1 &&
-               P.pro == fg::gemm::kProNone;
+        return !P.empty && !P.skinny && !P.rows && P.pipe && P.pro == fg::gemm::kProNone;
     };
-    if (pairable(P1, P2) || !plain(P1) || !plain(P2)) return;
+    if (pairable(P1, P2) || !plain(P1) || !plain(P2) || (P1.splits > 1 && P2.splits > 1)) return;
+    auto depth = [](const Planned &P) { return P.splits > 1 ? P.a.ksplit : P.a.K; };
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     // (Each with work for every CU: a narrow head's two stay apart.)
-    if (tiles(P1.a.M, P1.a.N, 64, 64) < cus || tiles(P2.a.M, P2.a.N, 64, 64) < cus) return;
+    if (tiles(P1.a.M, P1.a.N, 64, 64) * P1.splits < cus ||
+        tiles(P2.a.M, P2.a.N, 64, 64) * P2.splits < cus)
+        return;
     auto cost = [&](const Planned &P, int cfg, float &granule) {
         int bm, bn;
         fg::gemm::cfg_tile(cfg, bm, bn);
         float r = 0.0f;
         for (const Rate &q : kRates[P.layout])
             if (q.cfg == cfg) r = q.us;
-        granule = r * (bm / 64) * (bn / 64) * P.a.K;
-        return granule * tiles(P.a.M, P.a.N, bm, bn) / cus;
+        granule = r * (bm / 64) * (bn / 64) * depth(P);
+        return granule * tiles(P.a.M, P.a.N, bm, bn) * P.splits / cus;
     };
     auto alone = [&](const Planned &P) {
         float g;
@@ -716,6 +678,9 @@ void join(const fg_ctx *ctx, Planned &P1, Planned &P2) {
     int best = -1;
     float us = apart;
     for (int cfg : {kCfg128x64, kCfg64}) {
+        const int bk = fg::gemm::cfg_bk(cfg);  // (slices are whole K tiles)
+        if ((P1.splits > 1 && P1.a.ksplit % bk != 0) || (P2.splits > 1 && P2.a.ksplit % bk != 0))
+            continue;
         float g1, g2;
         // (On average half of the larger tile's time is left at the end.)
         const float t = cost(P1, cfg, g1) + cost(P2, cfg, g2);
@@ -808,9 +773,8 @@ namespace fg {
 // A layer's weight gradient dW (=|+=) X^T.dZ with dbias (=|+=) the column
 // sums of dZ (as fg_gemm_dw_f32) and its data gradient dX (=|+=)
 // (dZ.W^T) * act'(Zs) (as fg_gemm_bwd_f32, NT): independent GEMMs, one
-// launch when both take small 256-thread kernels, else one after the other:
-// the results of the two calls, bit for bit, unless share_slices cut K for the
-// two together.
+// launch when both take small 256-thread kernels, else one after the other.
+// The same results, bit for bit, either way.
 int gemm_dw_dx_f32(fg_ctx *ctx, int M1, int N1, int K1, const float *A1, int lda1,
                    const float *B1, int ldb1, float *C1, int ldc1, int acc1, float *colsum,
                    int colsum_acc, int M2, int N2, int K2, const float *A2, int lda2,
@@ -989,12 +953,10 @@ int gemm_dw_dw_dx_dispatches(fg_ctx *ctx, int M0, int N0, int K0, const void *A0
 }
 
 // Dispatches of gemm_dw_dx_f32 for these shapes: 1 (+1 per split GEMM) when
-// the two pair, else the sum of the two calls'.  splits (may be NULL): the K
-// slices of each where they pair, else 0 and 0.  No launch.
+// the two pair, else the sum of the two calls'.  No launch.
 int gemm_dw_dx_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A1, int lda1,
                           const void *B1, int ldb1, int M2, int N2, int K2, const void *A2,
-                          int lda2, const void *B2, int ldb2, int *splits) {
-    if (splits) splits[0] = splits[1] = 0;
+                          int lda2, const void *B2, int ldb2) {
     const int sep = gemm_f32_dispatches(ctx, FG_TN, M1, N1, K1, A1, lda1, B1, ldb1, true) +
                     gemm_f32_dispatches(ctx, FG_NT, M2, N2, K2, A2, lda2, B2, ldb2, false, true);
     if (!ctx || M1 <= 0 || N1 <= 0 || K1 <= 0 || M2 <= 0 || N2 <= 0 || K2 <= 0) return sep;
@@ -1007,10 +969,6 @@ int gemm_dw_dx_dispatches(fg_ctx *ctx, int M1, int N1, int K1, const void *A1, i
                                    FG_ACT_NONE, nullptr, 0, c, N2, 0), P2);
     join(ctx, P1, P2);
     if (!pairable(P1, P2)) return sep;
-    if (splits) {
-        splits[0] = P1.splits;
-        splits[1] = P2.splits;
-    }
     return 1 + (P1.splits > 1) + (P2.splits > 1);
 }
 }  // namespace fg
@@ -1063,7 +1021,7 @@ FG_API int fg_linear_bwd_f32(fg_ctx *ctx, int act, int M, int N, int K, const fl
     if (want_w) {  // dW = X^T.dZ (TN, dZ the B operand), dbias from its tiles if still due
         const int rc = gemm_dw(ctx, K, N, M, d_X, ldx, g, ldg, d_dW, lddw, accumulate,
                                dbias_done ? nullptr : d_dbias, accumulate, d_Zs, ldzs, pro_tn,
-                               who);
+                               who, true);
         if (rc) return rc;
     } else if (d_dbias && !dbias_done) {  // dbias alone: the column reduction (+ prologue)
         FG_HIP(hipSetDevice(ctx->device));
@@ -1091,7 +1049,7 @@ FG_API int fg_linear_bwd_f32(fg_ctx *ctx, int act, int M, int N, int K, const fl
         a.accumulate = accumulate ? 1 : 0;
         a.Pz = d_Zs;
         a.ldp = ldzs;
-        const int rc = gemm_common(ctx, FG_NT, a, who, pro_nt);
+        const int rc = gemm_common(ctx, FG_NT, a, who, pro_nt, true);
         if (rc) return rc;
     }
     return FG_OK;

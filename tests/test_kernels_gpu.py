@@ -791,11 +791,12 @@ def test_gemm_f32_deep_k(gpu_ctx, layout):
 
 
 @pytest.mark.parametrize("dims", [(448, 1024, 448), (640, 2992, 88), (512, 512, 64), (64, 256, 784),
-                                  (300, 700, 130), (67, 378, 2229)],
+                                  (300, 700, 130), (67, 378, 2229), (496, 960, 128)],
                          ids=lambda d: "x".join(map(str, d)))
 def test_matmul_bwd_slices(gpu_ctx, dims):
     """dW (+ dbias) and dX whose K splits, together or apart: small-integer
-    operands, every gradient bit for bit, with and without accumulation."""
+    operands, every gradient bit for bit, with and without accumulation; and on
+    normal ones the bits of the two calls."""
     torch = _torch()
     gpu_ctx.reserve_workspace(64 << 20)
     M, N, K = dims
@@ -813,6 +814,15 @@ def test_matmul_bwd_slices(gpu_ctx, dims):
         assert torch.equal(dW.cpu(), dw + dw0 if acc else dw)
         assert torch.equal(dB.cpu(), db + db0 if acc else db)
         assert torch.equal(dX.cpu(), dx + dx0 if acc else dx)
+    X, W, dZ, Zs = (torch.randn(t.shape, generator=g).cuda() for t in (x, w, dz, zs))
+    a, b = ([empty((M, K)), empty((K, N)), empty((N,))] for _ in range(2))
+    gpu_ctx.matmul_bwd(M, N, K, X, K, W, N, dZ, N, a[0], K, a[1], N, dbias=a[2], act=O.ACT_GELU,
+                       Zs=Zs, ldzs=K)
+    gpu_ctx.gemm_dw(K, N, M, X, K, dZ, N, b[1], N, colsum=b[2])
+    gpu_ctx.gemm_bwd(O.NT, M, K, N, dZ, N, W, N, b[0], K, act=O.ACT_GELU, Zs=Zs, ldzs=K)
+    torch.cuda.synchronize()
+    for p, q in zip(a, b):
+        assert torch.equal(p, q)
 
 
 # 16-bit tiles on rows of any alignment, as test_gemm_f32_any_rows: K
